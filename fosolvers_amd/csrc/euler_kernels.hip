@@ -18,12 +18,13 @@
 //    states of boundary faces are formed in the face loop.
 //  * tet_kernel (tetrahedral layout, the default): the ghost states of the boundary pairs are formed
 //    by a small kernel ahead of the face pass (ghost_kernel), which keeps the boundary-condition
-//    code and its registers out of the face loop, and each face adds its flux to its chunk-local
-//    cells' sums in LDS with atomic adds (as the reference's OpenMP atomics do, Euler.f90:127-151),
-//    which needs 5 values per cell instead of 5 per face.  The sums are FP64 for both arithmetic
-//    types: gfx950's FP32 LDS atomic add (ds_add_f32) ran the FP32 Jv kernels 2.5x slower than
-//    ds_add_f64 does.  The order of the adds varies from run to run, so results agree to rounding
-//    (~1e-16 relative per cell sum), not bitwise.
+//    code and its registers out of the face loop.  In FP64 and in the analytic Jv each face adds its
+//    flux to its chunk-local cells' sums in LDS with atomic adds (as the reference's OpenMP atomics do,
+//    Euler.f90:127-151), which needs 5 values per cell instead of 5 per face; the order of the adds
+//    varies from run to run, so these results agree to rounding (~1e-16 relative per cell sum), not
+//    bitwise.  The FP32 residual and difference quotients gather their fluxes as the generic kernel
+//    does (tet_gathers, below).  The sums are FP64 for both arithmetic types: gfx950's FP32 LDS atomic
+//    add (ds_add_f32) ran the FP32 Jv kernels 2.5x slower than ds_add_f64 does.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -346,27 +347,43 @@ int launch(const FluxLayout<TC> &L, const TS *y, const TS *v, TS sigma, const do
 // a boundary face's ghost primitives from ghost_kernel's output, and adds the face flux into the
 // chunk-local cells' sums.  Both chunks of a chunk-crossing face evaluate it with the same operand
 // order and the same FP64 coordinates, so its two copies agree bitwise.
+//
+// How the cells' sums are formed: with gather set, the fluxes are parked in LDS and each cell adds its
+// faces in slot order (FP64 sums, bitwise reproducible), else each face adds its flux to the sums with
+// LDS atomics.  The FP32 residual and difference quotients gather: their fluxes are half as wide, and
+// the ten FP64 atomics of a face took about half of the LDS pipe, which was busy 78 % of the kernel
+// (6M tets, FP32 residual: 151 -> 134 us).  In FP64 the parked fluxes cost a workgroup per CU and the
+// slots 8 bytes per cell, and the kernel moves its traffic at the copy rate already (6M tets: 210 us,
+// 251 gathered; 222 with the fluxes held in registers until the staged cells' space is free); the
+// analytic Jv is bound by its arithmetic (FP32, 6M tets: 319 us, 323 gathered).
+template <class TC>
+constexpr bool tet_gathers(int mode) { return sizeof(TC) == 4 && mode != JVP; }
+
 template <class TS, class TC, int MODE, int NS, bool NT>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
     MODE == 3 ? FOS_JVP_MIN_WAVES : FOS_TET_MIN_WAVES))) void tet_kernel(
     TetLayout<TC> L, const TS *__restrict__ y, const TS *__restrict__ v, TS sigmaVal,
     const double *__restrict__ sigmaPtr, const TS *__restrict__ fy, TS *__restrict__ out, unsigned *__restrict__ nf,
     int newton, TS ngam) {
-  constexpr bool JV = MODE != RES;
+  constexpr bool JV = MODE != RES, GATHER = tet_gathers<TC>(MODE);
   constexpr int NQ = nq_of(MODE);
   const TS sigma = JV && sigmaPtr ? (TS)*sigmaPtr : sigmaVal;
   extern __shared__ unsigned char smem_raw[];
   const int mn = L.maxNodes;
   TC *sQ = reinterpret_cast<TC *>(smem_raw);                 // [NQ][CHUNK]
-  double *sA = reinterpret_cast<double *>(sQ + NQ * CHUNK);  // [5][CHUNK] per-cell flux sums (FP64)
-  TC *sN = reinterpret_cast<TC *>(sA + 5 * CHUNK);           // [3][mn] node coordinates
+  // [5][CHUNK] per-cell flux sums (FP64), or [5][mcf] face fluxes
+  double *sA = reinterpret_cast<double *>(sQ + NQ * CHUNK);
+  TC *sF = sQ + NQ * CHUNK;
+  const int mcf = L.maxChunkFaces;
+  TC *sN = GATHER ? sF + 5 * mcf : reinterpret_cast<TC *>(sA + 5 * CHUNK);  // [3][mn] node coordinates
   const int chunk = xcd_remap(blockIdx.x, gridDim.x);
   const int nC = L.nC, c0 = chunk * CHUNK, ncell = min(CHUNK, nC - c0);
   const TC g1 = L.gamma - TC(1);
   const int t = threadIdx.x;
   // A: the first face record and the nodes are loaded before the cells are staged
+  if constexpr (!GATHER)
 #pragma unroll
-  for (int k = 0; k < 5; k++) sA[k * CHUNK + t] = 0.0;
+    for (int k = 0; k < 5; k++) sA[k * CHUNK + t] = 0.0;
   const int fb = L.chunkBeg[chunk], fe = L.chunkBeg[chunk + 1];
   uint2 recN = make_uint2(0u, 0u);
   // NT (working sets beyond the 256 MB last-level cache): the face records, node coordinates and
@@ -387,7 +404,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
     sN[mn + t] = ld(p + 1);
     sN[2 * mn + t] = ld(p + 2);
   }
-  if (t < ncell) stage_cell<TS, TC, MODE>(y, v, sigma, nC, c0 + t, g1, sQ, CHUNK, t);
+  unsigned long long slots = 0;  // the cell's face slots, for C
+  if (t < ncell) {
+    if constexpr (GATHER) slots = ld(reinterpret_cast<const unsigned long long *>(L.slots) + c0 + t);
+    stage_cell<TS, TC, MODE>(y, v, sigma, nC, c0 + t, g1, sQ, CHUNK, t);
+  }
   __syncthreads();
   // B: one Roe flux (or flux difference) per chunk face
   const TC *sy = sN + mn, *sz = sN + 2 * mn;
@@ -445,8 +466,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
       for (int k = 0; k < 5; k++) F[k] = (MODE == DQ_DIFF && pass == 0) ? -Fp[k] : F[k] + Fp[k];
     }
-    // the flux leaves L and enters R: each chunk-local side accumulates it (LDS atomics)
-    if (kind == 1) {
+    // the flux leaves L and enters R: each chunk-local side accumulates it
+    if constexpr (GATHER) {
+#pragma unroll
+      for (int k = 0; k < 5; k++) sF[k * mcf + (f - fb)] = F[k];
+    } else if (kind == 1) {
 #pragma unroll
       for (int k = 0; k < 5; k++) atomicAdd(&sA[k * CHUNK + lc], (double)F[k]);
     } else {
@@ -461,9 +485,23 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
   __syncthreads();
   // C: the cell's sum, divided by v
   if (t < ncell) {
+    double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    if constexpr (GATHER) {
+#pragma unroll
+      for (int j = 0; j < NS; j++) {
+        const int s = (short)(slots >> (16 * j));
+        if (s < 0) continue;
+        const TC *f = sF + (s >> 1);
+#pragma unroll
+        for (int k = 0; k < 5; k++) sum[k] += s & 1 ? (double)f[k * mcf] : -(double)f[k * mcf];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < 5; k++) sum[k] = sA[k * CHUNK + t];
+    }
     TC acc[5];
 #pragma unroll
-    for (int k = 0; k < 5; k++) acc[k] = (TC)sA[k * CHUNK + t];
+    for (int k = 0; k < 5; k++) acc[k] = (TC)sum[k];
     write_cell<TS, TC, MODE, NT>(acc, ld(&L.invV[c0 + t]), sigma, fy, out, nC, c0 + t, nf, v, newton, ngam);
   }
 }
@@ -511,7 +549,8 @@ constexpr size_t TET_LDS_LIMIT = 65536;
 template <class TC>
 size_t tet_lds(const TetLayout<TC> &L, int mode) {
   const size_t nq = nq_of(mode);
-  const size_t b = sizeof(double) * 5 * (size_t)CHUNK + sizeof(TC) * (nq * (size_t)CHUNK + 3 * (size_t)L.maxNodes);
+  const size_t sums = tet_gathers<TC>(mode) ? sizeof(TC) * 5 * (size_t)L.maxChunkFaces : sizeof(double) * 5 * (size_t)CHUNK;
+  const size_t b = sums + sizeof(TC) * (nq * (size_t)CHUNK + 3 * (size_t)L.maxNodes);
   return b <= TET_LDS_LIMIT ? b : 0;
 }
 
