@@ -26,23 +26,23 @@ struct BlockIlu {
   int nC = 0, nLev = 0, nCol = 0;
   bool haveJac = false, bjac = false;  // factors hold block ILU(0), or block Jacobi inverses
   std::vector<int> levPtr, colPtr, hOrder;
-  DBuf<int> dNbr;       // [NB nC] neighbour cell per slot (neib order), -1 = none / facet
-  DBuf<int> dRank;      // [nC] elimination step of each row (its position in the sweeps' vectors)
-  DBuf<int> dOrder;     // [nC] row eliminated at each step
-  DBuf<int> dLowOrd;    // [NB nC] slots of lower neighbours in elimination order, -1 padded
-  DBuf<int> dLevRows;   // rows grouped by factorisation level
   DBuf<int> dJSlot;     // [nSlots nC] neib slot j of residual-layout slot s (-1 boundary / none)
   DBuf<double> dJac;    // [125 nC] JacC(5, 25, nC) column-major
-  DBuf<double> dD, dOff;  // factor: inverted U diagonal blocks [25 nC], off-diagonal blocks [25 NB nC]
-  DBuf<float> dD32;       // FP32 copy of dD (block Jacobi apply)
-  // Copies of the factors for the sweeps (built after each factorisation in the context's apply
-  // precision): per chunk its rows' L blocks packed in the forward sweep's step order and its U
+  // Factorisation: its rows grouped by level, three int4 and a word each, and the tables that the general
+  // branch reads (factor_level_kernel)
+  DBuf<int4> dFacRec;
+  DBuf<unsigned> dFacBits;
+  DBuf<int> dNbr, dRank, dBPos;  // [NB nC] neighbour per slot, [nC] elimination step, [NB nC] packed block per slot
+  DBuf<double> dGamma;           // [1] the current setup's gamma
+  // The factors: per chunk its rows' L blocks packed in the forward sweep's step order and its U
   // blocks in the backward sweep's, each row's blocks consecutive; the inverted diagonal block of
-  // elimination position p at p.
-  DBuf<int> dLSrc, dUSrc;  // packed block -> source block NB*row + slot in dOff
+  // elimination position p at p.  FP64 contexts sweep dLf, dUf, dDb; FP32 ones sweep the FP32 arrays
+  // and keep dUf and dDb for the factorisation, which reads them.
   long long nLBlk = 0, nUBlk = 0;
   DBuf<double> dLf, dUf, dDb;
   DBuf<float> dLf32, dUf32, dDb32;
+  DBuf<double> dBj;   // block Jacobi's inverted diagonal blocks [25 nC] (FP32 contexts: dBj32)
+  DBuf<float> dBj32;
   // sweep schedule: the chunks of each colour (colPtr) in launch order, per launch slot the chunk's
   // metadata (two int4, forward and backward), per chunk its steps (forward by the lower, backward
   // by the upper neighbours inside the chunk) as step records of chunk-local codes, and its
@@ -166,16 +166,37 @@ __device__ inline void flux_col(const double (&Um)[5], const double (&Un)[5], bo
   for (int k = 0; k < 5; k++) col[k] = F[k].d;
 }
 
+// The Jacobian kernels' workgroup (one wave: JAC_THREADS / NS cells) stages its cells' rows of JacC, 1000
+// bytes each, in LDS and stores them as one contiguous run.  Stored by the lanes that formed them (8
+// bytes each, 200 bytes apart) they went out at 1.7 TB/s and set jac_kernel's time: 593 us at 1.07M tets
+// and 3.65 ms at 6M, 401 us and 2.17 ms as a run (4 TB/s with the reads, of the copy's 4.9).  8-byte
+// stores: a caller's array need not be aligned to more.
+constexpr int JAC_THREADS = 64;
+template <int NS>
+__device__ inline void store_jac_rows(const double *sJ, int blk, int nC, double *__restrict__ jac) {
+  constexpr int CELLS = JAC_THREADS / NS;
+  const int c0 = blk * CELLS, n = 125 * min(CELLS, nC - c0);
+  double *to = jac + (size_t)125 * c0;
+  // an array beyond the 256 MB last-level cache goes around the L2, which then keeps the cell states
+  const bool stream = (size_t)nC * 1000 > ((size_t)256 << 20);
+  __syncthreads();
+  if (stream)
+    for (int k = threadIdx.x; k < n; k += JAC_THREADS) __builtin_nontemporal_store(sJ[k], &to[k]);
+  else
+    for (int k = threadIdx.x; k < n; k += JAC_THREADS) to[k] = sJ[k];
+}
+
 // The exact, boundary-consistent JacC (FOS_JAC_EXACT): the blocks of the residual's true
 // derivative (not divided by v), column by column from flux_col -- the Roe dissipation
 // differentiated with its averages, boundary faces through their ghost states -- where
 // findEulerJac freezes |A~| and drops the ghost dependence (Euler.f90:210-219).  Same lanes,
 // layout and zeroing as jac_kernel.
 template <int NS>
-__global__ __launch_bounds__(256) void jac_exact_kernel(FluxLayout<double> L, const int *__restrict__ jslot,
+__global__ __launch_bounds__(JAC_THREADS) void jac_exact_kernel(FluxLayout<double> L, const int *__restrict__ jslot,
                                                         const double *__restrict__ y, double *__restrict__ jac) {
   static_assert(NS >= NB && (NS & (NS - 1)) == 0 && 64 % NS == 0, "slot lanes");
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int blk = xcd_remap(blockIdx.x, gridDim.x);  // neighbouring cells in one XCD's L2
+  const int t = blk * JAC_THREADS + threadIdx.x;
   const int c = t / NS, s = t % NS;
   const bool live = c < L.nC;
   const int nC = L.nC;
@@ -183,7 +204,8 @@ __global__ __launch_bounds__(256) void jac_exact_kernel(FluxLayout<double> L, co
 #pragma unroll
   for (int k = 0; k < 25; k++) D[k] = 0.0;
   int jj = -1;
-  double *out = jac + (size_t)125 * c;
+  __shared__ double sJ[JAC_THREADS / NS * 125];
+  double *out = sJ + 125 * (threadIdx.x / NS);
   const int code = live ? L.slots[(size_t)NS * c + s] : -1;
   if (code >= 0) {
     const int f = L.chunkBeg[c / CHUNK] + (code >> 1);
@@ -232,23 +254,24 @@ __global__ __launch_bounds__(256) void jac_exact_kernel(FluxLayout<double> L, co
     for (int k = 0; k < 25; k++) D[k] += __shfl_xor(D[k], m, NS);
     written |= __shfl_xor(written, m, NS);
   }
-  if (!live) return;
 #pragma unroll
   for (int k = 0; k < 25; k++)
     if (k % NS == s) out[k] = D[k];
   if (s < NB && !((written >> s) & 1))
     for (int k = 0; k < 25; k++) out[25 * (1 + s) + k] = 0.0;
+  store_jac_rows<NS>(sJ, blk, nC, jac);
 }
 
 // One thread per (cell, face slot): NS consecutive lanes hold one cell.  Each lane forms its face's
-// neighbour block of JacC (written directly: a neighbour shares one face with the cell) and its
+// neighbour block of JacC (a neighbour shares one face with the cell) and its
 // contribution to the diagonal block, which the cell's lanes sum by butterfly shuffles; the lanes
 // then zero the neighbour blocks no face wrote (facets).
 template <int NS>
-__global__ __launch_bounds__(256) void jac_kernel(FluxLayout<double> L, const int *__restrict__ jslot,
+__global__ __launch_bounds__(JAC_THREADS) void jac_kernel(FluxLayout<double> L, const int *__restrict__ jslot,
                                                   const double *__restrict__ y, double *__restrict__ jac) {
   static_assert(NS >= NB && (NS & (NS - 1)) == 0 && 64 % NS == 0, "slot lanes");
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int blk = xcd_remap(blockIdx.x, gridDim.x);  // neighbouring cells in one XCD's L2
+  const int t = blk * JAC_THREADS + threadIdx.x;
   const int c = t / NS, s = t % NS;
   const bool live = c < L.nC;  // every lane takes part in the shuffles
   const int nC = L.nC;
@@ -257,7 +280,8 @@ __global__ __launch_bounds__(256) void jac_kernel(FluxLayout<double> L, const in
 #pragma unroll
   for (int k = 0; k < 25; k++) D[k] = 0.0;
   int jj = -1;
-  double *out = jac + (size_t)125 * c;
+  __shared__ double sJ[JAC_THREADS / NS * 125];
+  double *out = sJ + 125 * (threadIdx.x / NS);
   const int code = live ? L.slots[(size_t)NS * c + s] : -1;
   if (code >= 0) {
     const int f = L.chunkBeg[c / CHUNK] + (code >> 1);
@@ -324,24 +348,15 @@ __global__ __launch_bounds__(256) void jac_kernel(FluxLayout<double> L, const in
     for (int k = 0; k < 25; k++) D[k] += __shfl_xor(D[k], m, NS);
     written |= __shfl_xor(written, m, NS);
   }
-  if (!live) return;
 #pragma unroll
   for (int k = 0; k < 25; k++)
     if (k % NS == s) out[k] = D[k];
   if (s < NB && !((written >> s) & 1))
     for (int k = 0; k < 25; k++) out[25 * (1 + s) + k] = 0.0;
+  store_jac_rows<NS>(sJ, blk, nC, jac);
 }
 
 // ---------------------------------------------------------------- block ILU(0)
-
-__device__ inline void mm5(const double *A, const double *B, double *C) {  // row-major C = A B
-  for (int i = 0; i < 5; i++)
-    for (int j = 0; j < 5; j++) {
-      double s = 0.0;
-      for (int k = 0; k < 5; k++) s += A[5 * i + k] * B[5 * k + j];
-      C[5 * i + j] = s;
-    }
-}
 
 __device__ inline bool inv5(const double *A, double *Ai) {  // Gauss-Jordan, partial pivoting, row-major
   // every index is a compile-time constant once the loops unroll (the pivot row is swapped in by
@@ -383,115 +398,189 @@ __device__ inline bool inv5(const double *A, double *Ai) {  // Gauss-Jordan, par
   return true;
 }
 
-// M = I - gamma JacC / v, blocks row-major: D <- diagonal block (not yet inverted), Off <- neighbours
-__global__ __launch_bounds__(256) void form_m_kernel(int nC, const double *__restrict__ jac,
-                                                     const double *__restrict__ invV, const int *__restrict__ nbr,
-                                                     double gamma, double *__restrict__ D, double *__restrict__ Off) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)nC * 25 * (1 + NB)) return;
-  const int c = (int)(t / (25 * (1 + NB)));
-  const int e = (int)(t % (25 * (1 + NB)));
-  const int blk = e / 25, k = e % 25, r = k / 5, q = k % 5;
-  const double s = -gamma * invV[c];
-  const double jv = jac[(size_t)125 * c + 25 * blk + 5 * q + r];  // JacC column-major: (row r, col q)
-  if (blk == 0) {
-    D[(size_t)25 * c + k] = (r == q ? 1.0 : 0.0) + s * jv;
-  } else {
-    const int j = blk - 1;
-    const int nb = nbr[(size_t)NB * c + j];
-    Off[((size_t)NB * c + j) * 25 + k] = nb >= 0 ? s * jv : 0.0;
-  }
-}
-
 __device__ inline int sel4(int4 v, int a) { return a == 0 ? v.x : a == 1 ? v.y : a == 2 ? v.z : v.w; }
 
-// C -= A B (row-major 5x5), B read from memory
-__device__ inline void mms5(const double *A, const double *__restrict__ B, double *C) {
+// r (row of 5) times the row-major 5x5 block at B
+__device__ inline void row_times(const double (&r)[5], const double *__restrict__ B, double (&out)[5]) {
   double b[25];
 #pragma unroll
-  for (int q = 0; q < 25; q++) b[q] = B[q];
+  for (int k = 0; k < 25; k++) b[k] = B[k];
 #pragma unroll
-  for (int i = 0; i < 5; i++)
+  for (int c = 0; c < 5; c++) {
+    double s = r[0] * b[c];
 #pragma unroll
-    for (int j = 0; j < 5; j++) {
-      double s = A[5 * i] * b[j];
-#pragma unroll
-      for (int k = 1; k < 5; k++) s += A[5 * i + k] * b[5 * k + j];
-      C[5 * i + j] -= s;
-    }
+    for (int k = 1; k < 5; k++) s += r[k] * b[5 * k + c];
+    out[c] = s;
+  }
 }
 
-// One level of the IKJ block factorisation: one thread per block row, "lower" meaning eliminated
-// earlier (rank).  The diagonal block and the current L_ik stay in registers (static indices only);
-// the rare update of another off-diagonal block of row i (a neighbour of both i and k) goes to
-// memory in place.
-__global__ __launch_bounds__(128) void factor_level_kernel(const int *__restrict__ rows, int n,
-                                                           const int *__restrict__ nbr, const int *__restrict__ lowOrd,
-                                                           const int *__restrict__ rank, double *__restrict__ D,
-                                                           double *__restrict__ Off, int *__restrict__ status) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n) return;
-  const int i = rows[t];
-  const int4 nbi = reinterpret_cast<const int4 *>(nbr)[i];
-  const int4 lo = reinterpret_cast<const int4 *>(lowOrd)[i];
-  double Aii[25];
+// The current setup's gamma and a cleared pivot status, for the recorded factorisation
+__global__ void factor_begin_kernel(double *gamma, double g, int *status) {
+  if (threadIdx.x == 0) {
+    *gamma = g;
+    *status = 0x7fffffff;
+  }
+}
+
+// One level of the IKJ block factorisation of M = I - gamma JacC / v, "lower" meaning eliminated
+// earlier.  Five lanes hold a block row, lane q row q of each of its blocks, so products with a block
+// of an earlier row need no exchange (the five lanes read the same block); the five rows of the
+// eliminated diagonal block meet in LDS, and lane q forms column q of its inverse.  M is formed from the
+// row's 1000 contiguous bytes of JacC, and the finished blocks go straight to where the sweeps (and
+// later rows) read them.  Every block the row needs is read at once, row q by lane q, and passed around
+// through LDS.  Before, one thread per row worked on a stored M, with M and the packed copies made in
+// passes of their own: 2.0 ms for the levels and 1.07 ms for the passes at 1.07M tets, 6.0 and 6.0 ms at
+// 6M; now 1.06 ms and 5.3 ms.  What bounds a level is its traffic (3.1 KB a row at 3.6 TB/s, 200-byte
+// blocks straddling cache lines), and on small meshes (24,000 tets: 25 -> 7 us a level) the latency of
+// its two dependent reads, its arithmetic and its stores.  At 204 registers two waves fit a SIMD; held to
+// 168 for three it was 18 % slower, and non-temporal reads of JacC were 7 % slower.
+// rec: per row {cell, elimination position p, first packed L block, first packed U block}, the lower
+// neighbours' positions in elimination order, and the packed U blocks that couple them to this row.
+// bits: 0-3 upper slots, 4-7 lower slots, 8-15 the lower neighbours' slots in elimination order (2
+// bits each), 16-18 their number, 19: two of the row's neighbours are neighbours of each other, so an
+// elimination may update another block of the row (general branch, which reads nbr, rank, bpos).
+constexpr int FAC_ROWS = 12;
+constexpr unsigned FAC_FILL = 1u << 19;
+template <class TF>
+__global__ __launch_bounds__(64) void factor_level_kernel(
+    const int4 *__restrict__ rec, const unsigned *__restrict__ bits, int n, const double *__restrict__ jac,
+    const double *__restrict__ invV, const double *__restrict__ gamma, const int *__restrict__ nbr,
+    const int *__restrict__ rank, const int *__restrict__ bpos, double *U64, double *D64, TF *L, TF *U, TF *D,
+    int *__restrict__ status) {
+  __shared__ double sB[2][(FAC_ROWS + 1) * 25];
+  const int lane = threadIdx.x, slot = lane / 5, q = lane - 5 * slot;
+  const int t = xcd_remap(blockIdx.x, gridDim.x) * FAC_ROWS + slot;
+  const bool live = slot < FAC_ROWS && t < n;
+  double *sD = sB[0] + 25 * slot, *sU = sB[1] + 25 * slot;
+  int4 r0 = make_int4(0, 0, 0, 0), kp = r0, ku = r0;
+  unsigned b = 0;
+  if (live) {
+    r0 = rec[3 * (size_t)t];
+    kp = rec[3 * (size_t)t + 1];
+    ku = rec[3 * (size_t)t + 2];
+    b = bits[t];
+  }
+  const int i = r0.x, p = r0.y, nLow = (b >> 16) & 7u;
+  // one round trip: row q of the row's own blocks and of every earlier block it needs
+  double A[5], O[NB][5], Dr[NB][5], Ur[NB][5];
 #pragma unroll
-  for (int q = 0; q < 25; q++) Aii[q] = D[(size_t)25 * i + q];
+  for (int a = 0; a < NB; a++)
+    if (a < nLow)
+#pragma unroll
+      for (int c = 0; c < 5; c++) {
+        Dr[a][c] = D64[(size_t)25 * sel4(kp, a) + 5 * q + c];
+        Ur[a][c] = U64[(size_t)25 * sel4(ku, a) + 5 * q + c];
+      }
+  if (live) {
+    const double s = -*gamma * invV[i];
+    const double *J = jac + (size_t)125 * i;  // column-major blocks: (row r, col c) at 5 c + r
+#pragma unroll
+    for (int c = 0; c < 5; c++) A[c] = (c == q ? 1.0 : 0.0) + s * J[5 * c + q];
+#pragma unroll
+    for (int j = 0; j < NB; j++)
+#pragma unroll
+      for (int c = 0; c < 5; c++) O[j][c] = s * J[25 * (1 + j) + 5 * c + q];  // 0 where there is no neighbour
+  }
 #pragma unroll
   for (int a = 0; a < NB; a++) {
-    const int js = sel4(lo, a);
-    if (js < 0) break;
-    const int k = sel4(nbi, js);
-    const int4 nbk = reinterpret_cast<const int4 *>(nbr)[k];
-    const int rk = rank[k];
-    double *Lik = Off + ((size_t)NB * i + js) * 25;
-    double A[25], Lk[25];
+    if (!__any(a < nLow)) break;
+    if (a < nLow)
 #pragma unroll
-    for (int q = 0; q < 25; q++) { A[q] = Lik[q]; Lk[q] = 0.0; }
-    mms5(A, D + (size_t)25 * k, Lk);  // Lk = -A_ik inv(U_kk)
+      for (int c = 0; c < 5; c++) {
+        sD[5 * q + c] = Dr[a][c];
+        sU[5 * q + c] = Ur[a][c];
+      }
+    __syncthreads();
+    if (a < nLow) {
+      const int js = (b >> (8 + 2 * a)) & 3u;
+      double r[5], Lr[5], u[5];
 #pragma unroll
-    for (int q = 0; q < 25; q++) { Lk[q] = -Lk[q]; Lik[q] = Lk[q]; }
+      for (int c = 0; c < 5; c++) r[c] = js == 0 ? O[0][c] : js == 1 ? O[1][c] : js == 2 ? O[2][c] : O[3][c];
+      row_times(r, sD, Lr);  // L_ik = A_ik inv(U_kk)
+      const int m = r0.z + __popc((b >> 4) & ((1u << js) - 1u));
 #pragma unroll
-    for (int jk = 0; jk < NB; jk++) {
-      const int j = sel4(nbk, jk);
-      if (j < 0 || rank[j] <= rk) continue;  // U part of row k: eliminated after k
-      const double *U = Off + ((size_t)NB * k + jk) * 25;
-      if (j == i) {
-        mms5(Lk, U, Aii);
-      } else {
-        const int ji = nbi.x == j ? 0 : nbi.y == j ? 1 : nbi.z == j ? 2 : nbi.w == j ? 3 : -1;
-        if (ji < 0) continue;
-        double *dst = Off + ((size_t)NB * i + ji) * 25;
-        double C[25];
+      for (int c = 0; c < 5; c++) L[(size_t)25 * m + 5 * q + c] = (TF)Lr[c];
+      row_times(Lr, sU, u);
 #pragma unroll
-        for (int q = 0; q < 25; q++) C[q] = dst[q];
-        mms5(Lk, U, C);
+      for (int c = 0; c < 5; c++) A[c] -= u[c];
+      if (b & FAC_FILL) {  // U_kj for the other neighbours j of k that are also neighbours of i
+        const int k = nbr[(size_t)NB * i + js], rk = rank[k];
+        for (int jk = 0; jk < NB; jk++) {
+          const int j = nbr[(size_t)NB * k + jk];
+          if (j < 0 || j == i || rank[j] <= rk) continue;
+          int ji = -1;
+          for (int e = 0; e < NB; e++)
+            if (nbr[(size_t)NB * i + e] == j) ji = e;
+          if (ji < 0) continue;
+          row_times(Lr, U64 + (size_t)25 * bpos[(size_t)NB * k + jk], u);
 #pragma unroll
-        for (int q = 0; q < 25; q++) dst[q] = C[q];
+          for (int e = 0; e < NB; e++)
+#pragma unroll
+            for (int c = 0; c < 5; c++) O[e][c] -= e == ji ? u[c] : 0.0;
+        }
       }
     }
+    __syncthreads();
   }
-  double Di[25];
-  if (!inv5(Aii, Di)) {
-    atomicMin(status, i);
+  if (live) {
 #pragma unroll
-    for (int q = 0; q < 25; q++) Di[q] = 0.0;
+    for (int j = 0; j < NB; j++)
+      if ((b >> j) & 1u) {
+        const size_t at = (size_t)25 * (r0.w + __popc(b & ((1u << j) - 1u))) + 5 * q;
+#pragma unroll
+        for (int c = 0; c < 5; c++) {
+          U64[at + c] = O[j][c];
+          if (!std::is_same<TF, double>::value) U[at + c] = (TF)O[j][c];
+        }
+      }
+#pragma unroll
+    for (int c = 0; c < 5; c++) sD[5 * q + c] = A[c];
   }
+  __syncthreads();
+  if (!live) return;
+  // column q of the inverse: Gauss-Jordan with partial pivoting, the five lanes in step (static
+  // indices only, the pivot row swapped in by selects, so M stays in registers)
+  double M[5][6];
 #pragma unroll
-  for (int q = 0; q < 25; q++) D[(size_t)25 * i + q] = Di[q];
+  for (int r = 0; r < 5; r++) {
+#pragma unroll
+    for (int c = 0; c < 5; c++) M[r][c] = sD[5 * r + c];
+    M[r][5] = r == q ? 1.0 : 0.0;
+  }
+  bool singular = false;
+#pragma unroll
+  for (int c = 0; c < 5; c++) {
+    int piv = c;
+    double best = fabs(M[c][c]);
+#pragma unroll
+    for (int r = c + 1; r < 5; r++)
+      if (fabs(M[r][c]) > best) { best = fabs(M[r][c]); piv = r; }
+    singular |= best == 0.0;
+#pragma unroll
+    for (int r = c + 1; r < 5; r++)
+      if (r == piv)
+#pragma unroll
+        for (int e = c; e < 6; e++) { const double x = M[c][e]; M[c][e] = M[r][e]; M[r][e] = x; }
+    const double d = 1.0 / M[c][c];
+#pragma unroll
+    for (int e = c + 1; e < 6; e++) M[c][e] *= d;
+#pragma unroll
+    for (int r = 0; r < 5; r++)
+      if (r != c) {
+        const double f = M[r][c];
+        if (f != 0.0)
+#pragma unroll
+          for (int e = c + 1; e < 6; e++) M[r][e] -= f * M[c][e];
+      }
+  }
+  if (singular && q == 0) atomicMin(status, i);
+#pragma unroll
+  for (int r = 0; r < 5; r++) {
+    const double x = singular ? 0.0 : M[r][5];
+    D64[(size_t)25 * p + 5 * r + q] = x;
+    if (!std::is_same<TF, double>::value) D[(size_t)25 * p + 5 * r + q] = (TF)x;
+  }
 }
-
-// Factor blocks into level order: to[m] = (TF) from[src[m]], 25 values per block.
-template <class TF>
-__global__ __launch_bounds__(256) void gather_blocks_kernel(long long nBlk, const int *__restrict__ src,
-                                                            const double *__restrict__ from, TF *__restrict__ to) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)nBlk * 25) return;
-  const size_t m = t / 25;
-  to[t] = (TF)from[(size_t)src[m] * 25 + (t - m * 25)];
-}
-
-// y[rank[i]][q] = r[q][i]: the right-hand side into elimination order, cell-major.
 
 template <class TF>
 __device__ inline double dot5(const TF *__restrict__ a, const double *__restrict__ b) {
@@ -922,21 +1011,23 @@ __global__ void ilu_io_kernel(const double **io, const double *r, double *z) {
   }
 }
 
-// Block Jacobi: D <- inv(D) per cell (also the FP32 copy); status = lowest singular cell
-__global__ __launch_bounds__(128) void bjac_invert_kernel(int nC, double *__restrict__ D, float *__restrict__ D32,
+// Block Jacobi: inv(M_cc) of M = I - gamma JacC / v per cell; status = lowest singular cell
+template <class TF>
+__global__ __launch_bounds__(128) void bjac_invert_kernel(int nC, const double *__restrict__ jac,
+                                                          const double *__restrict__ invV,
+                                                          const double *__restrict__ gamma, TF *__restrict__ D,
                                                           int *__restrict__ status) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nC) return;
+  const double s = -*gamma * invV[i];
   double A[25], Ai[25];
-  for (int q = 0; q < 25; q++) A[q] = D[(size_t)25 * i + q];
+  for (int r = 0; r < 5; r++)
+    for (int c = 0; c < 5; c++) A[5 * r + c] = (r == c ? 1.0 : 0.0) + s * jac[(size_t)125 * i + 5 * c + r];
   if (!inv5(A, Ai)) {
     atomicMin(status, i);
     for (int q = 0; q < 25; q++) Ai[q] = 0.0;
   }
-  for (int q = 0; q < 25; q++) {
-    D[(size_t)25 * i + q] = Ai[q];
-    D32[(size_t)25 * i + q] = (float)Ai[q];
-  }
+  for (int q = 0; q < 25; q++) D[(size_t)25 * i + q] = (TF)Ai[q];
 }
 
 // z_c = inv(D_c) r_c: one thread per cell
@@ -957,6 +1048,73 @@ __global__ __launch_bounds__(256) void bjac_apply_kernel(int nC, const TF *__res
     bad |= !isfinite(s);
   }
   if (bad) atomicOr(nf, 1u);
+}
+
+// to[src[m]] = m: the packed block of every slot that has one
+__global__ __launch_bounds__(256) void block_pos_kernel(int n, const int *__restrict__ src, int *__restrict__ to) {
+  const int m = blockIdx.x * blockDim.x + threadIdx.x;
+  if (m < n) to[src[m]] = m;
+}
+
+// The factorisation's records (factor_level_kernel) of the rows in level order
+__global__ __launch_bounds__(256) void factor_record_kernel(int n, const int *__restrict__ rows,
+                                                            const int *__restrict__ nbr, const int *__restrict__ rank,
+                                                            const int *__restrict__ bpos, int4 *__restrict__ rec,
+                                                            unsigned *__restrict__ bits) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= n) return;
+  const int i = rows[t], ri = rank[i];
+  unsigned b = 0;
+  int nLow = 0, firstL = 0, firstU = 0, kp[NB] = {-1, -1, -1, -1}, ks[NB] = {0, 0, 0, 0}, ku[NB] = {-1, -1, -1, -1};
+  for (int j = NB - 1; j >= 0; j--) {  // a row's packed blocks follow each other in slot order
+    const int k = nbr[(size_t)NB * i + j];
+    if (k < 0) continue;
+    const int rk = rank[k], pos = bpos[(size_t)NB * i + j];
+    for (int e = 0; e < j; e++) {
+      const int k2 = nbr[(size_t)NB * i + e];
+      for (int f = 0; k2 >= 0 && f < NB; f++)
+        if (nbr[(size_t)NB * k + f] == k2) b |= FAC_FILL;
+    }
+    if (rk > ri) {
+      b |= 1u << j;
+      firstU = pos;
+      continue;
+    }
+    b |= 1u << (4 + j);
+    firstL = pos;
+    int a = nLow++;  // lower neighbours by elimination position (insertion sort of at most NB)
+    for (; a > 0 && kp[a - 1] > rk; a--) { kp[a] = kp[a - 1]; ks[a] = ks[a - 1]; ku[a] = ku[a - 1]; }
+    kp[a] = rk;
+    ks[a] = j;
+    for (int f = 0; f < NB; f++)
+      if (nbr[(size_t)NB * k + f] == i) ku[a] = bpos[(size_t)NB * k + f];
+  }
+  for (int a = 0; a < nLow; a++) b |= (unsigned)ks[a] << (8 + 2 * a);
+  rec[3 * (size_t)t] = make_int4(i, ri, firstL, firstU);
+  rec[3 * (size_t)t + 1] = make_int4(kp[0], kp[1], kp[2], kp[3]);
+  rec[3 * (size_t)t + 2] = make_int4(ku[0], ku[1], ku[2], ku[3]);
+  bits[t] = b | (unsigned)nLow << 16;
+}
+
+int build_factor_records(BlockIlu *b, const std::vector<int> &rows, const std::vector<int> &lsrc,
+                         const std::vector<int> &usrc, hipStream_t s) {
+  const int nC = b->nC;
+  DBuf<int> dRows, dSrc[2];
+  if (dRows.upload(rows.data(), rows.size(), s) || dSrc[0].upload(lsrc.data(), lsrc.size(), s) ||
+      dSrc[1].upload(usrc.data(), usrc.size(), s) || b->dBPos.alloc((size_t)NB * nC) ||
+      b->dFacRec.alloc(3 * (size_t)nC) || b->dFacBits.alloc(nC))
+    return -1;
+  const size_t nSrc[2] = {lsrc.size(), usrc.size()};
+  for (int k = 0; k < 2; k++)
+    if (nSrc[k])
+      hipLaunchKernelGGL(block_pos_kernel, dim3((unsigned)((nSrc[k] + 255) / 256)), dim3(256), 0, s, (int)nSrc[k],
+                         dSrc[k].p, b->dBPos.p);
+  if (nC)
+    hipLaunchKernelGGL(factor_record_kernel, dim3((nC + 255) / 256), dim3(256), 0, s, nC, dRows.p, b->dNbr.p,
+                       b->dRank.p, b->dBPos.p, b->dFacRec.p, b->dFacBits.p);
+  FOS_HIP_TRY(hipGetLastError());
+  FOS_HIP_TRY(hipStreamSynchronize(s));  // the temporaries are freed on return
+  return 0;
 }
 
 int build_ilu_into(fos_euler *ctx, BlockIlu *b);
@@ -982,7 +1140,7 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
   b->nC = nC;
   const char *ev = getenv("FOS_ILU_EAGER");
   b->eager = ev && ev[0] == '1';
-  std::vector<int> nbr((size_t)NB * nC, -1), low((size_t)NB * nC, -1);
+  std::vector<int> nbr((size_t)NB * nC, -1);
   for (int c = 0; c < nC; c++)
     for (int j = 0; j < mf; j++) {
       int e = ctx->hNeib[(size_t)mf * c + j];
@@ -1029,7 +1187,7 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
       }
     }
   }
-  // factorisation levels over the elimination DAG; lower neighbours in elimination order
+  // factorisation levels over the elimination DAG
   std::vector<int> lev(nC, 0);
   int nl = 0;
   // chunks of one colour share no face, so their rows' levels depend only on lower colours and on
@@ -1043,19 +1201,11 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
         const int ch = colChunks[q];
         for (int c = ch * ICH; c < std::min(nC, (ch + 1) * ICH); c++) {
           const int st = rank[c];
-          int m = 0, nlo = 0;
-          int loR[NB], loJ[NB];  // lower neighbours by rank (insertion sort of at most NB)
+          int m = 0;
           for (int j = 0; j < NB; j++) {
             const int k = nbr[(size_t)NB * c + j];
-            if (k >= 0 && rank[k] < st) {
-              m = std::max(m, lev[k] + 1);
-              int a = nlo++;
-              for (; a > 0 && loR[a - 1] > rank[k]; a--) { loR[a] = loR[a - 1]; loJ[a] = loJ[a - 1]; }
-              loR[a] = rank[k];
-              loJ[a] = j;
-            }
+            if (k >= 0 && rank[k] < st) m = std::max(m, lev[k] + 1);
           }
-          for (int a = 0; a < nlo; a++) low[(size_t)NB * c + a] = loJ[a];
           lev[c] = m;
           partMax[pi] = std::max(partMax[pi], m + 1);
         }
@@ -1299,15 +1449,12 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
   }
   b->nLBlk = (long long)lsrc.size();
   b->nUBlk = (long long)usrc.size();
-  if (b->dNbr.upload(nbr.data(), nbr.size(), s) || b->dLowOrd.upload(low.data(), low.size(), s) ||
-      b->dRank.upload(rank.data(), rank.size(), s) || b->dOrder.upload(order.data(), order.size(), s) ||
-      b->dLevRows.upload(rows.data(), rows.size(), s) || b->dJSlot.upload(jslot.data(), jslot.size(), s) ||
-      b->dLSrc.upload(lsrc.data(), lsrc.size(), s) || b->dUSrc.upload(usrc.data(), usrc.size(), s) ||
+  if (b->dNbr.upload(nbr.data(), nbr.size(), s) || b->dRank.upload(rank.data(), rank.size(), s) ||
+      b->dJSlot.upload(jslot.data(), jslot.size(), s) || build_factor_records(b, rows, lsrc, usrc, s) ||
       b->dFMeta.upload(fMeta.data(), fMeta.size(), s) || b->dBMeta.upload(bMeta.data(), bMeta.size(), s) ||
       b->dFRec.upload(fRec.data(), fRec.size(), s) || b->dBRec.upload(bRec.data(), bRec.size(), s) ||
       b->dFOutCell.upload(fOutCell.data(), fOutCell.size(), s) || b->dBOutCell.upload(bOutCell.data(), bOutCell.size(), s) ||
-      b->dJac.alloc(125 * (size_t)nC) || b->dD.alloc(25 * (size_t)nC) || b->dOff.alloc(25 * (size_t)NB * nC) ||
-      b->dD32.alloc(25 * (size_t)nC) || b->dIo.alloc(2) ||
+      b->dJac.alloc(125 * (size_t)nC) || b->dIo.alloc(2) || b->dGamma.alloc(1) ||
       ctx->dStatus.alloc(1))
     return -1;
   return 0;
@@ -1320,52 +1467,43 @@ int jacobian_dev(fos_euler *ctx, const double *y, double *jac) {
   const int nC = ctx->nC;
   if (nC == 0) return 0;
   const int NS = ctx->L64.nSlots;
-  const dim3 blk(256);
+  const dim3 blk(JAC_THREADS);
   const bool exact = ctx->flags & FOS_JAC_EXACT;
+  const dim3 grid((unsigned)(((size_t)nC * NS + JAC_THREADS - 1) / JAC_THREADS));
   if (NS == 4)
-    hipLaunchKernelGGL(exact ? jac_exact_kernel<4> : jac_kernel<4>, dim3((unsigned)(((size_t)nC * 4 + 255) / 256)), blk,
-                       0, ctx->stream, ctx->L64, ctx->ilu->dJSlot.p, y, jac);
+    hipLaunchKernelGGL(exact ? jac_exact_kernel<4> : jac_kernel<4>, grid, blk, 0, ctx->stream, ctx->L64,
+                       ctx->ilu->dJSlot.p, y, jac);
   else
-    hipLaunchKernelGGL(exact ? jac_exact_kernel<8> : jac_kernel<8>, dim3((unsigned)(((size_t)nC * 8 + 255) / 256)), blk,
-                       0, ctx->stream, ctx->L64, ctx->ilu->dJSlot.p, y, jac);
+    hipLaunchKernelGGL(exact ? jac_exact_kernel<8> : jac_kernel<8>, grid, blk, 0, ctx->stream, ctx->L64,
+                       ctx->ilu->dJSlot.p, y, jac);
   FOS_HIP_TRY(hipGetLastError());
   return 0;
 }
 
-// Level-ordered copies of the factors in the apply precision TF.
+// one spare block after the packed ones: the FP32 sweeps' 16-byte aligned pieces may reach past the last run
 template <class TF>
-static int gather_factors(fos_euler *ctx, DBuf<TF> &Lf, DBuf<TF> &Uf, DBuf<TF> &Db) {
-  BlockIlu *b = ctx->ilu;
-  const int nC = ctx->nC;
-  // one spare block each: the FP32 sweeps' 16-byte aligned pieces may reach past the last run
-  if ((!Lf.p && Lf.alloc(25 * (size_t)(b->nLBlk + 1))) || (!Uf.p && Uf.alloc(25 * (size_t)(b->nUBlk + 1))) ||
-      (!Db.p && Db.alloc(25 * (size_t)nC)))
-    return -1;
-  auto go = [&](long long nBlk, const int *src, const double *from, TF *to) {
-    if (nBlk == 0) return;
-    const size_t nt = (size_t)nBlk * 25;
-    hipLaunchKernelGGL(gather_blocks_kernel<TF>, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, ctx->stream, nBlk,
-                       src, from, to);
-  };
-  go(b->nLBlk, b->dLSrc.p, b->dOff.p, Lf.p);
-  go(b->nUBlk, b->dUSrc.p, b->dOff.p, Uf.p);
-  go(nC, b->dOrder.p, b->dD.p, Db.p);
-  FOS_HIP_TRY(hipGetLastError());
-  return 0;
+static int ensure_blocks(DBuf<TF> &b, long long nBlk) {
+  return b.p ? 0 : b.alloc(25 * (size_t)(nBlk + 1));
 }
 
-int ilu_factor(fos_euler *ctx, double gamma) {
+// The pivot status after a factorisation (waits for the stream): 0, 1 for a singular block, -1
+static int factor_status(fos_euler *ctx, const char *what) {
+  int st = 0;
+  FOS_HIP_TRY(hipMemcpyAsync(&st, ctx->dStatus.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
+  if (st == 0x7fffffff) return 0;
+  set_error("%s at cell %d", what, st);
+  return 1;  // recoverable: the integrator may retry with a smaller step
+}
+
+template <class TF>
+static int factor_levels(fos_euler *ctx, double gamma, TF *L, TF *U, TF *D) {
   BlockIlu *b = ctx->ilu;
-  const int nC = ctx->nC;
-  const size_t nt = (size_t)nC * 25 * (1 + NB);
-  hipLaunchKernelGGL(form_m_kernel, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, ctx->stream, nC, b->dJac.p,
-                     ctx->dInvV64.p, b->dNbr.p, gamma, b->dD.p, b->dOff.p);
-  const int big = 0x7fffffff;
-  FOS_HIP_TRY(hipMemcpyAsync(ctx->dStatus.p, &big, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
   auto level = [&](int l, auto &&launch) {
-    const int n = b->levPtr[l + 1] - b->levPtr[l];
-    return launch(factor_level_kernel, dim3((n + 127) / 128), dim3(128), (size_t)0, b->dLevRows.p + b->levPtr[l], n,
-                  b->dNbr.p, b->dLowOrd.p, b->dRank.p, b->dD.p, b->dOff.p, ctx->dStatus.p);
+    const int r = b->levPtr[l], n = b->levPtr[l + 1] - r;
+    return launch(factor_level_kernel<TF>, dim3((n + FAC_ROWS - 1) / FAC_ROWS), dim3(64), (size_t)0,
+                  b->dFacRec.p + 3 * (size_t)r, b->dFacBits.p + r, n, b->dJac.p, ctx->dInvV64.p, b->dGamma.p,
+                  b->dNbr.p, b->dRank.p, b->dBPos.p, b->dUf.p, b->dDb.p, L, U, D, ctx->dStatus.p);
   };
   if (!b->eager && !b->factorChain.ready()) {
     int bad = 0;
@@ -1378,6 +1516,7 @@ int ilu_factor(fos_euler *ctx, double gamma) {
       return -1;
     }
   }
+  hipLaunchKernelGGL(factor_begin_kernel, dim3(1), dim3(64), 0, ctx->stream, b->dGamma.p, gamma, ctx->dStatus.p);
   if (b->eager) {
     for (int l = 0; l < b->nLev; l++)
       level(l, [&](auto k, dim3 g, dim3 blk, size_t lds, auto... a) {
@@ -1389,17 +1528,20 @@ int ilu_factor(fos_euler *ctx, double gamma) {
     return -1;
   }
   FOS_HIP_TRY(hipGetLastError());
-  if ((ctx->flags & FOS_PREC_FP32) ? gather_factors(ctx, b->dLf32, b->dUf32, b->dDb32)
-                                   : gather_factors(ctx, b->dLf, b->dUf, b->dDb))
-    return -1;
-  int st = big;
-  FOS_HIP_TRY(hipMemcpyAsync(&st, ctx->dStatus.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  if (st != big) {
-    set_error("psetup: singular pivot block at cell %d", st);
-    return 1;  // recoverable: the integrator may retry with a smaller step
-  }
   return 0;
+}
+
+int ilu_factor(fos_euler *ctx, double gamma) {
+  BlockIlu *b = ctx->ilu;
+  const bool f32 = ctx->flags & FOS_PREC_FP32;
+  if (ensure_blocks(b->dUf, b->nUBlk) || ensure_blocks(b->dDb, ctx->nC)) return -1;
+  if (f32 ? ensure_blocks(b->dLf32, b->nLBlk) || ensure_blocks(b->dUf32, b->nUBlk) || ensure_blocks(b->dDb32, ctx->nC)
+          : ensure_blocks(b->dLf, b->nLBlk))
+    return -1;
+  if (f32 ? factor_levels(ctx, gamma, b->dLf32.p, b->dUf32.p, b->dDb32.p)
+          : factor_levels(ctx, gamma, b->dLf.p, b->dUf.p, b->dDb.p))
+    return -1;
+  return factor_status(ctx, "psetup: singular pivot block");
 }
 
 // Both sweeps, from b->dIo[0] into b->dIo[1]: the forward sweep one launch per colour in ascending
@@ -1464,33 +1606,30 @@ int ilu_solve(fos_euler *ctx, const double *r, double *z) {
 int bjac_factor(fos_euler *ctx, double gamma) {
   BlockIlu *b = ctx->ilu;
   const int nC = ctx->nC;
-  const size_t nt = (size_t)nC * 25 * (1 + NB);
-  hipLaunchKernelGGL(form_m_kernel, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, ctx->stream, nC, b->dJac.p,
-                     ctx->dInvV64.p, b->dNbr.p, gamma, b->dD.p, b->dOff.p);
-  const int big = 0x7fffffff;
-  FOS_HIP_TRY(hipMemcpyAsync(ctx->dStatus.p, &big, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-  hipLaunchKernelGGL(bjac_invert_kernel, dim3((nC + 127) / 128), dim3(128), 0, ctx->stream, nC, b->dD.p, b->dD32.p,
-                     ctx->dStatus.p);
+  const bool f32 = ctx->flags & FOS_PREC_FP32;
+  if (f32 ? ensure_blocks(b->dBj32, nC) : ensure_blocks(b->dBj, nC)) return -1;
+  hipLaunchKernelGGL(factor_begin_kernel, dim3(1), dim3(64), 0, ctx->stream, b->dGamma.p, gamma, ctx->dStatus.p);
+  const dim3 grid((nC + 127) / 128), blk(128);
+  if (f32)
+    hipLaunchKernelGGL(bjac_invert_kernel<float>, grid, blk, 0, ctx->stream, nC, b->dJac.p, ctx->dInvV64.p, b->dGamma.p,
+                       b->dBj32.p, ctx->dStatus.p);
+  else
+    hipLaunchKernelGGL(bjac_invert_kernel<double>, grid, blk, 0, ctx->stream, nC, b->dJac.p, ctx->dInvV64.p,
+                       b->dGamma.p, b->dBj.p, ctx->dStatus.p);
   FOS_HIP_TRY(hipGetLastError());
-  int st = big;
-  FOS_HIP_TRY(hipMemcpyAsync(&st, ctx->dStatus.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  if (st != big) {
-    set_error("psetup_bjac: singular diagonal block at cell %d", st);
-    return 1;
-  }
-  b->bjac = true;
-  return 0;
+  const int rc = factor_status(ctx, "psetup_bjac: singular diagonal block");
+  if (rc == 0) b->bjac = true;
+  return rc;
 }
 
 int bjac_solve(fos_euler *ctx, const double *r, double *z) {
   BlockIlu *b = ctx->ilu;
   const int nC = ctx->nC;
   if (ctx->flags & FOS_PREC_FP32)
-    hipLaunchKernelGGL(bjac_apply_kernel<float>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dD32.p, r, z,
+    hipLaunchKernelGGL(bjac_apply_kernel<float>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dBj32.p, r, z,
                        ctx->dNonFinite.p);
   else
-    hipLaunchKernelGGL(bjac_apply_kernel<double>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dD.p, r, z,
+    hipLaunchKernelGGL(bjac_apply_kernel<double>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dBj.p, r, z,
                        ctx->dNonFinite.p);
   FOS_HIP_TRY(hipGetLastError());
   return 0;

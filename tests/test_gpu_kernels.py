@@ -36,3 +36,56 @@ def test_fp32_residual_gathers_faces_by_slot(cuda, dims, kind):
     print(f"  relative error {err:.2e}")
     assert err <= 2e-5
     assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])
+
+
+def _centroid_split(pg):
+    """Every tetrahedron split into four around its centroid: the four neighbour each other, so their
+    elimination updates off-diagonal blocks as well (no box mesh has two neighbours of a cell adjacent)."""
+    tet = np.flatnonzero(pg.sE == fa.TET)
+    rest = np.flatnonzero(pg.sE != fa.TET)
+    nd = pg.iNE[tet][:, :4]
+    centre = len(pg.pN) + np.arange(len(tet))
+    kids = np.repeat(nd[:, None, :], 4, 1)
+    for v in range(4):
+        kids[:, v, v] = centre
+    iNE = -np.ones((4 * len(tet) + len(rest), pg.iNE.shape[1]), np.int32)
+    iNE[:4 * len(tet), :4] = kids.reshape(-1, 4)
+    iNE[4 * len(tet):] = pg.iNE[rest]
+    n4 = 4 * len(tet)
+    return fa.PolyGrid(np.concatenate([pg.pN, pg.pN[nd].mean(1)]),
+                       np.concatenate([np.full(n4, fa.TET), pg.sE[rest]]),
+                       np.concatenate([np.full(n4, 4), pg.nNE[rest]]), iNE,
+                       np.concatenate([np.zeros(n4, int), pg.gid[rest]]))
+
+
+@pytest.mark.parametrize("flags,tol", [(0, 1e-10), (fa.PREC_FP32, 1e-5)])
+@pytest.mark.parametrize("dims,split", [((1, 1, 1), True), ((3, 2, 2), True), ((6, 4, 4), True), ((13, 3, 3), False)])
+def test_block_ilu_factorisation_matches_oracle(cuda, dims, split, flags, tol):
+    """The level kernel's rows (five lanes each, 48 to a workgroup) on levels of a few rows, with and
+    without updates of other blocks of the row, at a gamma where the off-diagonal blocks matter.  The
+    tolerances are the ILU tests' own: FP64 1e-10, FP32 factors 1e-5 (100 roundings of 6e-8 to 1e-7)."""
+    print(f"[case] block ilu factorisation dims={dims} split={split} flags={flags}", flush=True)
+    pg = M.box(*dims, 1.0, 0.5, 0.5, jitter=0.2, seed=3)
+    if split:
+        pg = _centroid_split(pg)
+        pg.renumber(fa.RENUMBER_CHUNKS)
+    fv = pg.up()
+    og = O.Grid(pg.pN, pg.sE, pg.nNE, pg.iNE, pg.gid)
+    cg, ct, cp = M.conds("mixed")
+    bc = O.BC(og, cg, ct, cp, r=M.R, gamm=M.GAMMA)
+    nC = og.nC
+    nb = np.where((og.neib >= 0) & (og.neib < nC), og.neib, -1)
+    triangles = sum(k >= 0 and len(set(nb[k]) & set(nb[c]) - {-1}) > 0 for c in range(nC) for k in nb[c])
+    assert (triangles > 0) == split
+    x = M.perturbed_state(og.p[:nC], mach=0.6, seed=8)
+    jac = O.find_euler_jac(og, *O.element_state(og, bc, x), M.GAMMA)
+    eu = fa.Euler(fv, fa.CondTab(cg, ct, cp), r=M.R, gamma=M.GAMMA, flags=flags)
+    y, r = _dev(x), np.random.default_rng(3).standard_normal(5 * nC)
+    z = y.clone()
+    order = eu.ilu_order()
+    for jok, gamma in ((0, 0.1 * np.cbrt(og.v.mean())), (1, 0.02 * np.cbrt(og.v.mean()))):
+        assert eu.psetup(y, y, gamma, jok=jok) == 1 - jok
+        eu.psolve(_dev(r), z, gamma)
+        err = M.rel(z.cpu().numpy(), O.Bilu(og, jac, gamma, order=order).solve(r))
+        print(f"  gamma {gamma:.2e}: relative error {err:.2e}")
+        assert err <= tol
