@@ -51,8 +51,16 @@ struct BlockIlu {
   DBuf<uint2> dFRec, dBRec;
   DBuf<int> dFOutCell, dBOutCell;
   int fMaxOut = 0, bMaxOut = 0;
+  // solve in one launch (ilu_flow_kernel): per cell its row records, the exchange arrays (two copies of
+  // [5 nC] forward and [5 nC] backward values), the counters (ticket, finished workgroups, copy in use)
+  bool flow = false;
+  int flowGrid = 0;  // resident workgroups
+  DBuf<uint2> dFRow, dBRow;
+  DBuf<unsigned long long> dX;
+  DBuf<unsigned> dCtl;
   DBuf<const double *> dIo;  // [2] the current apply's right-hand side r and result z (SoA, by cell)
-  // level sequences replayed as graphs (FOS_ILU_EAGER=1 in the environment launches them one by one)
+  // level sequences replayed as graphs (FOS_ILU_EAGER=1 in the environment launches them one by one, and
+  // sweeps by colour on every mesh)
   bool eager = false;
   KernelChain factorChain, solveChain;
 };
@@ -620,9 +628,12 @@ __host__ __device__ inline unsigned rec_nb(uint2 rc, int j) {
   return ((rc.x >> (8 * j)) & 255u) | ((rc.y >> (16 + j)) & 1u) << 8;
 }
 
+// Row records (solve in one launch): per cell the same uint2 with the row's in-chunk level in y bits 0-7
+// (0 .. ICH - 1; a level reads rows of lower ones) instead of its local index.
+//
 // Per launch slot of a colour launch (chunks in launch order), two int4: {first cell c0, first step
 // record s0, steps ns, first outside entry o0}, {outside entries nOut, first packed block, first
-// elimination position pb, 0}.
+// elimination position pb, in-chunk levels}.
 //
 // dynamic LDS of a colour-sweep launch: 5 ICH doubles of row values, 5 SWEEP_ROWS doubles of
 // exchange, 5 maxOut outside values
@@ -1003,6 +1014,154 @@ __global__ __launch_bounds__(64) void bwd_colour_kernel(int nC, const int4 *__re
   if (bad) atomicOr(nf, 1u);
 }
 
+// ---------------------------------------------------------------- the solve in one launch
+//
+// On small meshes the colour launches are latency: 18 dependent launches of ~9 us, each with three
+// dependent reads before its first step and one per step after, since a launch starts with cold L2s.
+// Here one launch does both sweeps.  Its items are the chunks' forward sweeps in colour order, then
+// their backward sweeps in reverse; a workgroup takes items by ticket, in order, so an item waits only
+// for items taken earlier by workgroups that are already running: whatever the dispatch order or the
+// number of resident workgroups, the first unfinished item can always proceed.  A lane owns one
+// component of one row (12 rows to a wave, 6 waves to a chunk), loads its blocks into registers while
+// the item waits, and the chunk's in-chunk levels then run out of LDS, a barrier each.
+// A value is published with one 8-byte store at agent scope and is its own flag: the exchange array
+// holds FLOW_EMPTY (a NaN no result is stored as) until then, and readers load it at agent scope until
+// it differs.  Nothing else passes between workgroups, so no fence is needed.  Two copies of the array
+// alternate: each apply clears the other one, and the last workgroup to finish resets the counters and
+// swaps the copies, so the state lives on the device (replays of a captured apply included).  A wait is
+// bounded (FLOW_MAX_POLLS, seconds): past it the value is a NaN, which the callback reports.
+// The arithmetic per row is the colour kernels', in the same order: the results are bitwise the same.
+// Per apply, colour launches -> one launch (FP64): 6,000 tets 136 -> 52 us, 24,000 174 -> 67, 270,000
+// 233 -> 142, 540,000 267 -> 244; FP32 factors alike.  What is left is the chain: about 3.3 us for each
+// of the 17 colours of both sweeps (publish, see, gather, the levels).
+constexpr int FLOW_THREADS = 384, FLOW_CTL = 32;
+constexpr unsigned long long FLOW_EMPTY = ~0ull;
+constexpr int FLOW_MAX_POLLS = 1 << 22;  // of a memory round trip (~1 us) each
+static_assert(FLOW_THREADS >= MAX_OUT && FLOW_THREADS / 64 * SWEEP_ROWS >= ICH, "a lane per outside cell and per row component");
+
+__device__ inline void flow_put(unsigned long long *X, size_t at, double v) {
+  unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  if (u == FLOW_EMPTY) u = 0x7ff8000000000000ull;  // the one NaN that means "not there yet"
+  __hip_atomic_store(X + at, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// v[c] = X[at + c] for c < N once they are there
+template <int N>
+__device__ inline void flow_get(unsigned long long *X, size_t at, double (&v)[N]) {
+  unsigned long long u[N];
+#pragma unroll
+  for (int c = 0; c < N; c++) u[c] = __hip_atomic_load(X + at + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  for (int polls = 0; polls < FLOW_MAX_POLLS; polls++) {
+    bool there = true;
+#pragma unroll
+    for (int c = 0; c < N; c++)
+      if (u[c] == FLOW_EMPTY) {
+        there = false;
+        u[c] = __hip_atomic_load(X + at + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+    if (there) break;
+    __builtin_amdgcn_s_sleep(1);
+  }
+#pragma unroll
+  for (int c = 0; c < N; c++) v[c] = __longlong_as_double((long long)u[c]);
+}
+
+template <class TF>
+__global__ __launch_bounds__(FLOW_THREADS) void ilu_flow_kernel(
+    int nC, int nCh, const int4 *__restrict__ fMeta, const int4 *__restrict__ bMeta, const uint2 *__restrict__ fRow,
+    const uint2 *__restrict__ bRow, const int *__restrict__ fOut, const int *__restrict__ bOut,
+    const TF *__restrict__ Lf, const TF *__restrict__ Uf, const TF *__restrict__ Db, const double *r, double *z,
+    unsigned long long *X, unsigned *ctl, unsigned *__restrict__ nf) {
+  __shared__ double sv[5 * ICH], so[5 * MAX_OUT], sT[FLOW_THREADS / 64 * 64];
+  __shared__ unsigned sItem[2];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, slot = lane / 5, q = lane - 5 * slot;
+  const int row = wave * SWEEP_ROWS + slot;
+  if (threadIdx.x == 0) {
+    sItem[0] = atomicAdd(ctl, 1u);
+    sItem[1] = __hip_atomic_load(ctl + 2 * FLOW_CTL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __syncthreads();
+  const size_t nv = 5 * (size_t)nC;
+  unsigned item = sItem[0];
+  const unsigned par = sItem[1] & 1u;
+  unsigned long long *Xf = X + 2 * nv * par, *Xb = Xf + nv, *clr = X + 2 * nv * (par ^ 1u);
+  bool bad = false;
+  while (item < 2u * (unsigned)nCh) {
+    unsigned next = 0;
+    if (threadIdx.x == 0) next = atomicAdd(ctl, 1u);
+    const bool fwd = item < (unsigned)nCh;
+    const int4 *meta = fwd ? fMeta + 2 * item : bMeta + 2 * (2u * nCh - 1u - item);
+    const int4 m0 = meta[0], m1 = meta[1];
+    const int c0 = m0.x, o0 = m0.w, nOut = m1.x, blk0 = m1.y, pb = m1.z, nLev = m1.w;
+    const bool act = slot < SWEEP_ROWS && row < min(ICH, nC - c0);
+    const size_t mine = 5 * (size_t)(c0 + row) + q;
+    uint2 rc = make_uint2(~0u, 0xF00FFu);  // no neighbours, a level that does not come
+    double own = 0.0;
+    int oc = 0;
+    if (act) {
+      rc = (fwd ? fRow : bRow)[c0 + row];
+      if (fwd) own = r[(size_t)q * nC + c0 + row];
+      __hip_atomic_store(clr + (fwd ? 0 : nv) + mine, FLOW_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if ((int)threadIdx.x < nOut) oc = (fwd ? fOut : bOut)[o0 + threadIdx.x];
+    TF B[4][5], Dq[5];
+    if (act) {
+      load_blocks(rc, fwd ? Lf : Uf, blk0, q, B);
+      if (!fwd)
+#pragma unroll
+        for (int c = 0; c < 5; c++) Dq[c] = Db[(size_t)25 * (pb + row) + 5 * q + c];
+    }
+    if ((int)threadIdx.x < nOut) {
+      double v[5];
+      flow_get<5>(fwd ? Xf : Xb, 5 * (size_t)oc, v);
+#pragma unroll
+      for (int c = 0; c < 5; c++) so[5 * threadIdx.x + c] = v[c];
+    }
+    if (act && !fwd) {
+      double v[1];
+      flow_get<1>(Xf, mine, v);
+      own = v[0];
+    }
+    __syncthreads();
+    for (int l = 0; l < nLev; l++) {
+      if (act && (int)(rc.y & 255u) == l) {
+        double v = own - nb_dot(rc, B, sv, so);
+        if (!fwd) {
+          sT[64 * wave + lane] = v;
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          v = 0.0;
+#pragma unroll
+          for (int c = 0; c < 5; c++) v += (double)Dq[c] * sT[64 * wave + 5 * slot + c];
+          bad |= !isfinite(v);
+        }
+        sv[5 * row + q] = v;
+        flow_put(fwd ? Xf : Xb, mine, v);
+      }
+      __syncthreads();
+    }
+    if (!fwd && threadIdx.x < ICH && (int)threadIdx.x < nC - c0)
+#pragma unroll
+      for (int c = 0; c < 5; c++) z[(size_t)c * nC + c0 + threadIdx.x] = sv[5 * threadIdx.x + c];
+    if (threadIdx.x == 0) sItem[0] = next;
+    __syncthreads();
+    item = sItem[0];
+    __syncthreads();
+  }
+  if (bad) atomicOr(nf, 1u);
+  if (threadIdx.x == 0 && atomicAdd(ctl + FLOW_CTL, 1u) == gridDim.x - 1) {
+    // the last workgroup: every other one has read the parity and taken its last item
+    __hip_atomic_store(ctl, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(ctl + FLOW_CTL, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(ctl + 2 * FLOW_CTL, par ^ 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+}
+
+// an empty exchange and zero counters, once per context
+__global__ __launch_bounds__(256) void flow_clear_kernel(size_t n, unsigned long long *X, unsigned *ctl) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) X[i] = FLOW_EMPTY;
+  if (blockIdx.x == 0 && threadIdx.x < 3) ctl[threadIdx.x * FLOW_CTL] = 0u;
+}
+
 // the current apply's vectors for the recorded sweeps
 __global__ void ilu_io_kernel(const double **io, const double *r, double *z) {
   if (threadIdx.x == 0) {
@@ -1116,6 +1275,12 @@ int build_factor_records(BlockIlu *b, const std::vector<int> &rows, const std::v
   FOS_HIP_TRY(hipStreamSynchronize(s));  // the temporaries are freed on return
   return 0;
 }
+
+// Chunks up to which a solve is one launch: beyond, the exchange's extra traffic (200 bytes a cell, and a
+// ticket per item) costs more than the launches.  Measured per apply, colour launches against one: 8,440
+// chunks FP64 267 / 244 us, FP32 239 / 233; 16,800 chunks 397 / 459 and 322 / 444; 93,750 chunks
+// 1,770 / 2,470 and 1,210 / 2,370.
+constexpr int FLOW_MAX_CHUNKS = 8192;
 
 int build_ilu_into(fos_euler *ctx, BlockIlu *b);
 
@@ -1299,17 +1464,20 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
   struct Sched {  // one range of chunks' steps, records and outside lists
     std::vector<int> outPos, stepRel, outRel;
     std::vector<uint2> rec;
+    std::vector<int> levels;  // per chunk: its number of in-chunk levels
     int nStep = 0, maxOut = 0;
   };
+  b->flow = nCh > 0 && nCh <= FLOW_MAX_CHUNKS && !b->eager;
+  std::vector<uint2> fRow(b->flow ? nC : 0), bRow(b->flow ? nC : 0);
   // packed block sources in step order (each chunk keeps its range; rows in the order of its steps)
   std::vector<int> lsrcStep(lsrc.size()), usrcStep(usrc.size());
   auto schedule = [&](bool fwd, std::vector<int> &stepOff, std::vector<uint2> &rec, std::vector<int> &outOff,
-                      std::vector<int> &outPos, int &maxOut) {
+                      std::vector<int> &outPos, int &maxOut, std::vector<int> &levels, std::vector<uint2> &rowRec) {
     const int cparts = host_parts((size_t)nCh, 1 << 10);
     std::vector<Sched> part(cparts);
     host_parallel((size_t)nCh, cparts, [&](size_t k0_, size_t k1_, int pi) {
       Sched &S = part[pi];
-      std::vector<int> outs, loc(ICH), byLev(ICH), pend(ICH);
+      std::vector<int> outs, loc(ICH), byLev(ICH), pend(ICH), rowLev(ICH);
       const size_t cap = (size_t)(k1_ - k0_) * (ICH + SWEEP_ROWS * 4);  // rows plus padding of a few levels
       S.rec.reserve(cap);
       for (int ch = (int)k0_; ch < (int)k1_; ch++) {
@@ -1332,6 +1500,19 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
           pend[i] = d;  // unfinished rows it waits on
         }
         S.stepRel.push_back(S.nStep);
+        // the rows' in-chunk levels (single-launch solve)
+        int nLev = 0;
+        for (int t = 0; t < n && b->flow; t++) {
+          const int i = fwd ? t : n - 1 - t, c = c0 + i;
+          int h = 0;
+          for (int j = 0; j < NB; j++) {
+            const int k = nbr[(size_t)NB * c + j];
+            if (onSide(c, k)) h = std::max(h, rowLev[k - c0] + 1);
+          }
+          rowLev[i] = h;
+          nLev = std::max(nLev, h + 1);
+        }
+        S.levels.push_back(nLev);
         // the chunk's neighbours outside it, and the records' code for each neighbour
         const int pb = rank[c0];
         outs.clear();
@@ -1384,6 +1565,7 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
               rc.y |= (k >> 8) << (16 + j);
             }
             S.rec.push_back(rc);
+            if (!rowRec.empty()) rowRec[c0 + i] = make_uint2(rc.x, (rc.y & 0xFFF00u) | (unsigned)rowLev[i]);
           }
           for (int a = nr; a < REC_SLOTS; a++) S.rec.push_back(empty);  // pad the step
           for (size_t m = r0; m < S.rec.size(); m++) S.rec[m].y |= (unsigned)(acc - acc0) << REC_BLK_SHIFT;
@@ -1417,6 +1599,7 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
       for (size_t q = 0; q < S.stepRel.size(); q++, ch++) {
         stepOff[ch] = sb + S.stepRel[q];
         outOff[ch] = ob + S.outRel[q];
+        levels[ch] = S.levels[q];
       }
       sb += S.nStep;
       rec.insert(rec.end(), S.rec.begin(), S.rec.end());
@@ -1427,8 +1610,9 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
     outOff[nCh] = (int)outPos.size();
     outPos.push_back(0);  // padding: the kernels' clamped index loads stay inside the list
   };
-  schedule(true, fStepOff, fRec, fOutOff, fOutCell, b->fMaxOut);
-  schedule(false, bStepOff, bRec, bOutOff, bOutCell, b->bMaxOut);
+  std::vector<int> fLevels(nCh), bLevels(nCh);
+  schedule(true, fStepOff, fRec, fOutOff, fOutCell, b->fMaxOut, fLevels, fRow);
+  schedule(false, bStepOff, bRec, bOutOff, bOutCell, b->bMaxOut, bLevels, bRow);
   lsrc.swap(lsrcStep);
   usrc.swap(usrcStep);
   // launch order inside each colour: chunks with the most sweep steps first, so the short ones fill
@@ -1443,9 +1627,9 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
   for (int p = 0; p < nCh; p++) {
     const int ch = colChunks[p];
     fMeta[2 * p] = make_int4(ch * ICH, fStepOff[ch], fStepOff[ch + 1] - fStepOff[ch] - REC_PAD_STEPS, fOutOff[ch]);
-    fMeta[2 * p + 1] = make_int4(fOutOff[ch + 1] - fOutOff[ch], fChunkBlk[ch], chunkStart[ch], 0);
+    fMeta[2 * p + 1] = make_int4(fOutOff[ch + 1] - fOutOff[ch], fChunkBlk[ch], chunkStart[ch], fLevels[ch]);
     bMeta[2 * p] = make_int4(ch * ICH, bStepOff[ch], bStepOff[ch + 1] - bStepOff[ch] - REC_PAD_STEPS, bOutOff[ch]);
-    bMeta[2 * p + 1] = make_int4(bOutOff[ch + 1] - bOutOff[ch], bChunkBlk[ch], chunkStart[ch], 0);
+    bMeta[2 * p + 1] = make_int4(bOutOff[ch + 1] - bOutOff[ch], bChunkBlk[ch], chunkStart[ch], bLevels[ch]);
   }
   b->nLBlk = (long long)lsrc.size();
   b->nUBlk = (long long)usrc.size();
@@ -1454,9 +1638,17 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
       b->dFMeta.upload(fMeta.data(), fMeta.size(), s) || b->dBMeta.upload(bMeta.data(), bMeta.size(), s) ||
       b->dFRec.upload(fRec.data(), fRec.size(), s) || b->dBRec.upload(bRec.data(), bRec.size(), s) ||
       b->dFOutCell.upload(fOutCell.data(), fOutCell.size(), s) || b->dBOutCell.upload(bOutCell.data(), bOutCell.size(), s) ||
+      (b->flow && (b->dFRow.upload(fRow.data(), fRow.size(), s) || b->dBRow.upload(bRow.data(), bRow.size(), s) ||
+                   b->dX.alloc(20 * (size_t)nC) || b->dCtl.alloc(3 * FLOW_CTL))) ||
       b->dJac.alloc(125 * (size_t)nC) || b->dIo.alloc(2) || b->dGamma.alloc(1) ||
       ctx->dStatus.alloc(1))
     return -1;
+  if (b->flow) {
+    hipLaunchKernelGGL(flow_clear_kernel, dim3((unsigned)std::min<size_t>(1024, ((size_t)nC * 20 + 255) / 256)),
+                       dim3(256), 0, s, 20 * (size_t)nC, b->dX.p, b->dCtl.p);
+    FOS_HIP_TRY(hipGetLastError());
+    FOS_HIP_TRY(hipStreamSynchronize(s));
+  }
   return 0;
 }
 
@@ -1570,6 +1762,19 @@ static int ilu_levels(BlockIlu *b, const TF *Lf, const TF *Uf, const TF *Db, uns
 template <class TF>
 static int ilu_sweeps(fos_euler *ctx, const TF *Lf, const TF *Uf, const TF *Db, const double *r, double *z) {
   BlockIlu *b = ctx->ilu;
+  if (b->flow) {
+    if (!b->flowGrid) {
+      int per = 0, cus = 0;
+      FOS_HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ilu_flow_kernel<TF>, FLOW_THREADS, 0));
+      FOS_HIP_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device));
+      b->flowGrid = std::max(1, per * cus);
+    }
+    const int nCh = (b->nC + ICH - 1) / ICH;
+    hipLaunchKernelGGL(ilu_flow_kernel<TF>, dim3(std::min(2 * nCh, b->flowGrid)), dim3(FLOW_THREADS), 0, ctx->stream,
+                       b->nC, nCh, b->dFMeta.p, b->dBMeta.p, b->dFRow.p, b->dBRow.p, b->dFOutCell.p, b->dBOutCell.p,
+                       Lf, Uf, Db, r, z, b->dX.p, b->dCtl.p, ctx->dNonFinite.p);
+    return 0;
+  }
   if (!b->eager && !b->solveChain.ready()) {
     if (ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite.p,
                    [&](auto k, dim3 g, dim3 bl, size_t lds, auto... a) {

@@ -89,3 +89,42 @@ def test_block_ilu_factorisation_matches_oracle(cuda, dims, split, flags, tol):
         err = M.rel(z.cpu().numpy(), O.Bilu(og, jac, gamma, order=order).solve(r))
         print(f"  gamma {gamma:.2e}: relative error {err:.2e}")
         assert err <= tol
+
+
+@pytest.mark.parametrize("flags", [0, fa.PREC_FP32], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (11, 2, 2), (40, 10, 10), (32, 27, 20), (45, 45, 44)],
+                         ids=["6", "264", "24000", "103680", "534600"])
+def test_block_ilu_solve_in_one_launch_equals_colour_launches(cuda, dims, flags, monkeypatch):
+    """The single-launch solve (a partial chunk; fewer and more items than resident workgroups) and, past
+    its size limit, the recorded colour launches, against colour launches one by one: bitwise, over
+    repeated applies (the two copies of the exchange alternate), in place, and after a non-finite
+    right-hand side, which is reported and leaves nothing behind."""
+    import torch
+    print(f"[case] block ilu one launch dims={dims} flags={flags}", flush=True)
+    pg = M.box(*dims, 1.0, 0.5, 0.5, jitter=0.2, seed=3, renumber=fa.RENUMBER_CHUNKS)
+    fv = pg.up()
+    ctab = fa.CondTab(*M.conds("mixed"))
+    nC = fv.nC
+    y = _dev(M.perturbed_state(fv.p[:nC], mach=0.6, seed=8))
+    gamma = 0.1 * np.cbrt(fv.v.mean())
+    monkeypatch.setenv("FOS_ILU_EAGER", "1")
+    eager = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA, flags=flags)
+    assert eager.psetup(y, y, gamma) == 1
+    monkeypatch.delenv("FOS_ILU_EAGER")
+    eu = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA, flags=flags)
+    assert eu.psetup(y, y, gamma) == 1
+    rng = np.random.default_rng(11)
+    for k in range(5):
+        r = _dev(rng.standard_normal(5 * nC))
+        ze, z = torch.zeros_like(r), torch.zeros_like(r)
+        eager.psolve(r, ze, gamma)
+        eu.psolve(r, z, gamma)
+        assert torch.equal(ze, z), (k, float((ze - z).abs().max()))
+        assert float(z.norm()) > 0
+        eu.psolve(r, r, gamma)
+        assert torch.equal(ze, r)
+        if k == 2:
+            bad = _dev(rng.standard_normal(5 * nC))
+            bad[nC // 2] = float("nan")
+            with pytest.raises(RuntimeError, match="non-finite"):
+                eu.psolve(bad, z, gamma)
