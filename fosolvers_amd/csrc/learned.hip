@@ -7,10 +7,9 @@
 // pairs (r, target) at the solver's states, loss |S^-1 (P r - target)|^2.
 //
 // Dense layers run on MFMA: BF16 weights and activations, FP32 accumulation.  The forward layers
-// use v_mfma_f32_16x16x32_bf16 in persistent workgroups (mlp_layer_kernel); the backward data
-// products (gemm_kernel) and the weight gradients (MFMA reductions over cells) use
-// v_mfma_f32_16x16x16_bf16.  FP32 master weights and
-// Adam moments.  Parameter packing (flat FP32): W0[20][128] b0 W1[256][128] b1 W2[256][128] b2
+// and the backward data products use v_mfma_f32_16x16x32_bf16 in persistent workgroups
+// (mlp_layer_kernel), the weight gradients (MFMA reductions over cells) v_mfma_f32_16x16x16_bf16.  FP32
+// master weights and Adam moments.  Parameter packing (flat FP32): W0[20][128] b0 W1[256][128] b1 W2[256][128] b2
 // W3[128][30] b3, the same as the oracle (oracle/learned.c).
 #include <hip/hip_runtime.h>
 
@@ -29,7 +28,13 @@ constexpr int NI = 20, NIP = 32, NH = 128, NO = 30, NOP = 32, NBR = 4;
 constexpr int NPAR = NI * NH + NH + 2 * NH * NH + NH + 2 * NH * NH + NH + NH * NO + NO;
 constexpr int OFF_W0 = 0, OFF_B0 = OFF_W0 + NI * NH, OFF_W1 = OFF_B0 + NH, OFF_B1 = OFF_W1 + 2 * NH * NH;
 constexpr int OFF_W2 = OFF_B1 + NH, OFF_B2 = OFF_W2 + 2 * NH * NH, OFF_W3 = OFF_B2 + NH, OFF_B3 = OFF_W3 + NH * NO;
-constexpr int WG_ROWS = 2048;  // rows per weight-gradient partial
+// The weight-gradient partials of one slice of rows: the layers' [K][N] products, padded as their
+// operands are, then the bias gradients
+constexpr int PW3 = 0, PW2 = PW3 + NH * NOP, PW1 = PW2 + 2 * NH * NH, PW0 = PW1 + 2 * NH * NH, PB3 = PW0 + NIP * NH;
+constexpr int PB2 = PB3 + NOP, PB1 = PB2 + NH, PB0 = PB1 + NH, NPART = PB0 + NH;
+// rows per slice: 512, so that 65,536 rows give each of the 256 CUs work, and more where there would be
+// over 256 slices (whose partials the last pass reads)
+inline int slice_rows(size_t n) { return (int)std::max<size_t>(512, ((n + 255) / 256 + 31) / 32 * 32); }
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -85,71 +90,24 @@ namespace {
 
 // ---------------------------------------------------------------- MFMA GEMMs
 
-// C[r][n0 + c] = sum_k A[r][k] * Bn[n0 + c][k] (+ bias), c < NCB; A bf16 [R][lda], Bn bf16 [NC][K].
 enum { EPI_SILU = 0, EPI_F32 = 1, EPI_DSILU = 2, EPI_BF16 = 3 };
-template <int K, int NCB, int EPI>
-__global__ __launch_bounds__(256) void gemm_kernel(int R, const uint16_t *__restrict__ A, int lda,
-                                                   const uint16_t *__restrict__ Bn, const float *__restrict__ bias,
-                                                   float *__restrict__ pre, int ldp, uint16_t *__restrict__ outb,
-                                                   int ldo, float *__restrict__ outf, int ldf) {
-  constexpr int KP = K + 4;  // padded LDS row (8-byte aligned, spreads banks)
-  __shared__ uint16_t sB[NCB * KP];
-  const int n0 = blockIdx.y * NCB;
-  for (int i = threadIdx.x; i < NCB * K / 4; i += 256) {
-    const int n = (4 * i) / K, k = (4 * i) % K;
-    *reinterpret_cast<uint2 *>(&sB[n * KP + k]) = *reinterpret_cast<const uint2 *>(&Bn[(size_t)(n0 + n) * K + k]);
-  }
-  __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int row0 = blockIdx.x * 64 + wave * 16;
-  const int lr = lane & 15, lk = (lane >> 4) * 4;
-  f32x4 acc[NCB / 16];
-#pragma unroll
-  for (int t = 0; t < NCB / 16; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int arow = row0 + lr;
-#pragma unroll 4
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    bf16x4 a = bf16x4{0, 0, 0, 0};
-    if (arow < R) a = *reinterpret_cast<const bf16x4 *>(&A[(size_t)arow * lda + k0 + lk]);
-#pragma unroll
-    for (int t = 0; t < NCB / 16; t++) {
-      const bf16x4 b = *reinterpret_cast<const bf16x4 *>(&sB[(t * 16 + lr) * KP + k0 + lk]);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
-    }
-  }
-#pragma unroll
-  for (int t = 0; t < NCB / 16; t++)
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int row = row0 + lk + j, col = n0 + t * 16 + lr;
-      if (row >= R) continue;
-      float v = acc[t][j] + (bias ? bias[col] : 0.f);
-      if (EPI == EPI_SILU) {
-        if (pre) pre[(size_t)row * ldp + col] = v;
-        outb[(size_t)row * ldo + col] = f2bf(silu_f(v));
-      } else if (EPI == EPI_F32) {
-        outf[(size_t)row * ldf + col] = v;
-      } else if (EPI == EPI_BF16) {
-        outb[(size_t)row * ldo + col] = f2bf(v);
-      } else {  // EPI_DSILU: multiply by silu'(pre) of the forward pass, store bf16
-        outb[(size_t)row * ldo + col] = f2bf(v * dsilu_f(pre[(size_t)row * ldp + col]));
-      }
-    }
-}
 
-// Forward layer out[r][c] = act(sum_k A[r][k] Bn[c][k] + bias[c]) for all N columns, on the gfx950
+// Layer out[r][c] = epi(sum_k A[r][k] Bn[c][k]) for all N columns -- EPI_SILU and EPI_F32 add the bias
+// (forward), EPI_DSILU multiplies by silu' of the forward pass's pre and EPI_BF16 rounds (the backward
+// data products, which with a column block per workgroup re-read A for every 64 columns) -- on the gfx950
 // v_mfma_f32_16x16x32_bf16 (8 bf16 per lane and operand: lane l holds row l%16 and the k-octet
 // l/16 of each 32-wide k step; A and B use the same octets, so the product sums every k once).
 // Persistent workgroups keep the whole weight matrix in LDS and stream 16-row tiles per wave, the
 // next tile's A fragments loaded while the current tile's MFMAs run, so A is read from HBM once.
 // MEAN: the k >= 128 half of A is the mean of the row's neighbours' k < 128 half (message passing
-// fused into the load: the same sum order and rounding as nbr_mean_kernel, never stored).
+// fused into the load, summed in slot order); meanOut, when given, receives it in the k >= 128 half of
+// A's rows (training: the weight gradients read it).
 template <int K, int N, bool MEAN, int EPI>
-__global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *__restrict__ A, int lda,
+__global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *A, int lda,
                                                         const int *__restrict__ nbr, const uint16_t *__restrict__ Bn,
                                                         const float *__restrict__ bias, float *__restrict__ pre,
                                                         int ldp, uint16_t *__restrict__ outb, int ldo,
-                                                        float *__restrict__ outf, int ldf) {
+                                                        float *__restrict__ outf, int ldf, uint16_t *meanOut) {
   static_assert(K % 32 == 0 && N % 16 == 0 && (!MEAN || K == 256), "layer shape");
   constexpr int KS = K / 32, NT = N / 16, NOCT = K / 8;
   // LDS: row n of Bn as K/8 16-byte octets, octet o stored at o ^ (n & SW): the 16 rows one MFMA
@@ -223,7 +181,7 @@ __global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *_
 #pragma unroll
     for (int st = 0; st < KA; st++) mma(acc, st, a[st]);
     if (MEAN) {
-      // mean over the present neighbours, summed in slot order (as nbr_mean_kernel)
+      // mean over the present neighbours, summed in slot order
       const int d[4] = {nb.x, nb.y, nb.z, nb.w};
       const int cnt = (d[0] >= 0) + (d[1] >= 0) + (d[2] >= 0) + (d[3] >= 0);
       const float ic = cnt ? 1.0f / cnt : 0.f;
@@ -241,6 +199,9 @@ __global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *_
 #pragma unroll
         for (int q = 0; q < 8; q++) o[q] = f2bf(sm[q] * ic);
         mma(acc, KS / 2 + st, *reinterpret_cast<const uint4 *>(o));
+        if (meanOut && tile * 16 + lr < R)
+          *reinterpret_cast<uint4 *>(meanOut + (size_t)(tile * 16 + lr) * lda + K / 2 + 32 * st + 8 * kq) =
+              *reinterpret_cast<const uint4 *>(o);
       }
     }
     const int row = tile * 16 + lr;
@@ -248,6 +209,19 @@ __global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *_
 #pragma unroll
       for (int t = 0; t < NT; t++) {
         const int col = t * 16 + 4 * kq;
+        if (EPI == EPI_BF16 || EPI == EPI_DSILU) {
+          float v[4] = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
+          if (EPI == EPI_DSILU) {
+            const float4 x = *reinterpret_cast<const float4 *>(&pre[(size_t)row * ldp + col]);
+            v[0] *= dsilu_f(x.x);
+            v[1] *= dsilu_f(x.y);
+            v[2] *= dsilu_f(x.z);
+            v[3] *= dsilu_f(x.w);
+          }
+          *reinterpret_cast<uint2 *>(&outb[(size_t)row * ldo + col]) =
+              make_uint2(f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
+          continue;
+        }
         const float4 bb = *reinterpret_cast<const float4 *>(&bias[col]);
         const float v[4] = {acc[t][0] + bb.x, acc[t][1] + bb.y, acc[t][2] + bb.z, acc[t][3] + bb.w};
         if (EPI == EPI_SILU) {
@@ -266,95 +240,163 @@ __global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *_
   }
 }
 
-// Weight gradient partials: part[slice][k][n] = sum_{r in slice} A[r][k] * D[r][n] for a 32x32 block
-// (4 waves, one 16x16 tile each); the row index is the MFMA reduction dimension.
-__global__ __launch_bounds__(256) void wgrad_kernel(int R, const uint16_t *__restrict__ A, int lda,
-                                                    const uint16_t *__restrict__ D, int ldd, int K, int N,
-                                                    float *__restrict__ part) {
-  const int slice = blockIdx.x, kb = blockIdx.y * 32, nb = blockIdx.z * 32;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int k0 = kb + (wave & 1) * 16, n0 = nb + (wave >> 1) * 16;
-  const int lr = lane & 15, lk = (lane >> 4) * 4;
-  f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-  const int rb = slice * WG_ROWS, re = min(R, rb + WG_ROWS);
-  for (int r0 = rb; r0 < re; r0 += 16) {
-    bf16x4 a, b;
+// Weight gradient partials of one slice of rows: w[k][n] = sum_r A[r][k] D[r][n] for KB of A's columns and
+// all N of D's, and from the first column block b[n] = sum_r D[r][n].  The row index is the MFMA
+// reduction dimension, so both operands are needed by column: 32 rows of each are staged in LDS with
+// 16-byte loads (the next 32 in flight) and read back by column, 2 bytes at a time, each value for four
+// MFMAs.  Rows are padded by 16 bytes: the four row groups of a fragment then lie 16 banks apart.  Loaded
+// straight from memory 2 bytes at a time, once per 32 x 32 block, the four products took 64 us each and
+// the bias sums, a workgroup per column, 86 us each (65,536 rows); now 29 us for the wide layers and 17 us
+// for the narrow ones, bias sums included.  What bounds it now is the 2-byte LDS reads.
+template <int KB, int N>
+__global__ __launch_bounds__(256) void wgrad_kernel(int R, int rows, const uint16_t *__restrict__ A, int lda,
+                                                    const uint16_t *__restrict__ D, float *__restrict__ w,
+                                                    float *__restrict__ b) {
+  constexpr int WK = KB == 32 ? 1 : N == 32 ? 4 : 2, WN = 4 / WK;      // waves along k and n
+  constexpr int TK = KB / 16 / WK, TN = N / 16 / WN;                   // 16 x 16 tiles per wave
+  constexpr int SA = KB + 8, SD = N + 8, OA = KB / 8, OD = N / 8;      // LDS rows; octets per row
+  constexpr int LA = (32 * OA + 255) / 256, LD = (32 * OD + 255) / 256;  // octets per thread
+  __shared__ alignas(16) uint16_t sA[32 * SA], sD[32 * SD];
+  __shared__ float sB[256 * 8];
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = (lane >> 4) * 4;
+  const int kc = blockIdx.y * KB, kb = (wave % WK) * TK * 16, nb = (wave / WK) * TN * 16;
+  const int rb = blockIdx.x * rows, re = min(R, rb + rows);
+  uint4 a[LA], d[LD];
+  auto load = [&](int r0) {
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int r = r0 + lk + q;
-      const bool in = r < re;
-      a[q] = in ? (short)A[(size_t)r * lda + k0 + lr] : (short)0;
-      b[q] = in ? (short)D[(size_t)r * ldd + n0 + lr] : (short)0;
+    for (int j = 0; j < LA; j++) {
+      const int o = tid + 256 * j, r = r0 + o / OA;
+      a[j] = o < 32 * OA && r < re ? *reinterpret_cast<const uint4 *>(&A[(size_t)r * lda + kc + 8 * (o % OA)])
+                                   : make_uint4(0u, 0u, 0u, 0u);
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
-  }
 #pragma unroll
-  for (int j = 0; j < 4; j++) part[((size_t)slice * K + k0 + lk + j) * N + n0 + lr] = acc[j];
-}
-
-// grad[k][n] (flat, unpadded to Kr x Nr) = sum over slices; also bias grads from column sums of D
-__global__ void wgrad_reduce(const float *__restrict__ part, int nslice, int K, int N, int Kr, int Nr,
-                             float *__restrict__ g) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= Kr * Nr) return;
-  const int k = i / Nr, n = i % Nr;
-  float s = 0.f;
-  for (int sl = 0; sl < nslice; sl++) s += part[((size_t)sl * K + k) * N + n];
-  g[i] = s;
-}
-
-__global__ void colsum_kernel(int R, const uint16_t *__restrict__ D, int ldd, int Nr, float *__restrict__ g) {
-  __shared__ float sm[256];
-  const int n = blockIdx.x;
-  float s = 0.f;
-  for (int r = threadIdx.x; r < R; r += 256) s += bf2f(D[(size_t)r * ldd + n]);
-  sm[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sm[threadIdx.x] += sm[threadIdx.x + o];
+    for (int j = 0; j < LD; j++) {
+      const int o = tid + 256 * j, r = r0 + o / OD;
+      d[j] = o < 32 * OD && r < re ? *reinterpret_cast<const uint4 *>(&D[(size_t)r * N + 8 * (o % OD)])
+                                   : make_uint4(0u, 0u, 0u, 0u);
+    }
+  };
+  f32x4 acc[TK][TN];
+#pragma unroll
+  for (int i = 0; i < TK; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float cs[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // column sums of this thread's octets of D (one column octet)
+  load(rb);
+  for (int r0 = rb; r0 < re; r0 += 32) {
+#pragma unroll
+    for (int j = 0; j < LA; j++) {
+      const int o = tid + 256 * j;
+      if (o < 32 * OA) *reinterpret_cast<uint4 *>(&sA[(o / OA) * SA + 8 * (o % OA)]) = a[j];
+    }
+#pragma unroll
+    for (int j = 0; j < LD; j++) {
+      const int o = tid + 256 * j;
+      if (o < 32 * OD) *reinterpret_cast<uint4 *>(&sD[(o / OD) * SD + 8 * (o % OD)]) = d[j];
+      const uint16_t *h = reinterpret_cast<const uint16_t *>(&d[j]);
+#pragma unroll
+      for (int e = 0; e < 8; e++) cs[e] += bf2f(h[e]);
+    }
+    if (r0 + 32 < re) load(r0 + 32);
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      bf16x4 fa[TK], fd[TN];
+#pragma unroll
+      for (int i = 0; i < TK; i++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) fa[i][e] = (short)sA[(16 * h + lk + e) * SA + kb + 16 * i + lr];
+#pragma unroll
+      for (int j = 0; j < TN; j++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) fd[j][e] = (short)sD[(16 * h + lk + e) * SD + nb + 16 * j + lr];
+#pragma unroll
+      for (int i = 0; i < TK; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[i], fd[j], acc[i][j], 0, 0, 0);
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0 && n < Nr) g[n] = sm[0];
+  w += (size_t)blockIdx.x * NPART;
+#pragma unroll
+  for (int i = 0; i < TK; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) w[(size_t)(kc + kb + 16 * i + lk + e) * N + nb + 16 * j + lr] = acc[i][j][e];
+  if (blockIdx.y) return;
+  // thread tid summed column octet tid % OD (256 is a multiple of OD)
+#pragma unroll
+  for (int e = 0; e < 8; e++) sB[tid * 8 + e] = cs[e];
+  __syncthreads();
+  if (tid < N) {
+    float s = 0.f;
+    for (int t = tid / 8; t < 256; t += OD) s += sB[t * 8 + tid % 8];
+    b[(size_t)blockIdx.x * NPART + tid] = s;
+  }
+}
+
+// The gradient in the flat parameter order, summed over the slices (64 parameters to a workgroup, its four
+// waves a quarter of the slices each)
+__global__ __launch_bounds__(256) void wgrad_reduce(const float *__restrict__ part, int ns, float *__restrict__ g) {
+  __shared__ float sm[4][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+  float s = 0.f;
+  if (i < NPAR) {
+    int at;
+    if (i < OFF_B0) at = PW0 + i;  // the first NI of NIP rows
+    else if (i < OFF_W1) at = PB0 + i - OFF_B0;
+    else if (i < OFF_B1) at = PW1 + i - OFF_W1;
+    else if (i < OFF_W2) at = PB1 + i - OFF_B1;
+    else if (i < OFF_B2) at = PW2 + i - OFF_W2;
+    else if (i < OFF_W3) at = PB2 + i - OFF_B2;
+    else if (i < OFF_B3) at = PW3 + (i - OFF_W3) / NO * NOP + (i - OFF_W3) % NO;
+    else at = PB3 + i - OFF_B3;
+#pragma unroll 8
+    for (int sl = wave; sl < ns; sl += 4) s += part[(size_t)sl * NPART + at];
+  }
+  sm[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && i < NPAR) g[i] = (sm[0][lane] + sm[1][lane]) + (sm[2][lane] + sm[3][lane]);
 }
 
 // ---------------------------------------------------------------- graph and elementwise kernels
 
-// H[c][128:256] = mean over neighbours of H[nb][0:128]  (8 columns per thread)
-__global__ void nbr_mean_kernel(int R, const int *__restrict__ nbr, uint16_t *__restrict__ H) {
+// Backward of [h, mean_nb h] -> h, then silu': dP[c][k] = (dX[c][k] + sum_nb dX[nb][128+k]/cnt_nb) silu'(pre),
+// 8 columns per thread (by single columns, each thread counting its neighbours' neighbours for itself:
+// 62 us at 65,536 cells, 21 us now)
+__global__ __launch_bounds__(256) void mp_backward_kernel(int R, const int *__restrict__ nbr,
+                                                          const uint16_t *__restrict__ dX,
+                                                          const float *__restrict__ pre, uint16_t *__restrict__ dP) {
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)R * 16) return;
-  const int c = (int)(t >> 4), g = (int)(t & 15) * 8;
-  float s[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  int cnt = 0;
+  if (t >= (size_t)R * (NH / 8)) return;
+  const int c = (int)(t / (NH / 8)), k = (int)(t % (NH / 8)) * 8;
+  const int4 *nb4 = reinterpret_cast<const int4 *>(nbr);
+  const int4 nb = nb4[c];
+  const int d[NBR] = {nb.x, nb.y, nb.z, nb.w};
+  uint4 own = *reinterpret_cast<const uint4 *>(&dX[(size_t)c * 256 + k]), v[NBR];
+  float cnt[NBR];
+#pragma unroll
   for (int j = 0; j < NBR; j++) {
-    const int d = nbr[(size_t)NBR * c + j];
-    if (d < 0) continue;
-    cnt++;
-    const uint4 v = *reinterpret_cast<const uint4 *>(&H[(size_t)d * 256 + g]);
-    const uint16_t *h = reinterpret_cast<const uint16_t *>(&v);
-    for (int q = 0; q < 8; q++) s[q] += bf2f(h[q]);
+    if (d[j] < 0) continue;
+    const int4 q = nb4[d[j]];
+    cnt[j] = (float)((q.x >= 0) + (q.y >= 0) + (q.z >= 0) + (q.w >= 0));
+    v[j] = *reinterpret_cast<const uint4 *>(&dX[(size_t)d[j] * 256 + 128 + k]);
   }
+  const float4 p0 = *reinterpret_cast<const float4 *>(&pre[(size_t)c * NH + k]);
+  const float4 p1 = *reinterpret_cast<const float4 *>(&pre[(size_t)c * NH + k + 4]);
+  const float p[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
   uint16_t o[8];
-  const float ic = cnt ? 1.0f / cnt : 0.f;
-  for (int q = 0; q < 8; q++) o[q] = f2bf(s[q] * ic);
-  *reinterpret_cast<uint4 *>(&H[(size_t)c * 256 + 128 + g]) = *reinterpret_cast<const uint4 *>(o);
-}
-
-// Backward of [h, mean_nb h] -> h, then silu': dP[c][k] = (dX[c][k] + sum_nb dX[nb][128+k]/cnt_nb) silu'(pre)
-__global__ void mp_backward_kernel(int R, const int *__restrict__ nbr, const uint16_t *__restrict__ dX,
-                                   const float *__restrict__ pre, uint16_t *__restrict__ dP) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)R * NH) return;
-  const int c = (int)(t / NH), k = (int)(t % NH);
-  float s = bf2f(dX[(size_t)c * 256 + k]);
-  for (int j = 0; j < NBR; j++) {
-    const int d = nbr[(size_t)NBR * c + j];
-    if (d < 0) continue;
-    int cnt = 0;
-    for (int q = 0; q < NBR; q++) cnt += nbr[(size_t)NBR * d + q] >= 0;
-    s += bf2f(dX[(size_t)d * 256 + 128 + k]) / (float)cnt;
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    float s = bf2f(reinterpret_cast<const uint16_t *>(&own)[e]);
+#pragma unroll
+    for (int j = 0; j < NBR; j++)
+      if (d[j] >= 0) s += bf2f(reinterpret_cast<const uint16_t *>(&v[j])[e]) / cnt[j];
+    o[e] = f2bf(s * dsilu_f(p[e]));
   }
-  dP[(size_t)c * NH + k] = f2bf(s * dsilu_f(pre[(size_t)c * NH + k]));
+  *reinterpret_cast<uint4 *>(&dP[(size_t)c * NH + k]) = *reinterpret_cast<const uint4 *>(o);
 }
 
 // Features (20, zero-padded to 32): U/S, log(v/vmean), 4 area-normals / v^(2/3), gamma c / v^(1/3),
@@ -611,10 +653,17 @@ __global__ void scale_partial(int nC, const double *__restrict__ y, double *__re
   if (threadIdx.x < 3) part[blockIdx.x * 3 + threadIdx.x] = sm[threadIdx.x][0];
 }
 
-__global__ void scale_final(int nb, int nC, const double *__restrict__ part, float *__restrict__ S) {
-  if (threadIdx.x) return;
+// one wave: lane l adds the partials l, l + 64, ...
+__global__ __launch_bounds__(64) void scale_final(int nb, int nC, const double *__restrict__ part,
+                                                  float *__restrict__ S) {
   double a = 0, b = 0, c = 0;
-  for (int i = 0; i < nb; i++) { a += part[3 * i]; b += part[3 * i + 1]; c += part[3 * i + 2]; }
+  for (int i = threadIdx.x; i < nb; i += 64) { a += part[3 * i]; b += part[3 * i + 1]; c += part[3 * i + 2]; }
+  for (int m = 32; m > 0; m >>= 1) {
+    a += __shfl_xor(a, m, 64);
+    b += __shfl_xor(b, m, 64);
+    c += __shfl_xor(c, m, 64);
+  }
+  if (threadIdx.x) return;
   const double ra = sqrt(a / nC), rb = sqrt(b / (3.0 * nC)), rc = sqrt(c / nC);
   const double fl = 1e-6 * rc + 1e-300;
   S[0] = (float)fmax(ra, fl);
@@ -622,22 +671,15 @@ __global__ void scale_final(int nb, int nC, const double *__restrict__ part, flo
   S[4] = (float)fmax(rc, fl);
 }
 
-template <int K, int NCB, int EPI>
-void gemm(hipStream_t s, int R, int NC, const uint16_t *A, int lda, const uint16_t *Bn, const float *bias, float *pre,
-          int ldp, uint16_t *outb, int ldo, float *outf, int ldf) {
-  dim3 g((R + 63) / 64, NC / NCB);
-  hipLaunchKernelGGL((gemm_kernel<K, NCB, EPI>), g, dim3(256), 0, s, R, A, lda, Bn, bias, pre, ldp, outb, ldo, outf, ldf);
-}
-
 template <int K, int N, bool MEAN, int EPI>
 void layer(hipStream_t s, int R, const uint16_t *A, int lda, const int *nbr, const uint16_t *Bn, const float *bias,
-           float *pre, int ldp, uint16_t *outb, int ldo, float *outf, int ldf) {
+           float *pre, int ldp, uint16_t *outb, int ldo, float *outf, int ldf, uint16_t *meanOut = nullptr) {
   const size_t lds = sizeof(uint16_t) * N * K;
   const int tiles = (R + 15) / 16;
   const int per = std::max(1, (int)(160 * 1024 / lds));  // workgroups per CU that the LDS allows
   const int grid = 8 * std::max(1, std::min((tiles + 31) / 32, 32 * std::min(per, 4)));  // a multiple of 8
   hipLaunchKernelGGL((mlp_layer_kernel<K, N, MEAN, EPI>), dim3(grid), dim3(256), lds, s, R, A, lda, nbr, Bn, bias,
-                     pre, ldp, outb, ldo, outf, ldf);
+                     pre, ldp, outb, ldo, outf, ldf, meanOut);
 }
 
 int ensure_fwd(Learned *L, size_t n) {
@@ -651,9 +693,9 @@ int ensure_train(Learned *L, size_t n) {
   if (ensure_fwd(L, n)) return -1;
   if (L->capT >= n) return 0;
   L->capT = n;
-  const size_t ns = (n + WG_ROWS - 1) / WG_ROWS;
+  const size_t rows = slice_rows(n), ns = (n + rows - 1) / rows;
   return (L->pre0.alloc(n * NH) || L->pre1.alloc(n * NH) || L->pre2.alloc(n * NH) || L->rh.alloc(n * 8) ||
-          L->e.alloc(n * 8) || L->ds.alloc(n * 8) || L->part.alloc(ns * 256 * NH) || L->dO16.alloc(n * NOP) ||
+          L->e.alloc(n * 8) || L->ds.alloc(n * 8) || L->part.alloc(ns * NPART) || L->dO16.alloc(n * NOP) ||
           L->dP.alloc(n * NH) || L->dX.alloc(n * 256) || L->bnbr.alloc(n * NBR) ||
           L->red.alloc(std::max<size_t>(1024, (n + 255) / 256 + 8))) ? -1 : 0;
 }
@@ -670,25 +712,16 @@ int compute_scale(fos_euler *ctx, Learned *L, const double *y) {
 int forward(fos_euler *ctx, Learned *L, const double *y, int c0, int R, const int *nbr, double gamma, bool keepPre) {
   hipStream_t s = ctx->stream;
   const float *bias = L->bias.p;
-  const dim3 g16((unsigned)(((size_t)R * 16 + 255) / 256));
   hipLaunchKernelGGL(features_kernel, dim3((R + 255) / 256), dim3(256), 0, s, R, c0, ctx->nC, y, L->geo.p,
                      L->scale.p, gamma, ctx->gamm, L->X.p);
-  // inference fuses the neighbour means into the next layer's loads; training stores them (the
-  // weight gradients read [h, mean h])
+  // the neighbour means are fused into the next layer's loads; training also stores them (the weight
+  // gradients read [h, mean h]) and the layers' inputs to silu
   layer<NIP, NH, false, EPI_SILU>(s, R, L->X.p, NIP, nullptr, L->W0t.p, bias, keepPre ? L->pre0.p : nullptr, NH, L->H0.p,
                                   256, nullptr, 0);
-  if (keepPre) {
-    hipLaunchKernelGGL(nbr_mean_kernel, g16, dim3(256), 0, s, R, nbr, L->H0.p);
-    layer<256, NH, false, EPI_SILU>(s, R, L->H0.p, 256, nbr, L->W1t.p, bias + NH, L->pre1.p, NH, L->H1.p, 256, nullptr,
-                                    0);
-    hipLaunchKernelGGL(nbr_mean_kernel, g16, dim3(256), 0, s, R, nbr, L->H1.p);
-    layer<256, NH, false, EPI_SILU>(s, R, L->H1.p, 256, nbr, L->W2t.p, bias + 2 * NH, L->pre2.p, NH, L->H2.p, NH,
-                                    nullptr, 0);
-  } else {
-    layer<256, NH, true, EPI_SILU>(s, R, L->H0.p, 256, nbr, L->W1t.p, bias + NH, nullptr, NH, L->H1.p, 256, nullptr, 0);
-    layer<256, NH, true, EPI_SILU>(s, R, L->H1.p, 256, nbr, L->W2t.p, bias + 2 * NH, nullptr, NH, L->H2.p, NH, nullptr,
-                                   0);
-  }
+  layer<256, NH, true, EPI_SILU>(s, R, L->H0.p, 256, nbr, L->W1t.p, bias + NH, keepPre ? L->pre1.p : nullptr, NH,
+                                 L->H1.p, 256, nullptr, 0, keepPre ? L->H0.p : nullptr);
+  layer<256, NH, true, EPI_SILU>(s, R, L->H1.p, 256, nbr, L->W2t.p, bias + 2 * NH, keepPre ? L->pre2.p : nullptr, NH,
+                                 L->H2.p, NH, nullptr, 0, keepPre ? L->H1.p : nullptr);
   layer<NH, NOP, false, EPI_F32>(s, R, L->H2.p, NH, nullptr, L->W3t.p, bias + 3 * NH, nullptr, 0, nullptr, 0, L->O.p,
                                  NOP);
   hipLaunchKernelGGL(out_scale_kernel, dim3((R + 255) / 256), dim3(256), 0, s, R, L->X.p, L->O.p);
@@ -784,36 +817,27 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
                      L->dO16.p);
   std::vector<double> parts(gb);
   FOS_HIP_TRY(hipMemcpyAsync(parts.data(), L->red.p, sizeof(double) * gb, hipMemcpyDeviceToHost, s));
-  const int ns = (R + WG_ROWS - 1) / WG_ROWS;
-  float *g = L->grad.p;
-  const dim3 gr((unsigned)(((size_t)R * NH + 255) / 256));
+  const int rows = slice_rows(R), ns = (R + rows - 1) / rows;
+  const dim3 gr((unsigned)(((size_t)R * (NH / 8) + 255) / 256)), blk(256);
+  float *pt = L->part.p;
   // layer 3: dW3 = H2^T dO, db3 = sum dO; dP = (dO W3^T) silu'(pre2)
-  hipLaunchKernelGGL(wgrad_kernel, dim3(ns, NH / 32, NOP / 32), dim3(256), 0, s, R, L->H2.p, NH, L->dO16.p, NOP, NH,
-                     NOP, L->part.p);
-  hipLaunchKernelGGL(wgrad_reduce, dim3((NH * NO + 255) / 256), dim3(256), 0, s, L->part.p, ns, NH, NOP, NH, NO,
-                     g + OFF_W3);
-  hipLaunchKernelGGL(colsum_kernel, dim3(NOP), dim3(256), 0, s, R, L->dO16.p, NOP, NO, g + OFF_B3);
-  gemm<NOP, 64, EPI_DSILU>(s, R, NH, L->dO16.p, NOP, L->W3b.p, nullptr, L->pre2.p, NH, L->dP.p, NH, nullptr, 0);
+  hipLaunchKernelGGL((wgrad_kernel<NH, NOP>), dim3(ns, 1), blk, 0, s, R, rows, L->H2.p, NH, L->dO16.p, pt + PW3, pt + PB3);
+  layer<NOP, NH, false, EPI_DSILU>(s, R, L->dO16.p, NOP, nullptr, L->W3b.p, nullptr, L->pre2.p, NH, L->dP.p, NH,
+                                   nullptr, 0);
   // layers 2 and 1: dW = [h, m]^T dP, db = sum dP; dX = dP W^T; dP <- mp-backward(dX) silu'(pre)
   const uint16_t *Hin[2] = {L->H1.p, L->H0.p};
   const uint16_t *Wb[2] = {L->W2b.p, L->W1b.p};
   float *preIn[2] = {L->pre1.p, L->pre0.p};
-  const int offW[2] = {OFF_W2, OFF_W1}, offB[2] = {OFF_B2, OFF_B1};
+  const int offW[2] = {PW2, PW1}, offB[2] = {PB2, PB1};
   for (int l = 0; l < 2; l++) {
-    hipLaunchKernelGGL(wgrad_kernel, dim3(ns, 256 / 32, NH / 32), dim3(256), 0, s, R, Hin[l], 256, L->dP.p, NH, 256,
-                       NH, L->part.p);
-    hipLaunchKernelGGL(wgrad_reduce, dim3((256 * NH + 255) / 256), dim3(256), 0, s, L->part.p, ns, 256, NH, 256, NH,
-                       g + offW[l]);
-    hipLaunchKernelGGL(colsum_kernel, dim3(NH), dim3(256), 0, s, R, L->dP.p, NH, NH, g + offB[l]);
-    gemm<NH, 64, EPI_BF16>(s, R, 256, L->dP.p, NH, Wb[l], nullptr, nullptr, 0, L->dX.p, 256, nullptr, 0);
-    hipLaunchKernelGGL(mp_backward_kernel, gr, dim3(256), 0, s, R, nb, L->dX.p, preIn[l], L->dP.p);
+    hipLaunchKernelGGL((wgrad_kernel<NH, NH>), dim3(ns, 2), blk, 0, s, R, rows, Hin[l], 256, L->dP.p, pt + offW[l],
+                       pt + offB[l]);
+    layer<NH, 256, false, EPI_BF16>(s, R, L->dP.p, NH, nullptr, Wb[l], nullptr, nullptr, 0, L->dX.p, 256, nullptr, 0);
+    hipLaunchKernelGGL(mp_backward_kernel, gr, blk, 0, s, R, nb, L->dX.p, preIn[l], L->dP.p);
   }
   // layer 0: dW0 = X^T dP, db0
-  hipLaunchKernelGGL(wgrad_kernel, dim3(ns, NIP / 32, NH / 32), dim3(256), 0, s, R, L->X.p, NIP, L->dP.p, NH, NIP, NH,
-                     L->part.p);
-  hipLaunchKernelGGL(wgrad_reduce, dim3((NI * NH + 255) / 256), dim3(256), 0, s, L->part.p, ns, NIP, NH, NI, NH,
-                     g + OFF_W0);
-  hipLaunchKernelGGL(colsum_kernel, dim3(NH), dim3(256), 0, s, R, L->dP.p, NH, NH, g + OFF_B0);
+  hipLaunchKernelGGL((wgrad_kernel<NIP, NH>), dim3(ns, 1), blk, 0, s, R, rows, L->X.p, NIP, L->dP.p, pt + PW0, pt + PB0);
+  hipLaunchKernelGGL(wgrad_reduce, dim3((NPAR + 63) / 64), blk, 0, s, pt, ns, L->grad.p);
   FOS_HIP_TRY(hipGetLastError());
   FOS_HIP_TRY(hipStreamSynchronize(s));
   double l2 = 0.0;

@@ -128,3 +128,39 @@ def test_block_ilu_solve_in_one_launch_equals_colour_launches(cuda, dims, flags,
             bad[nC // 2] = float("nan")
             with pytest.raises(RuntimeError, match="non-finite"):
                 eu.psolve(bad, z, gamma)
+
+
+@pytest.mark.parametrize("start,size", [(0, 1), (7, 33), (256, 517), (3, 1200), (0, 1536)])
+def test_learned_gradient_of_a_batch_matches_oracle(cuda, start, size):
+    """The backward pass on batches that are no multiple of its tiles (16 rows), staged steps (32) or
+    slices (512), from an odd first cell, per parameter block against the FP64 oracle on the batch's
+    sub-mesh.  Tolerance 5e-2: eight BF16 roundings of 2^-9 lie between the inputs and a gradient
+    (1.6e-2 if they all agree in sign), times three for blocks whose cells cancel."""
+    print(f"[case] learned gradient start={start} size={size}", flush=True)
+    from tests.test_gpu_learned import BLOCKS, _random_params, bf16
+    _pg, fv, og, _bc, ctab = M.setup(16, 4, 4, kind="mixed")
+    nC = og.nC
+    assert nC == 1536
+    y = _dev(M.perturbed_state(og.p[:nC], mach=0.7, seed=6, width=0.2))
+    eu = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA)
+    p = _random_params(eu, 5)
+    gamma = 0.02
+    X, S = eu.learned_inputs(y, gamma)
+    rng = np.random.default_rng(1)
+    r = rng.standard_normal(5 * nC) * np.repeat(S, nC)
+    delta = 0.5 * r + 0.1 * rng.standard_normal(5 * nC) * np.repeat(S, nC)
+    cells = slice(start, start + size)
+    nb = np.asarray(og.neib[cells])
+    nb = np.where((nb >= start) & (nb < start + size), nb - start, -1).astype(np.int32)
+
+    def part(v):
+        return np.ascontiguousarray(v.reshape(5, nC)[:, cells]).ravel()
+    loss_o, g_o = O.mlp_loss_grad(np.ascontiguousarray(X[cells]), np.ascontiguousarray(nb), bf16(p), S, part(r),
+                                  part(delta), np.ones(size, np.int32))
+    loss, g = eu.learned_loss_grad(y, _dev(r), _dev(delta), gamma, start, size)
+    assert abs(loss - loss_o) <= 2e-2 * loss_o
+    worst = {k: M.rel(g[a:a + n].astype(np.float64), g_o[a:a + n]) for k, (a, n) in BLOCKS.items()}
+    print("  " + " ".join(f"{k} {e:.1e}" for k, e in worst.items()))
+    assert max(worst.values()) <= 5e-2
+    loss2, g2 = eu.learned_loss_grad(y, _dev(r), _dev(delta), gamma, start, size)
+    assert loss2 == loss and np.array_equal(g, g2)
