@@ -24,7 +24,7 @@
 
 namespace fos {
 
-constexpr int NI = 20, NIP = 32, NH = 128, NO = 30, NOP = 32, NBR = 4;
+constexpr int NI = 20, NIP = 32, NH = 128, NO = 30, NOP = 32, NBR = 4, NTR = 12;
 constexpr int NPAR = NI * NH + NH + 2 * NH * NH + NH + 2 * NH * NH + NH + NH * NO + NO;
 constexpr int OFF_W0 = 0, OFF_B0 = OFF_W0 + NI * NH, OFF_W1 = OFF_B0 + NH, OFF_B1 = OFF_W1 + 2 * NH * NH;
 constexpr int OFF_W2 = OFF_B1 + NH, OFF_B2 = OFF_W2 + 2 * NH * NH, OFF_W3 = OFF_B2 + NH, OFF_B3 = OFF_W3 + NH * NO;
@@ -72,7 +72,7 @@ struct Learned {
   // forward activations (rows = max(nC used for inference, training batch))
   size_t capF = 0, capT = 0;
   DBuf<uint16_t> X, H0, H1, H2;  // X [.][32], H0/H1 [.][256] = (h | mean_nb h), H2 [.][128]
-  DBuf<float> O, t;              // O [.][32] network output, t [.][8] = B^ r^
+  DBuf<float> O, t, kappa;       // O [.][32] network output, t [.][12] = B^ r^ and the weights, kappa [.] output scale
   // training-only buffers (rows = batch)
   DBuf<float> pre0, pre1, pre2, rh, e, ds, part;
   DBuf<uint16_t> dO16, dP, dX;   // dO16 [.][32], dP [.][128], dX [.][256]
@@ -90,88 +90,282 @@ namespace {
 
 // ---------------------------------------------------------------- MFMA GEMMs
 
-enum { EPI_SILU = 0, EPI_F32 = 1, EPI_DSILU = 2, EPI_BF16 = 3 };
+enum { EPI_SILU = 0, EPI_DSILU = 2, EPI_BF16 = 3 };
 
-// Layer out[r][c] = epi(sum_k A[r][k] Bn[c][k]) for all N columns -- EPI_SILU and EPI_F32 add the bias
-// (forward), EPI_DSILU multiplies by silu' of the forward pass's pre and EPI_BF16 rounds (the backward
-// data products, which with a column block per workgroup re-read A for every 64 columns) -- on the gfx950
-// v_mfma_f32_16x16x32_bf16 (8 bf16 per lane and operand: lane l holds row l%16 and the k-octet
-// l/16 of each 32-wide k step; A and B use the same octets, so the product sums every k once).
-// Persistent workgroups keep the whole weight matrix in LDS and stream 16-row tiles per wave, the
-// next tile's A fragments loaded while the current tile's MFMAs run, so A is read from HBM once.
+// One cell's 20 features, zero-padded to 32, as four octets (BF16): U/S, log(v/vmean), 4 area-normals /
+// v^(2/3), gamma c / v^(1/3), |u|/c; from its state U and its 13 geometry features g.
+struct FeatIn {
+  double U[5];
+  float g[13];
+};
+__device__ inline void feat_load(FeatIn &f, int c, int nC, const double *__restrict__ y, const float *__restrict__ geo) {
+#pragma unroll
+  for (int k = 0; k < 5; k++) f.U[k] = y[(size_t)k * nC + c];
+#pragma unroll
+  for (int k = 0; k < 13; k++) f.g[k] = geo[(size_t)13 * c + k];
+}
+__device__ inline void feat_row(const FeatIn &f, const float *__restrict__ S, float vm13, double gamma, double gm,
+                                uint4 (&out)[NIP / 8]) {
+  uint16_t x[NIP];
+#pragma unroll
+  for (int k = 0; k < NIP; k++) x[k] = 0;
+#pragma unroll
+  for (int k = 0; k < 5; k++) x[k] = f2bf((float)(f.U[k] / S[k]));
+#pragma unroll
+  for (int k = 0; k < 13; k++) x[5 + k] = f2bf(f.g[k]);
+  const double ir = 1.0 / f.U[0];
+  const double q2 = (f.U[1] * f.U[1] + f.U[2] * f.U[2] + f.U[3] * f.U[3]) * ir * ir;
+  const double p = (gm - 1.0) * (f.U[4] - 0.5 * f.U[0] * q2);
+  const double cs = sqrt(fmax(gm * p * ir, 1e-300));
+  const double vol13 = exp(f.g[0] / 3.0) * (double)vm13;  // v^(1/3) = exp(log(v/vm)/3) vm^(1/3)
+  x[18] = f2bf((float)(gamma * cs / vol13));
+  x[19] = f2bf((float)(sqrt(q2) / cs));
+#pragma unroll
+  for (int q = 0; q < NIP / 8; q++)
+    out[q] = make_uint4(x[8 * q] | (uint32_t)x[8 * q + 1] << 16, x[8 * q + 2] | (uint32_t)x[8 * q + 3] << 16,
+                        x[8 * q + 4] | (uint32_t)x[8 * q + 5] << 16, x[8 * q + 6] | (uint32_t)x[8 * q + 7] << 16);
+}
+// features of the cells [c0, c0+R) alone (fos_learned_inputs)
+__global__ void features_kernel(int R, int c0, int nC, const double *__restrict__ y, const float *__restrict__ geo,
+                                const float *__restrict__ S, double gamma, double gm, uint16_t *__restrict__ X) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= R) return;
+  FeatIn f;
+  uint4 x[NIP / 8];
+  feat_load(f, c0 + i, nC, y, geo);
+  feat_row(f, S, geo[(size_t)13 * nC], gamma, gm, x);
+#pragma unroll
+  for (int q = 0; q < NIP / 8; q++) reinterpret_cast<uint4 *>(&X[(size_t)i * NIP])[q] = x[q];
+}
+// The output scale: O[c] *= k_c = min(1, x_c[18] (1 + x_c[19])) from the cell's (BF16) features,
+// its CFL number gamma (c + |u|) / v^(1/3) capped at 1: the operator tends to the identity as the
+// time step shrinks, where the Newton matrix I - gamma J differs from I by O(CFL).
+__device__ inline float out_kappa(uint4 octet2) {
+  return fminf(1.f, bf2f((uint16_t)octet2.y) * (1.f + bf2f((uint16_t)(octet2.y >> 16))));
+}
+
+// Layer out[r][c] = epi(sum_k A[r][k] Bn[c][k]) for all N columns -- EPI_SILU adds the bias (forward),
+// EPI_DSILU multiplies by silu' of the forward pass's pre and EPI_BF16 rounds (the backward data
+// products) -- on the gfx950 v_mfma_f32_16x16x32_bf16 (8 bf16 per lane and operand: lane l holds row l%16
+// and the k-octet l/16 of each 32-wide k step; A and B use the same octets, so the product sums every k
+// once).  Persistent workgroups keep the whole weight matrix in LDS and stream 16-row tiles per wave, so
+// A is read from HBM once.
+// The product is formed transposed (weights as the row operand), and the weight rows are dealt to the
+// MFMAs' rows so that a lane ends up with 8 consecutive columns of one row in two accumulators: it stores
+// them as one 16-byte vector, and they are the lane's own k-octet of the next layer.
+// FEAT (layer 0): a wave takes 64 rows at a time; each lane forms one row's features from the state and
+// leaves them in LDS for the four tiles.  kappa receives the rows' output scale and, when given, X the
+// features (training).
 // MEAN: the k >= 128 half of A is the mean of the row's neighbours' k < 128 half (message passing
 // fused into the load, summed in slot order); meanOut, when given, receives it in the k >= 128 half of
 // A's rows (training: the weight gradients read it).
-template <int K, int N, bool MEAN, int EPI>
-__global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *A, int lda,
-                                                        const int *__restrict__ nbr, const uint16_t *__restrict__ Bn,
-                                                        const float *__restrict__ bias, float *__restrict__ pre,
-                                                        int ldp, uint16_t *__restrict__ outb, int ldo,
-                                                        float *__restrict__ outf, int ldf, uint16_t *meanOut) {
-  static_assert(K % 32 == 0 && N % 16 == 0 && (!MEAN || K == 256), "layer shape");
+// TAIL (layer 2): the output layer's 128 x 32 product and the output scale follow on the lane's own
+// octets, so the last hidden layer is not stored (outb, when given, still receives it: training).
+// At 1.5M cells, per layer: 0 with the features 48 + 184 -> 128 us, 1 399 -> 327 us, 2 with the output
+// layer and its scale 399 + 110 + 102 -> 347 us (the whole set-up and apply 1,382 -> 844 us), all bitwise
+// the same.  The mean layers are bound by the latency of the gathers and the arithmetic of the means and
+// silu at two waves per SIMD (64 KB of weights per workgroup); 384 and 512 threads around the same weights
+// were 14 % and 50 % slower (fewer registers per wave, spills).
+struct LayerArgs {
+  int R, lda, ldo;
+  const uint16_t *A, *Bn;
+  const int *nbr;
+  const float *bias;
+  float *pre;        // [R][N], null for inference
+  uint16_t *outb, *meanOut;
+  // FEAT
+  const double *y;
+  const float *geo, *S;
+  double gamma, gm;
+  int c0, nC;
+  uint16_t *X;
+  float *kappa;
+  // TAIL
+  const uint16_t *B3;
+  const float *bias3;
+  float *O;
+};
+// LDS octet slot of octet o in row n: the 16 rows that one operand read touches (8 apart in groups of
+// four) land on distinct bank groups
+template <int NOCT>
+__device__ inline int oct_slot(int n, int o) {
+  return n * NOCT + (o ^ (NOCT >= 16 ? (n & 3) | ((n >> 1) & 12) : (n >> 3) & 3));
+}
+// Memory is read and written with four consecutive lanes on 64 consecutive bytes of a row (lane l: row
+// l / 4, 16-byte piece l % 4); the MFMAs want row l % 16, octet l / 16.  In that order no two neighbouring
+// lanes share a row, every 16 bytes are an access of their own to the L1, and the L1 bounded the mean
+// layers (157M accesses, 69 % of the cycles at 1.5M cells).  The neighbours are summed in memory order, and
+// four lane permutations per octet change the order (to_mfma, from_mfma).
+__device__ inline uint4 lane_perm(int from, uint4 v) {
+  return make_uint4(__builtin_amdgcn_ds_bpermute(4 * from, v.x), __builtin_amdgcn_ds_bpermute(4 * from, v.y),
+                    __builtin_amdgcn_ds_bpermute(4 * from, v.z), __builtin_amdgcn_ds_bpermute(4 * from, v.w));
+}
+constexpr int TPB = 256;
+template <int K, int N, bool FEAT, bool MEAN, bool TAIL, int EPI>
+__global__ __launch_bounds__(TPB) void mlp_layer_kernel(LayerArgs P) {
+  static_assert(K % 32 == 0 && N % 32 == 0 && (!MEAN || K == 256) && (!FEAT || K == NIP) && (!TAIL || N == NH),
+                "layer shape");
   constexpr int KS = K / 32, NT = N / 16, NOCT = K / 8;
-  // LDS: row n of Bn as K/8 16-byte octets, octet o stored at o ^ (n & SW): the 16 rows one MFMA
-  // operand read touches land on 16 distinct octet slots (no bank conflicts, no padding)
-  constexpr int SW = NOCT < 16 ? NOCT - 1 : 15;
   extern __shared__ uint4 lds_raw[];
-  uint4 *sB = lds_raw;
-  for (int i = threadIdx.x; i < N * NOCT; i += blockDim.x) {
+  uint4 *sB = lds_raw, *s3 = lds_raw + N * NOCT;  // TAIL: the output layer's weights; FEAT: the waves' features
+  for (int i = threadIdx.x; i < N * NOCT; i += TPB) {
     const int n = i / NOCT, o = i % NOCT;
-    sB[n * NOCT + (o ^ (n & SW))] = *reinterpret_cast<const uint4 *>(&Bn[(size_t)n * K + 8 * o]);
+    sB[oct_slot<NOCT>(n, o)] = *reinterpret_cast<const uint4 *>(&P.Bn[(size_t)n * K + 8 * o]);
   }
+  if (TAIL)
+    for (int i = threadIdx.x; i < NOP * NH / 8; i += TPB) {
+      const int n = i / (NH / 8), o = i % (NH / 8);
+      s3[oct_slot<NH / 8>(n, o)] = *reinterpret_cast<const uint4 *>(&P.B3[(size_t)n * NH + 8 * o]);
+    }
+  __shared__ float4 sBias[N / 4];
+  if (EPI == EPI_SILU && threadIdx.x < N / 4) sBias[threadIdx.x] = reinterpret_cast<const float4 *>(P.bias)[threadIdx.x];
   __syncthreads();
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, kq = lane >> 4;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lr = lane & 15, kq = lane >> 4, R = P.R;
+  const int mr = lane >> 2, mp = lane & 3;  // row and piece in memory order
+  auto to_mfma = [&](uint4 v) { return lane_perm(4 * lr + kq, v); };
+  auto from_mfma = [&](uint4 v) { return lane_perm(mr + 16 * mp, v); };
+  const int n0 = 8 * (lr >> 2) + (lr & 3);  // this lane's weight row within 32 columns, + 4 for the odd tile
   // XCD-aware tiling: workgroup b runs on XCD b % 8 (round-robin dispatch; the grid is a multiple of
   // 8), and each XCD walks its own contiguous eighth of the tiles, so the rows a tile's neighbours
   // read (nearby in the chunk numbering) sit in the same XCD's L2
-  const int nTiles = (R + 15) / 16, wpb = blockDim.x >> 6;
+  constexpr int ROWS = FEAT ? 64 : 16;  // rows a wave takes at a time
+  const int nTiles = (R + ROWS - 1) / ROWS, wpb = TPB >> 6;
   const int xcd = blockIdx.x & 7, perX = (nTiles + 7) / 8;
   const int tBeg = min(nTiles, xcd * perX), tEnd = min(nTiles, tBeg + perX);
   const int stride = (gridDim.x >> 3) * wpb;
   constexpr int KA = MEAN ? KS / 2 : KS;  // k steps read directly from A
-  // the directly read fragments (and for MEAN the neighbour list) of a tile
-  auto load = [&](int tile, uint4 (&a)[KA], int4 &nb) {
-    const int row = tile * 16 + lr;
-    nb = make_int4(-1, -1, -1, -1);
-    if (tile >= tEnd || row >= R) {
+  auto load_a = [&](int tile, uint4 (&a)[KA]) {
+    const int row = tile * 16 + mr;
+    const bool in = tile < tEnd && row < R;
+    const uint16_t *ar = P.A + (size_t)(in ? row : 0) * P.lda + 8 * mp;
 #pragma unroll
-      for (int st = 0; st < KA; st++) a[st] = make_uint4(0u, 0u, 0u, 0u);
-      return;
-    }
-    const uint16_t *ar = A + (size_t)row * lda + 8 * kq;
+    for (int st = 0; st < KA; st++) a[st] = in ? *reinterpret_cast<const uint4 *>(ar + 32 * st) : make_uint4(0u, 0u, 0u, 0u);
+  };
+  auto load_nb = [&](int tile) {
+    const int row = tile * 16 + mr;
+    return tile < tEnd && row < R ? *reinterpret_cast<const int4 *>(&P.nbr[(size_t)NBR * row]) : make_int4(-1, -1, -1, -1);
+  };
+  constexpr int GN = MEAN ? 4 : 1, GS = MEAN ? KS / 2 : 1;
+  auto load_g = [&](int4 nb, uint4 (&g)[GN][GS]) {
+    const int d[4] = {nb.x, nb.y, nb.z, nb.w};
 #pragma unroll
-    for (int st = 0; st < KA; st++) a[st] = *reinterpret_cast<const uint4 *>(ar + 32 * st);
-    if (MEAN) nb = *reinterpret_cast<const int4 *>(&nbr[(size_t)NBR * row]);
+    for (int j = 0; j < GN; j++)
+#pragma unroll
+      for (int st = 0; st < GS; st++)
+        g[j][st] = d[j] >= 0 ? *reinterpret_cast<const uint4 *>(P.A + (size_t)d[j] * P.lda + 32 * st + 8 * mp)
+                             : make_uint4(0u, 0u, 0u, 0u);
   };
   auto mma = [&](f32x4 (&acc)[NT], int st, uint4 av) {
 #pragma unroll
     for (int t = 0; t < NT; t++) {
-      const int n = t * 16 + lr;
-      const uint4 bv = sB[n * NOCT + ((4 * st + kq) ^ (n & SW))];
-      // transposed product (weights as the row operand): the lane then holds 4 consecutive output
-      // columns of one row, stored as one 8-byte (bf16) or 16-byte (FP32) vector
+      const uint4 bv = sB[oct_slot<NOCT>(32 * (t >> 1) + 4 * (t & 1) + n0, 4 * st + kq)];
       acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, bv), __builtin_bit_cast(bf16x8, av),
                                                        acc[t], 0, 0, 0);
     }
   };
-  uint4 a[KA], an[KA];
-  int4 nb, nbn;
-  int tile = tBeg + (blockIdx.x >> 3) * wpb + wave;
-  load(tile, a, nb);
-  for (; tile < tEnd; tile += stride) {
-    // MEAN: issue this tile's neighbour gathers first, then the next tile's loads; the MFMAs of the
-    // directly read half run while both are in flight
-    uint4 g[MEAN ? 4 : 1][MEAN ? KS / 2 : 1];
-    if (MEAN) {
-      const int d[4] = {nb.x, nb.y, nb.z, nb.w};
+  auto finish = [&](int row0, const f32x4 (&acc)[NT]) {
+    const int row = row0 + lr, mrow = row0 + mr;
+    uint4 hid[N / 32];
 #pragma unroll
-      for (int j = 0; j < 4; j++)
+    for (int u = 0; u < N / 32; u++) {
+      const int col = 32 * u + 8 * kq;
+      float v[8];
 #pragma unroll
-        for (int st = 0; st < KS / 2; st++)
-          g[j][st] = d[j] >= 0 ? *reinterpret_cast<const uint4 *>(A + (size_t)d[j] * lda + 32 * st + 8 * kq)
-                               : make_uint4(0u, 0u, 0u, 0u);
+      for (int e = 0; e < 8; e++) v[e] = acc[2 * u + e / 4][e % 4];
+      if (EPI == EPI_SILU) {
+        const float4 b0 = sBias[col / 4], b1 = sBias[col / 4 + 1];
+        const float bb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] += bb[e];
+        if (P.pre && row < R) {
+          float4 *p4 = reinterpret_cast<float4 *>(&P.pre[(size_t)row * N + col]);
+          p4[0] = make_float4(v[0], v[1], v[2], v[3]);
+          p4[1] = make_float4(v[4], v[5], v[6], v[7]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = silu_f(v[e]);
+      } else if (EPI == EPI_DSILU && row < R) {
+        const float4 *p4 = reinterpret_cast<const float4 *>(&P.pre[(size_t)row * N + col]);
+        const float4 b0 = p4[0], b1 = p4[1];
+        const float bb[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] *= dsilu_f(bb[e]);
+      }
+      hid[u] = make_uint4(f2bf(v[0]) | (uint32_t)f2bf(v[1]) << 16, f2bf(v[2]) | (uint32_t)f2bf(v[3]) << 16,
+                          f2bf(v[4]) | (uint32_t)f2bf(v[5]) << 16, f2bf(v[6]) | (uint32_t)f2bf(v[7]) << 16);
+      if (!TAIL || P.outb) {
+        const uint4 m = from_mfma(hid[u]);
+        if (mrow < R) *reinterpret_cast<uint4 *>(&P.outb[(size_t)mrow * P.ldo + 32 * u + 8 * mp]) = m;
+      }
     }
-    load(tile + stride, an, nbn);
+    if constexpr (TAIL) {
+      f32x4 o3[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int st = 0; st < NH / 32; st++)
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+          o3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+              __builtin_bit_cast(bf16x8, s3[oct_slot<NH / 8>(4 * t + n0, 4 * st + kq)]),
+              __builtin_bit_cast(bf16x8, hid[st]), o3[t], 0, 0, 0);
+      const float k = row < R ? P.kappa[row] : 0.f;
+#pragma unroll
+      for (int t = 0; t < 2; t++) {
+        const float4 bb = *reinterpret_cast<const float4 *>(&P.bias3[8 * kq + 4 * t]);
+        const float4 o = make_float4((o3[t][0] + bb.x) * k, (o3[t][1] + bb.y) * k, (o3[t][2] + bb.z) * k, (o3[t][3] + bb.w) * k);
+        const uint4 m = from_mfma(__builtin_bit_cast(uint4, o));
+        if (mrow < R) *reinterpret_cast<uint4 *>(&P.O[(size_t)mrow * NOP + 8 * mp + 4 * t]) = m;
+      }
+    }
+  };
+  int tile = tBeg + (blockIdx.x >> 3) * wpb + wave;
+  if constexpr (FEAT) {
+    uint4 *sX = s3 + wave * 64 * (NIP / 8);
+    const float vm13 = P.geo[(size_t)13 * P.nC];
+    FeatIn f;
+    auto fetch = [&](int t) {
+      if (t < tEnd && t * 64 + lane < R) feat_load(f, P.c0 + t * 64 + lane, P.nC, P.y, P.geo);
+    };
+    fetch(tile);
+    for (; tile < tEnd; tile += stride) {
+      const int mine = tile * 64 + lane;
+      if (mine < R) {
+        uint4 x[NIP / 8];
+        feat_row(f, P.S, vm13, P.gamma, P.gm, x);
+        P.kappa[mine] = out_kappa(x[2]);
+#pragma unroll
+        for (int q = 0; q < NIP / 8; q++) {
+          sX[lane * (NIP / 8) + (q ^ ((lane >> 2) & 3))] = x[q];
+          if (P.X) reinterpret_cast<uint4 *>(&P.X[(size_t)mine * NIP])[q] = x[q];
+        }
+      }
+      fetch(tile + stride);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __asm__ volatile("" ::: "memory");
+#pragma unroll
+      for (int h = 0; h < 4; h++) {
+        f32x4 acc[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+        const int w = 16 * h + lr;
+        mma(acc, 0, sX[w * (NIP / 8) + (kq ^ ((w >> 2) & 3))]);
+        finish(tile * 64 + 16 * h, acc);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    return;
+  }
+  // Loads run ahead of their use in the registers that the current tile has done with: the next tile's own
+  // rows once its own half is multiplied, its neighbours' rows once the means are formed (so that they are
+  // in flight during the epilogue and the next own half), its neighbour list a tile earlier.
+  uint4 a[KA], g[GN][GS];
+  int4 nb = make_int4(-1, -1, -1, -1), nbn = nb;
+  load_a(tile, a);
+  if (MEAN) {
+    nb = load_nb(tile);
+    nbn = load_nb(tile + stride);
+    load_g(nb, g);
+  }
+  for (; tile < tEnd; tile += stride) {
     // keep the weight fragments in LDS (read per tile) instead of letting them be hoisted into
     // registers, which would cost the occupancy that hides the A loads' latency
     __asm__ volatile("" ::: "memory");
@@ -179,17 +373,18 @@ __global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *A
 #pragma unroll
     for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int st = 0; st < KA; st++) mma(acc, st, a[st]);
+    for (int st = 0; st < KA; st++) mma(acc, st, to_mfma(a[st]));
+    load_a(tile + stride, a);
     if (MEAN) {
       // mean over the present neighbours, summed in slot order
       const int d[4] = {nb.x, nb.y, nb.z, nb.w};
       const int cnt = (d[0] >= 0) + (d[1] >= 0) + (d[2] >= 0) + (d[3] >= 0);
       const float ic = cnt ? 1.0f / cnt : 0.f;
 #pragma unroll
-      for (int st = 0; st < KS / 2; st++) {
+      for (int st = 0; st < GS; st++) {
         float sm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (int j = 0; j < GN; j++) {
           if (d[j] < 0) continue;
           const uint16_t *h = reinterpret_cast<const uint16_t *>(&g[j][st]);
 #pragma unroll
@@ -198,45 +393,16 @@ __global__ __launch_bounds__(256) void mlp_layer_kernel(int R, const uint16_t *A
         uint16_t o[8];
 #pragma unroll
         for (int q = 0; q < 8; q++) o[q] = f2bf(sm[q] * ic);
-        mma(acc, KS / 2 + st, *reinterpret_cast<const uint4 *>(o));
-        if (meanOut && tile * 16 + lr < R)
-          *reinterpret_cast<uint4 *>(meanOut + (size_t)(tile * 16 + lr) * lda + K / 2 + 32 * st + 8 * kq) =
-              *reinterpret_cast<const uint4 *>(o);
+        const uint4 m = *reinterpret_cast<const uint4 *>(o);
+        mma(acc, GS + st, to_mfma(m));
+        if (P.meanOut && tile * 16 + mr < R)
+          *reinterpret_cast<uint4 *>(P.meanOut + (size_t)(tile * 16 + mr) * P.lda + K / 2 + 32 * st + 8 * mp) = m;
       }
+      load_g(nbn, g);
+      nb = nbn;
+      nbn = load_nb(tile + 2 * stride);
     }
-    const int row = tile * 16 + lr;
-    if (row < R) {
-#pragma unroll
-      for (int t = 0; t < NT; t++) {
-        const int col = t * 16 + 4 * kq;
-        if (EPI == EPI_BF16 || EPI == EPI_DSILU) {
-          float v[4] = {acc[t][0], acc[t][1], acc[t][2], acc[t][3]};
-          if (EPI == EPI_DSILU) {
-            const float4 x = *reinterpret_cast<const float4 *>(&pre[(size_t)row * ldp + col]);
-            v[0] *= dsilu_f(x.x);
-            v[1] *= dsilu_f(x.y);
-            v[2] *= dsilu_f(x.z);
-            v[3] *= dsilu_f(x.w);
-          }
-          *reinterpret_cast<uint2 *>(&outb[(size_t)row * ldo + col]) =
-              make_uint2(f2bf(v[0]) | ((uint32_t)f2bf(v[1]) << 16), f2bf(v[2]) | ((uint32_t)f2bf(v[3]) << 16));
-          continue;
-        }
-        const float4 bb = *reinterpret_cast<const float4 *>(&bias[col]);
-        const float v[4] = {acc[t][0] + bb.x, acc[t][1] + bb.y, acc[t][2] + bb.z, acc[t][3] + bb.w};
-        if (EPI == EPI_SILU) {
-          if (pre) *reinterpret_cast<float4 *>(&pre[(size_t)row * ldp + col]) = make_float4(v[0], v[1], v[2], v[3]);
-          const uint32_t lo = f2bf(silu_f(v[0])) | ((uint32_t)f2bf(silu_f(v[1])) << 16);
-          const uint32_t hi = f2bf(silu_f(v[2])) | ((uint32_t)f2bf(silu_f(v[3])) << 16);
-          *reinterpret_cast<uint2 *>(&outb[(size_t)row * ldo + col]) = make_uint2(lo, hi);
-        } else {
-          *reinterpret_cast<float4 *>(&outf[(size_t)row * ldf + col]) = make_float4(v[0], v[1], v[2], v[3]);
-        }
-      }
-    }
-#pragma unroll
-    for (int st = 0; st < KA; st++) a[st] = an[st];
-    nb = nbn;
+    finish(tile * 16, acc);
   }
 }
 
@@ -399,47 +565,10 @@ __global__ __launch_bounds__(256) void mp_backward_kernel(int R, const int *__re
   *reinterpret_cast<uint4 *>(&dP[(size_t)c * NH + k]) = *reinterpret_cast<const uint4 *>(o);
 }
 
-// Features (20, zero-padded to 32): U/S, log(v/vmean), 4 area-normals / v^(2/3), gamma c / v^(1/3),
-// |u|/c.  Cells [c0, c0+R) of the full-mesh state y.
-__global__ void features_kernel(int R, int c0, int nC, const double *__restrict__ y, const float *__restrict__ geo,
-                                const float *__restrict__ S, double gamma, double gm, uint16_t *__restrict__ X) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= R) return;
-  const int c = c0 + i;
-  double U[5];
-  for (int k = 0; k < 5; k++) U[k] = y[(size_t)k * nC + c];
-  uint16_t x[NIP];
-  for (int k = 0; k < NIP; k++) x[k] = 0;
-  for (int k = 0; k < 5; k++) x[k] = f2bf((float)(U[k] / S[k]));
-  const float *gc = geo + (size_t)13 * c;
-  for (int k = 0; k < 13; k++) x[5 + k] = f2bf(gc[k]);
-  const double ir = 1.0 / U[0];
-  const double q2 = (U[1] * U[1] + U[2] * U[2] + U[3] * U[3]) * ir * ir;
-  const double p = (gm - 1.0) * (U[4] - 0.5 * U[0] * q2);
-  const double cs = sqrt(fmax(gm * p * ir, 1e-300));
-  const double vol13 = exp(gc[0] / 3.0) * (double)geo[(size_t)13 * nC];  // v^(1/3) = exp(log(v/vm)/3) vm^(1/3)
-  x[18] = f2bf((float)(gamma * cs / vol13));
-  x[19] = f2bf((float)(sqrt(q2) / cs));
-  uint4 *dst = reinterpret_cast<uint4 *>(&X[(size_t)i * NIP]);
-  const uint4 *src = reinterpret_cast<const uint4 *>(x);
-  for (int k = 0; k < NIP / 8; k++) dst[k] = src[k];
-}
-
-// The output scale: O[c] *= k_c = min(1, x_c[18] (1 + x_c[19])) from the cell's (BF16) features,
-// its CFL number gamma (c + |u|) / v^(1/3) capped at 1: the operator tends to the identity as the
-// time step shrinks, where the Newton matrix I - gamma J differs from I by O(CFL).
-__device__ inline float out_kappa(const uint16_t *__restrict__ X, int i) {
-  return fminf(1.f, bf2f(X[(size_t)i * NIP + 18]) * (1.f + bf2f(X[(size_t)i * NIP + 19])));
-}
-__global__ void out_scale_kernel(int R, const uint16_t *__restrict__ X, float *__restrict__ O) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= R) return;
-  const float k = out_kappa(X, i);
-  for (int q = 0; q < NO; q++) O[(size_t)NOP * i + q] *= k;
-}
-
 // t[c][a] = rhat_a + sum_b O[c][5a+b] rhat_b, rhat = r / S (r: SoA with stride nC, cells [c0, c0+R));
-// the 128-byte output row is read as 16-byte vectors
+// the 128-byte output row is read as 16-byte vectors, and its five weights go beside t, so that
+// apply_z_kernel, which needs them and its neighbours' t, does not read the rows again (1.5M cells: 51 + 77 us
+// -> 61 + 52 us for the two kernels)
 __global__ void apply_t_kernel(int R, int c0, int nC, const float *__restrict__ O, const float *__restrict__ S,
                                const double *__restrict__ r, float *__restrict__ t, float *__restrict__ rh) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -456,7 +585,7 @@ __global__ void apply_t_kernel(int R, int c0, int nC, const float *__restrict__ 
     o[4 * k + 2] = v.z;
     o[4 * k + 3] = v.w;
   }
-  float ta[8];
+  float ta[5];
 #pragma unroll
   for (int a = 0; a < 5; a++) {
     float sa = q[a];
@@ -464,36 +593,34 @@ __global__ void apply_t_kernel(int R, int c0, int nC, const float *__restrict__ 
     for (int b = 0; b < 5; b++) sa += o[5 * a + b] * q[b];
     ta[a] = sa;
   }
-  ta[5] = ta[6] = ta[7] = 0.f;
-  float4 *t4 = reinterpret_cast<float4 *>(t + (size_t)8 * i);
+  const float4 w = o4[7];  // o[28..29]
+  float4 *t4 = reinterpret_cast<float4 *>(t + (size_t)NTR * i);
   t4[0] = make_float4(ta[0], ta[1], ta[2], ta[3]);
-  t4[1] = make_float4(ta[4], 0.f, 0.f, 0.f);
+  t4[1] = make_float4(ta[4], o[25], o[26], o[27]);
+  t4[2] = make_float4(w.x, w.y, 0.f, 0.f);
   if (rh)
     for (int a = 0; a < 5; a++) rh[(size_t)8 * i + a] = q[a];
 }
 
 // z_a[c] = S_a ((1 + s4[c]) t[c][a] + sum_j s_j[c] t[nb_j(c)][a]), s = O[c][25:30]: weights of the
 // 4 face neighbours (neib slot order) and of the cell itself
-__global__ void apply_z_kernel(int R, int nC, const int *__restrict__ nbr, const float *__restrict__ O,
-                               const float *__restrict__ S, const float *__restrict__ t, double *__restrict__ z,
+__global__ void apply_z_kernel(int R, int nC, const int *__restrict__ nbr, const float *__restrict__ S, const float *__restrict__ t, double *__restrict__ z,
                                unsigned *__restrict__ nf) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= R) return;
-  const float4 w0 = reinterpret_cast<const float4 *>(O + (size_t)NOP * c)[6];  // o[24..27]
-  const float2 w1 = reinterpret_cast<const float2 *>(O + (size_t)NOP * c)[14];  // o[28..29]
-  const float sw[5] = {w0.y, w0.z, w0.w, w1.x, w1.y};
+  const float4 *t4 = reinterpret_cast<const float4 *>(t);
+  constexpr int T4 = NTR / 4;
+  const float4 tc0 = t4[T4 * (size_t)c], tc1 = t4[T4 * (size_t)c + 1], tc2 = t4[T4 * (size_t)c + 2];
+  const float sw[5] = {tc1.y, tc1.z, tc1.w, tc2.x, tc2.y}, tc4 = tc1.x;
   const int4 nb = reinterpret_cast<const int4 *>(nbr)[c];
   const int d[4] = {nb.x, nb.y, nb.z, nb.w};
-  const float4 *t4 = reinterpret_cast<const float4 *>(t);
-  const float4 tc0 = t4[2 * (size_t)c];
-  const float tc4 = t4[2 * (size_t)c + 1].x;
   float acc[5] = {(1.f + sw[4]) * tc0.x, (1.f + sw[4]) * tc0.y, (1.f + sw[4]) * tc0.z, (1.f + sw[4]) * tc0.w,
                   (1.f + sw[4]) * tc4};
 #pragma unroll
   for (int j = 0; j < NBR; j++) {
     if (d[j] < 0) continue;
-    const float4 a = t4[2 * (size_t)d[j]];
-    const float a4 = t4[2 * (size_t)d[j] + 1].x;
+    const float4 a = t4[T4 * (size_t)d[j]];
+    const float a4 = t4[T4 * (size_t)d[j] + 1].x;
     acc[0] += sw[j] * a.x;
     acc[1] += sw[j] * a.y;
     acc[2] += sw[j] * a.z;
@@ -520,12 +647,12 @@ __global__ void loss_e_kernel(int R, int c0, int nC, const int *__restrict__ nbr
   if (c < R) {
     const float *o = O + (size_t)NOP * c;
     float zh[5];
-    for (int a = 0; a < 5; a++) zh[a] = (1.f + o[29]) * t[(size_t)8 * c + a];
+    for (int a = 0; a < 5; a++) zh[a] = (1.f + o[29]) * t[(size_t)NTR * c + a];
     int nb[NBR];
     for (int j = 0; j < NBR; j++) {
       nb[j] = nbr[(size_t)NBR * c + j];
       if (nb[j] < 0) continue;
-      for (int a = 0; a < 5; a++) zh[a] += o[25 + j] * t[(size_t)8 * nb[j] + a];
+      for (int a = 0; a < 5; a++) zh[a] += o[25 + j] * t[(size_t)NTR * nb[j] + a];
     }
     float ea[5];
     for (int a = 0; a < 5; a++) {
@@ -537,11 +664,11 @@ __global__ void loss_e_kernel(int R, int c0, int nC, const int *__restrict__ nbr
     for (int j = 0; j < NBR; j++) {
       float g = 0.f;
       if (nb[j] >= 0)
-        for (int a = 0; a < 5; a++) g += ea[a] * t[(size_t)8 * nb[j] + a];
+        for (int a = 0; a < 5; a++) g += ea[a] * t[(size_t)NTR * nb[j] + a];
       ds[(size_t)8 * c + j] = g;
     }
     float g4 = 0.f;
-    for (int a = 0; a < 5; a++) g4 += ea[a] * t[(size_t)8 * c + a];
+    for (int a = 0; a < 5; a++) g4 += ea[a] * t[(size_t)NTR * c + a];
     ds[(size_t)8 * c + 4] = g4;
   }
   sm[threadIdx.x] = l;
@@ -558,7 +685,7 @@ __global__ void loss_e_kernel(int R, int c0, int nC, const int *__restrict__ nbr
 // layer's gradient; bf16 dO [R][32]
 __global__ void loss_dO_kernel(int R, const int *__restrict__ nbr, const float *__restrict__ O,
                                const float *__restrict__ e, const float *__restrict__ rh, const float *__restrict__ ds,
-                               const uint16_t *__restrict__ X, uint16_t *__restrict__ dO) {
+                               const float *__restrict__ kappa, uint16_t *__restrict__ dO) {
   const int c = blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= R) return;
   float dt[5];
@@ -574,7 +701,7 @@ __global__ void loss_dO_kernel(int R, const int *__restrict__ nbr, const float *
     }
   }
   uint16_t *o = dO + (size_t)NOP * c;
-  const float k = out_kappa(X, c);
+  const float k = kappa[c];
   for (int a = 0; a < 5; a++)
     for (int b = 0; b < 5; b++) o[5 * a + b] = f2bf(k * dt[a] * rh[(size_t)8 * c + b]);
   for (int j = 0; j < 5; j++) o[25 + j] = f2bf(k * ds[(size_t)8 * c + j]);
@@ -671,22 +798,20 @@ __global__ __launch_bounds__(64) void scale_final(int nb, int nC, const double *
   S[4] = (float)fmax(rc, fl);
 }
 
-template <int K, int N, bool MEAN, int EPI>
-void layer(hipStream_t s, int R, const uint16_t *A, int lda, const int *nbr, const uint16_t *Bn, const float *bias,
-           float *pre, int ldp, uint16_t *outb, int ldo, float *outf, int ldf, uint16_t *meanOut = nullptr) {
-  const size_t lds = sizeof(uint16_t) * N * K;
-  const int tiles = (R + 15) / 16;
+template <int K, int N, bool FEAT, bool MEAN, bool TAIL, int EPI>
+void layer(hipStream_t s, const LayerArgs &P) {
+  const size_t lds = sizeof(uint16_t) * ((size_t)N * K + (TAIL ? NOP * NH : FEAT ? TPB * NIP : 0));
+  const int rows = FEAT ? 64 : 16, tiles = (P.R + rows - 1) / rows, wpb = TPB / 64;
   const int per = std::max(1, (int)(160 * 1024 / lds));  // workgroups per CU that the LDS allows
-  const int grid = 8 * std::max(1, std::min((tiles + 31) / 32, 32 * std::min(per, 4)));  // a multiple of 8
-  hipLaunchKernelGGL((mlp_layer_kernel<K, N, MEAN, EPI>), dim3(grid), dim3(256), lds, s, R, A, lda, nbr, Bn, bias,
-                     pre, ldp, outb, ldo, outf, ldf, meanOut);
+  const int grid = 8 * std::max(1, std::min((tiles + 8 * wpb - 1) / (8 * wpb), 32 * std::min(per, 1024 / TPB)));
+  hipLaunchKernelGGL((mlp_layer_kernel<K, N, FEAT, MEAN, TAIL, EPI>), dim3(grid), dim3(TPB), lds, s, P);
 }
 
 int ensure_fwd(Learned *L, size_t n) {
   if (L->capF >= n) return 0;
   L->capF = n;
   return (L->X.alloc(n * NIP) || L->H0.alloc(n * 256) || L->H1.alloc(n * 256) || L->H2.alloc(n * NH) ||
-          L->O.alloc(n * NOP) || L->t.alloc(n * 8)) ? -1 : 0;
+          L->O.alloc(n * NOP) || L->t.alloc(n * NTR) || L->kappa.alloc(n)) ? -1 : 0;
 }
 
 int ensure_train(Learned *L, size_t n) {
@@ -712,19 +837,45 @@ int compute_scale(fos_euler *ctx, Learned *L, const double *y) {
 int forward(fos_euler *ctx, Learned *L, const double *y, int c0, int R, const int *nbr, double gamma, bool keepPre) {
   hipStream_t s = ctx->stream;
   const float *bias = L->bias.p;
-  hipLaunchKernelGGL(features_kernel, dim3((R + 255) / 256), dim3(256), 0, s, R, c0, ctx->nC, y, L->geo.p,
-                     L->scale.p, gamma, ctx->gamm, L->X.p);
-  // the neighbour means are fused into the next layer's loads; training also stores them (the weight
-  // gradients read [h, mean h]) and the layers' inputs to silu
-  layer<NIP, NH, false, EPI_SILU>(s, R, L->X.p, NIP, nullptr, L->W0t.p, bias, keepPre ? L->pre0.p : nullptr, NH, L->H0.p,
-                                  256, nullptr, 0);
-  layer<256, NH, true, EPI_SILU>(s, R, L->H0.p, 256, nbr, L->W1t.p, bias + NH, keepPre ? L->pre1.p : nullptr, NH,
-                                 L->H1.p, 256, nullptr, 0, keepPre ? L->H0.p : nullptr);
-  layer<256, NH, true, EPI_SILU>(s, R, L->H1.p, 256, nbr, L->W2t.p, bias + 2 * NH, keepPre ? L->pre2.p : nullptr, NH,
-                                 L->H2.p, NH, nullptr, 0, keepPre ? L->H1.p : nullptr);
-  layer<NH, NOP, false, EPI_F32>(s, R, L->H2.p, NH, nullptr, L->W3t.p, bias + 3 * NH, nullptr, 0, nullptr, 0, L->O.p,
-                                 NOP);
-  hipLaunchKernelGGL(out_scale_kernel, dim3((R + 255) / 256), dim3(256), 0, s, R, L->X.p, L->O.p);
+  // training also stores the features, the means, the last hidden layer and the layers' inputs to silu
+  // (the weight gradients read [h, mean h] as one row); inference keeps the hidden rows at 256 bytes
+  const int ld = keepPre ? 256 : NH;
+  LayerArgs P{};
+  P.R = R;
+  P.lda = P.ldo = ld;
+  P.nbr = nbr;
+  P.kappa = L->kappa.p;
+  P.y = y;
+  P.geo = L->geo.p;
+  P.S = L->scale.p;
+  P.gamma = gamma;
+  P.gm = ctx->gamm;
+  P.c0 = c0;
+  P.nC = ctx->nC;
+  P.X = keepPre ? L->X.p : nullptr;
+  P.Bn = L->W0t.p;
+  P.bias = bias;
+  P.pre = keepPre ? L->pre0.p : nullptr;
+  P.outb = L->H0.p;
+  layer<NIP, NH, true, false, false, EPI_SILU>(s, P);
+  P.A = L->H0.p;
+  P.Bn = L->W1t.p;
+  P.bias = bias + NH;
+  P.pre = keepPre ? L->pre1.p : nullptr;
+  P.outb = L->H1.p;
+  P.meanOut = keepPre ? L->H0.p : nullptr;
+  layer<256, NH, false, true, false, EPI_SILU>(s, P);
+  P.A = L->H1.p;
+  P.Bn = L->W2t.p;
+  P.bias = bias + 2 * NH;
+  P.pre = keepPre ? L->pre2.p : nullptr;
+  P.outb = keepPre ? L->H2.p : nullptr;
+  P.ldo = NH;
+  P.meanOut = keepPre ? L->H1.p : nullptr;
+  P.B3 = L->W3t.p;
+  P.bias3 = bias + 3 * NH;
+  P.O = L->O.p;
+  layer<256, NH, false, true, true, EPI_SILU>(s, P);
   FOS_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -813,7 +964,7 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
                      L->rh.p);
   hipLaunchKernelGGL(loss_e_kernel, dim3(gb), dim3(256), 0, s, R, c0, ctx->nC, nb, L->O.p, L->scale.p, L->t.p, delta,
                      L->e.p, L->ds.p, L->red.p);
-  hipLaunchKernelGGL(loss_dO_kernel, dim3(gb), dim3(256), 0, s, R, nb, L->O.p, L->e.p, L->rh.p, L->ds.p, L->X.p,
+  hipLaunchKernelGGL(loss_dO_kernel, dim3(gb), dim3(256), 0, s, R, nb, L->O.p, L->e.p, L->rh.p, L->ds.p, L->kappa.p,
                      L->dO16.p);
   std::vector<double> parts(gb);
   FOS_HIP_TRY(hipMemcpyAsync(parts.data(), L->red.p, sizeof(double) * gb, hipMemcpyDeviceToHost, s));
@@ -822,8 +973,15 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
   float *pt = L->part.p;
   // layer 3: dW3 = H2^T dO, db3 = sum dO; dP = (dO W3^T) silu'(pre2)
   hipLaunchKernelGGL((wgrad_kernel<NH, NOP>), dim3(ns, 1), blk, 0, s, R, rows, L->H2.p, NH, L->dO16.p, pt + PW3, pt + PB3);
-  layer<NOP, NH, false, EPI_DSILU>(s, R, L->dO16.p, NOP, nullptr, L->W3b.p, nullptr, L->pre2.p, NH, L->dP.p, NH,
-                                   nullptr, 0);
+  LayerArgs P{};
+  P.R = R;
+  P.A = L->dO16.p;
+  P.lda = NOP;
+  P.Bn = L->W3b.p;
+  P.pre = L->pre2.p;
+  P.outb = L->dP.p;
+  P.ldo = NH;
+  layer<NOP, NH, false, false, false, EPI_DSILU>(s, P);
   // layers 2 and 1: dW = [h, m]^T dP, db = sum dP; dX = dP W^T; dP <- mp-backward(dX) silu'(pre)
   const uint16_t *Hin[2] = {L->H1.p, L->H0.p};
   const uint16_t *Wb[2] = {L->W2b.p, L->W1b.p};
@@ -832,7 +990,13 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
   for (int l = 0; l < 2; l++) {
     hipLaunchKernelGGL((wgrad_kernel<NH, NH>), dim3(ns, 2), blk, 0, s, R, rows, Hin[l], 256, L->dP.p, pt + offW[l],
                        pt + offB[l]);
-    layer<NH, 256, false, EPI_BF16>(s, R, L->dP.p, NH, nullptr, Wb[l], nullptr, nullptr, 0, L->dX.p, 256, nullptr, 0);
+    P.A = L->dP.p;
+    P.lda = NH;
+    P.Bn = Wb[l];
+    P.pre = nullptr;
+    P.outb = L->dX.p;
+    P.ldo = 256;
+    layer<NH, 256, false, false, false, EPI_BF16>(s, P);
     hipLaunchKernelGGL(mp_backward_kernel, gr, blk, 0, s, R, nb, L->dX.p, preIn[l], L->dP.p);
   }
   // layer 0: dW0 = X^T dP, db0
@@ -870,7 +1034,7 @@ int learned_psolve(fos_euler *ctx, const double *r, double *z) {
   const int nC = ctx->nC, gb = (nC + 255) / 256;
   hipLaunchKernelGGL(apply_t_kernel, dim3(gb), dim3(256), 0, ctx->stream, nC, 0, nC, L->O.p, L->scale.p, r, L->t.p,
                      nullptr);
-  hipLaunchKernelGGL(apply_z_kernel, dim3(gb), dim3(256), 0, ctx->stream, nC, nC, L->nbr.p, L->O.p, L->scale.p, L->t.p,
+  hipLaunchKernelGGL(apply_z_kernel, dim3(gb), dim3(256), 0, ctx->stream, nC, nC, L->nbr.p, L->scale.p, L->t.p,
                      z, ctx->dNonFinite.p);
   FOS_HIP_TRY(hipGetLastError());
   return 0;

@@ -164,3 +164,30 @@ def test_learned_gradient_of_a_batch_matches_oracle(cuda, start, size):
     assert max(worst.values()) <= 5e-2
     loss2, g2 = eu.learned_loss_grad(y, _dev(r), _dev(delta), gamma, start, size)
     assert loss2 == loss and np.array_equal(g, g2)
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (11, 1, 1), (13, 3, 3), (40, 10, 10)], ids=["6", "66", "702", "24000"])
+def test_learned_apply_matches_oracle_at_tile_edges(cuda, dims):
+    """Inference (features, fused layers, apply) where the last 64-row group or 16-row tile is partial and
+    where a wave walks one tile or several; the learned tests' own BF16 tolerance of 3e-2."""
+    import torch
+    print(f"[case] learned apply dims={dims}", flush=True)
+    from tests.test_gpu_learned import _cells_nbr, _random_params, bf16
+    _pg, fv, og, _bc, ctab = M.setup(*dims, kind="mixed")
+    nC = og.nC
+    y = _dev(M.perturbed_state(og.p[:nC], mach=0.7, seed=4, width=0.2))
+    eu = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA)
+    p = _random_params(eu, 3)
+    gamma = 0.02
+    X, S = eu.learned_inputs(y, gamma)
+    r = np.random.default_rng(0).standard_normal(5 * nC) * np.repeat(S, nC)
+    nbr = _cells_nbr(og)
+    zref = O.mlp_apply(O.mlp_forward(X, nbr, bf16(p)), nbr, S, r)
+    z = torch.zeros_like(y)
+    for _ in range(2):
+        eu.psetup_learned(y, gamma)
+        eu.psolve_learned(_dev(r), z)
+        err = M.rel(z.cpu().numpy(), zref)
+        print(f"  relative error {err:.2e}")
+        assert err <= 3e-2
+        eu.learned_loss_grad(y, _dev(r), _dev(r), gamma, 0, min(nC, 100))  # training overwrites the rows
