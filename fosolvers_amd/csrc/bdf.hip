@@ -25,7 +25,7 @@
 
 #include "../../include/fosolvers_amd.h"
 #include "common.h"
-#include "hip_util.h"
+#include "context.h"
 
 namespace fos {
 namespace {
@@ -138,7 +138,9 @@ __global__ __launch_bounds__(VT) void k_maxratio(size_t n, const double *__restr
   }
 }
 
-__global__ __launch_bounds__(VT) void k_reduce_max(const double *__restrict__ part, int nb, double *__restrict__ out) {
+// (host: the scalar once more, in pinned host memory)
+__global__ __launch_bounds__(VT) void k_reduce_max(const double *__restrict__ part, int nb, double *__restrict__ out,
+                                                   double *__restrict__ host) {
   __shared__ double sm[VT];
   double m = 0.0;
   for (int b = threadIdx.x; b < nb; b += VT) m = fmax(m, part[b]);
@@ -148,7 +150,7 @@ __global__ __launch_bounds__(VT) void k_reduce_max(const double *__restrict__ pa
     if (threadIdx.x < o) sm[threadIdx.x] = fmax(sm[threadIdx.x], sm[threadIdx.x + o]);
     __syncthreads();
   }
-  if (threadIdx.x == 0) out[0] = sm[0];
+  if (threadIdx.x == 0) out[0] = host[0] = sm[0];
 }
 
 // z = a x + b y; z may be x or y (no restrict: the integrator updates vectors in place)
@@ -295,8 +297,9 @@ __global__ __launch_bounds__(VT) void k_bdf_residual(size_t n, double a1, const 
   block_partials(acc, 1, 1, sm, part);
 }
 
+// the sums over the blocks, to the device (out) and, for fetch, to pinned host memory (host)
 __global__ __launch_bounds__(VT) void k_reduce(const double *__restrict__ part, int nb, int nk,
-                                               double *__restrict__ out) {
+                                               double *__restrict__ out, double *__restrict__ host) {
   __shared__ double sm[VT];
   for (int k = 0; k < nk; k++) {
     double s = 0.0;
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(VT) void k_reduce(const double *__restrict__ part, 
       if (threadIdx.x < o) sm[threadIdx.x] += sm[threadIdx.x + o];
       __syncthreads();
     }
-    if (threadIdx.x == 0) out[k] = sm[0];
+    if (threadIdx.x == 0) out[k] = host[k] = sm[0];
     __syncthreads();
   }
 }
@@ -375,22 +378,26 @@ __global__ __launch_bounds__(VT) void k_sub_comb_scale(size_t n, const TV *__res
   }
 }
 
-// x += sum_{k<nk} c_k V_k, or x = sum_k c_k V_k when OVW (x is not read); NK = 0: any nk
+// x += sum_{k<nk} c_k V_k, or x = sum_k c_k V_k when OVW (x is not read); NK = 0: any nk, with the
+// coefficients in device memory (cp) instead of the arguments
+struct CombCoef {
+  double c[32];
+};
 template <class TV, int NK, bool OVW>
-__global__ __launch_bounds__(VT) void k_add_comb(size_t n, const TV *__restrict__ V, size_t ldv, int nk,
-                                                 const double *__restrict__ c, double *__restrict__ x) {
+__global__ __launch_bounds__(VT) void k_add_comb(size_t n, const TV *__restrict__ V, size_t ldv, int nk, CombCoef cv,
+                                                 const double *__restrict__ cp, double *__restrict__ x) {
   const size_t kl = (size_t)(nk > 0 ? nk - 1 : 0), st = (size_t)gridDim.x * VT;
   if (NK == 0) {
     for (size_t i = (size_t)blockIdx.x * VT + threadIdx.x; i < n; i += st) {
       double s = OVW ? 0.0 : x[i];
-      for (int k = 0; k < nk; k++) s += c[k] * (double)V[k * ldv + i];
+      for (int k = 0; k < nk; k++) s += cp[k] * (double)V[k * ldv + i];
       x[i] = s;
     }
     return;
   }
   double ck[NK > 0 ? NK : 1];
 #pragma unroll
-  for (int k = 0; k < NK; k++) ck[k] = k < nk ? c[k] : 0.0;
+  for (int k = 0; k < NK; k++) ck[k] = k < nk ? cv.c[k] : 0.0;
   size_t i = (size_t)blockIdx.x * VT + threadIdx.x;
   for (; i + st < n; i += 2 * st) {
     const size_t i2 = i + st;
@@ -495,7 +502,7 @@ struct fos_bdf {
   DBuf<float> Vf, w2f;  // (w2f: the weights in FP32, for the FP32 basis's inner products)
   DBuf<double> wv, dv;
   std::vector<double> hostY, hostYd;  // host staging for host-vector callbacks
-  double *pinned = nullptr;
+  double *pinned = nullptr, *dpinned = nullptr;  // the reductions' scalars in host memory, and their device address
   size_t npinned = 256;
 
   ~fos_bdf() {
@@ -514,7 +521,7 @@ struct fos_bdf {
                                                    : reinterpret_cast<const TV *>(w2.p);
     if (unit) {  // nk == 0, self
       hipLaunchKernelGGL(k_sumsq, grid(), dim3(VT), 0, stream, (size_t)n, x, part.p);
-      hipLaunchKernelGGL(k_reduce, dim3(1), dim3(VT), 0, stream, part.p, nblocks(), 1, out);
+      hipLaunchKernelGGL(k_reduce, dim3(1), dim3(VT), 0, stream, part.p, nblocks(), 1, out, dpinned);
       FOS_HIP_TRY(hipGetLastError());
       return 0;
     }
@@ -533,7 +540,8 @@ struct fos_bdf {
           hipLaunchKernelGGL((k_dots<TV, NK, false>), grid(), dim3(VT), 0, stream, (size_t)n, Vk, (size_t)n, m, sf, x,
                              xs, theta, wts, part.p);
       });
-      hipLaunchKernelGGL(k_reduce, dim3(1), dim3(VT), 0, stream, part.p, nblocks(), m + sf, out + k0);
+      hipLaunchKernelGGL(k_reduce, dim3(1), dim3(VT), 0, stream, part.p, nblocks(), m + sf, out + k0,
+                         dpinned + k0);
       k0 += m;
     } while (k0 < nk);
     FOS_HIP_TRY(hipGetLastError());
@@ -554,25 +562,35 @@ struct fos_bdf {
                            h, scale, xs, theta, x, outV, outD);
     });
   }
-  // x (+)= V c over nk basis vectors (c on the device); overwrite: x is not read
+  // x (+)= V c over nk basis vectors (c on the host, an argument of the kernel up to 32 of them);
+  // overwrite: x is not read
   template <class TV>
-  void add_comb(const TV *V, int nk, const double *c, bool overwrite, double *x) {
+  int add_comb(const TV *V, int nk, const double *c, bool overwrite, double *x) {
+    CombCoef cv{};
+    if (nk <= 32) {
+      std::copy(c, c + nk, cv.c);
+    } else {
+      FOS_HIP_TRY(hipMemcpyAsync(hcol.p, c, sizeof(double) * nk, hipMemcpyHostToDevice, stream));
+      FOS_HIP_TRY(hipStreamSynchronize(stream));  // c is the caller's
+    }
     with_nk(nk, [&](auto cc) {
       constexpr int NK = decltype(cc)::value;
       if (overwrite)
-        hipLaunchKernelGGL((k_add_comb<TV, NK, true>), grid(), dim3(VT), 0, stream, (size_t)n, V, (size_t)n, nk, c, x);
+        hipLaunchKernelGGL((k_add_comb<TV, NK, true>), grid(), dim3(VT), 0, stream, (size_t)n, V, (size_t)n, nk, cv,
+                           hcol.p, x);
       else
-        hipLaunchKernelGGL((k_add_comb<TV, NK, false>), grid(), dim3(VT), 0, stream, (size_t)n, V, (size_t)n, nk, c, x);
+        hipLaunchKernelGGL((k_add_comb<TV, NK, false>), grid(), dim3(VT), 0, stream, (size_t)n, V, (size_t)n, nk, cv,
+                           hcol.p, x);
     });
+    return 0;
   }
   int wnorm2(const double *x, double *out) { return dots<double>(nullptr, 0, x, out, true); }
-  // copy device scalars to host (pinned) and wait
-  int fetch(const double *dsrc, int cnt, double *h) {
+  // wait for the last reduction's scalars, which it also wrote to pinned host memory
+  int fetch(int cnt, double *h) {
     if (cnt < 0 || (size_t)cnt > npinned) {
       set_error("bdf: %d scalars exceed the host staging buffer (%zu)", cnt, npinned);
       return -1;
     }
-    FOS_HIP_TRY(hipMemcpyAsync(pinned, dsrc, sizeof(double) * cnt, hipMemcpyDeviceToHost, stream));
     FOS_HIP_TRY(hipStreamSynchronize(stream));
     std::memcpy(h, pinned, sizeof(double) * cnt);
     return 0;
@@ -603,7 +621,7 @@ struct fos_bdf {
     } else {
       // CVODE's difference quotient: sigma = 1 / ||v||_WRMS (step weights)
       double nv;
-      if (wnorm2(v, dres.p) || fetch(dres.p, 1, &nv)) return -1;
+      if (wnorm2(v, dres.p) || fetch(1, &nv)) return -1;
       nv = std::sqrt(nv / n);
       if (nv == 0.0) {
         FOS_HIP_TRY(hipMemcpyAsync(out, v, sizeof(double) * n, hipMemcpyDeviceToDevice, stream));
@@ -642,8 +660,38 @@ struct fos_bdf {
   // in its first cycle adds V y to yAcc directly, without writing x and a separate pass y += x.
   int gmres(double gamma, const double *b, double *x, int &iters, bool &conv, double absTol = 0.0,
             double *yAcc = nullptr) {
-    return (flags & FOS_PREC_FP32) ? gmres_t<float>(gamma, b, x, iters, conv, absTol, yAcc)
-                                   : gmres_t<double>(gamma, b, x, iters, conv, absTol, yAcc);
+    const Deferred d(*this);
+    const int rc = (flags & FOS_PREC_FP32) ? gmres_t<float>(gamma, b, x, iters, conv, absTol, yAcc)
+                                           : gmres_t<double>(gamma, b, x, iters, conv, absTol, yAcc);
+    if (rc < 0 && d.eu && hipStreamSynchronize(stream) == hipSuccess) (void)take_nonfinite(d.eu);  // unread
+    return rc;
+  }
+  // While GMRES runs on the library's own Euler callbacks, on this integrator's stream, they leave their
+  // wait and their check for a non-finite result to the fetch of the inner products that follows each of
+  // them (three waits per iteration become one).
+  struct Deferred {
+    fos_euler *eu;
+    explicit Deferred(const fos_bdf &b) : eu(b.own_euler()) {
+      if (eu) eu->defer = true;
+    }
+    ~Deferred() {
+      if (eu) eu->defer = false;
+    }
+  };
+  fos_euler *own_euler() const {
+    const fos_psolve_fn ps = onFallback ? fbSol : psol;
+    const bool ours = (nmv == fos_euler_newton_matvec || nmv == fos_euler_newton_matvec_analytic) && jtimes &&
+                      (!ps || ps == fos_euler_psolve || ps == fos_euler_psolve_bjac || ps == fos_euler_psolve_learned);
+    if (!ours || !ud || (flags & FOS_VECTORS_ON_HOST)) return nullptr;
+    fos_euler *eu = static_cast<fos_euler *>(ud);
+    return eu->stream == stream && !(eu->flags & FOS_ASYNC_CALLBACKS) ? eu : nullptr;
+  }
+  // after a wait: 1 if a deferred callback's result was not finite
+  int deferred_check() {
+    fos_euler *eu = own_euler();
+    if (!eu || !eu->defer || !take_nonfinite(eu)) return 0;
+    set_error("%s: non-finite value in the result", eu->deferWho);
+    return 1;
   }
   template <class TV>
   int gmres_t(double gamma, const double *b, double *x, int &iters, bool &conv, double absTol, double *yAcc) {
@@ -689,7 +737,8 @@ struct fos_bdf {
         r = r0v;
       }
       double bb;
-      if (dots<TV>(nullptr, 0, r, dres.p, true) || fetch(dres.p, 1, &bb)) return -1;  // GMRES's own weights
+      if (dots<TV>(nullptr, 0, r, dres.p, true) || fetch(1, &bb)) return -1;  // GMRES's own weights
+      if (deferred_check()) return 1;
       double beta = std::sqrt(bb);
       if (beta0 < 0) beta0 = beta;
       const double tol = absTol > 0.0 ? absTol : linTol * beta0;
@@ -735,14 +784,18 @@ struct fos_bdf {
         const double theta = precd || !std::isfinite(ritz) ? 1.0 : ritz;
         std::fill(hc.begin(), hc.end(), 0.0);
         std::vector<double> hp(j + 2);
-        if (dots<TV>(V, j + 1, w, hcol.p, true, vj, theta) || fetch(hcol.p, j + 2, hp.data())) return -1;
+        if (dots<TV>(V, j + 1, w, hcol.p, true, vj, theta) || fetch(j + 2, hp.data())) return -1;
+        if (deferred_check()) {
+          iters--;  // not an iteration: its product or preconditioner solve failed
+          return 1;
+        }
         double ww = hp[j + 1], s2 = ww;
         for (int k = 0; k <= j; k++) { hc[k] = hp[k]; s2 -= hp[k] * hp[k]; }
         const TV *shift = vj;
         if (!(s2 >= 0.5 * ww)) {
           sub_comb<TV>(V, j + 1, hcol.p, 1.0, vj, theta, w, nullptr, nullptr);
           shift = nullptr;  // w now holds w' - V h
-          if (dots<TV>(V, j + 1, w, hcol.p, true) || fetch(hcol.p, j + 2, hp.data())) return -1;
+          if (dots<TV>(V, j + 1, w, hcol.p, true) || fetch(j + 2, hp.data())) return -1;
           s2 = hp[j + 1];
           for (int k = 0; k <= j; k++) { hc[k] += hp[k]; s2 -= hp[k] * hp[k]; }
           st.nreorth++;
@@ -777,17 +830,15 @@ struct fos_bdf {
         for (int q = k + 1; q < j; q++) s -= H[(size_t)k * m + q] * yv[q];
         yv[k] = s / H[(size_t)k * m + k];
       }
-      FOS_HIP_TRY(hipMemcpyAsync(hcol.p, yv.data(), sizeof(double) * j, hipMemcpyHostToDevice, stream));
       const bool last = done || iters >= cap || restart == maxRestarts;
       if (yAcc && last && restart == 0) {
-        add_comb<TV>(V, j, hcol.p, false, yAcc);
+        if (add_comb<TV>(V, j, yv.data(), false, yAcc)) return -1;
       } else {
-        add_comb<TV>(V, j, hcol.p, restart == 0, x);
+        if (add_comb<TV>(V, j, yv.data(), restart == 0, x)) return -1;
         if (yAcc && last)
           hipLaunchKernelGGL(k_lin2, grid(), dim3(VT), 0, stream, (size_t)n, 1.0, yAcc, 1.0, x, yAcc);
       }
       FOS_HIP_TRY(hipGetLastError());
-      FOS_HIP_TRY(hipStreamSynchronize(stream));
       if (done) { conv = true; return 0; }
       if (iters >= cap) return 0;
     }
@@ -809,7 +860,7 @@ struct fos_bdf {
   double *znj(int j) { return zn.p + (size_t)j * n; }
   int wrms(const double *x, double &out) {
     double s2;
-    if (wnorm2(x, dres.p) || fetch(dres.p, 1, &s2)) return -1;
+    if (wnorm2(x, dres.p) || fetch(1, &s2)) return -1;
     out = std::sqrt(s2 / (double)n);
     return 0;
   }
@@ -927,9 +978,10 @@ struct fos_bdf {
     }
     const double hlb = 100.0 * tround;
     hipLaunchKernelGGL(k_maxratio, grid(), dim3(VT), 0, stream, (size_t)n, znj(0), znj(1), 0.1, atol, part.p);
-    hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(VT), 0, stream, part.p, nblocks(), dres.p);
+    hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(VT), 0, stream, part.p, nblocks(), dres.p,
+                       dpinned);
     double hubInv;
-    if (fetch(dres.p, 1, &hubInv)) return -1;
+    if (fetch(1, &hubInv)) return -1;
     double hub = 0.1 * tdist;
     if (hub * hubInv > 1.0) hub = 1.0 / hubInv;
     double hg = std::sqrt(hlb * hub);
@@ -1274,7 +1326,8 @@ fos_bdf *fos_bdf_create(int nEq, fos_rhs_fn f, int maxl, fos_psetup_fn pSet, fos
   if (b->y.alloc(n) || b->yn.alloc(n) || b->ynm1.alloc(n) || b->ypred.alloc(n) || b->r0.alloc(n) || b->G.alloc(n) ||
       b->fy.alloc(n) || b->w2.alloc(n) || b->d.alloc(n) || b->tmp.alloc(n) || b->tmp2.alloc(n) ||
       b->Vb.alloc((size_t)(b->maxl + 1) * n) || b->part.alloc((size_t)VB * (DOTS + 1)) || b->dres.alloc(DOTS) ||
-      b->hcol.alloc(64 + b->maxl) || b->scal.alloc(4) || hipHostMalloc((void **)&b->pinned, sizeof(double) * b->npinned) != hipSuccess) {
+      b->hcol.alloc(64 + b->maxl) || b->scal.alloc(4) || hipHostMalloc((void **)&b->pinned, sizeof(double) * b->npinned) != hipSuccess ||
+      hipHostGetDevicePointer((void **)&b->dpinned, b->pinned, 0) != hipSuccess) {
     delete b;
     return nullptr;
   }
@@ -1444,9 +1497,10 @@ int fos_bdf_step(fos_bdf *b, double tOut, double *tRet, double *yOut) {
       hipLaunchKernelGGL(k_bdf_residual, gr, bl, 0, s, n, a1, b->yn.p, a2, b->order >= 2 ? b->ynm1.p : b->yn.p,
                          gamma, b->fy.p, b->y.p, b->w2.p, b->rtol, b->atol, b->G.p, b->part.p,
                          newton == 0 ? b->ypred.p : nullptr, newton == 0 ? b->r0.p : nullptr);
-      hipLaunchKernelGGL(k_reduce, dim3(1), dim3(VT), 0, s, b->part.p, b->nblocks(), 2, b->dres.p);
+      hipLaunchKernelGGL(k_reduce, dim3(1), dim3(VT), 0, s, b->part.p, b->nblocks(), 2, b->dres.p,
+                         b->dpinned);
       double g2[2];
-      if (b->fetch(b->dres.p, 2, g2)) return -1;
+      if (b->fetch(2, g2)) return -1;
       gn = std::sqrt(g2[0] / (double)n);
       gnCv = std::sqrt(g2[1] / (double)n);
       if (!std::isfinite(gn)) { rc = 1; break; }

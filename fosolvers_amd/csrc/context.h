@@ -80,11 +80,13 @@ struct fos_euler {
   fos::DBuf<int> dStatus;
   fos::Learned *learned = nullptr;
 
-  // non-finite results: the kernels that write a callback's output set this device word; a
-  // callback reads it back (pinned word) and clears it before returning, unless
-  // FOS_ASYNC_CALLBACKS, where it accumulates until fos_euler_nonfinite
-  fos::DBuf<unsigned> dNonFinite;
-  unsigned *hNonFinite = nullptr;
+  // non-finite results: the kernels that write a callback's output set this word in pinned host memory
+  // (dNonFinite: its device address); a callback reads and clears it once the stream is done, unless
+  // FOS_ASYNC_CALLBACKS, where it accumulates until fos_euler_nonfinite.  While the integrator sets defer,
+  // the callbacks return without waiting and it takes the word at its next wait (take_nonfinite).
+  unsigned *hNonFinite = nullptr, *dNonFinite = nullptr;
+  bool defer = false;
+  const char *deferWho = "";
 
   // the host's N_Vector data accessor for the *_nv callbacks (N_VGetArrayPointer or its device form)
   fos_nvector_data_fn nvData = nullptr;
@@ -114,6 +116,8 @@ int ensure_pair_arrays(fos_euler *ctx);
 // SUNDIALS convention) when a kernel flagged a non-finite output since the last check, 0 otherwise
 // (the word is cleared); -1 on a HIP error.
 int finish_call(fos_euler *ctx, const char *who);
+// Whether a kernel flagged a non-finite output; clears the word.  The stream must be done.
+bool take_nonfinite(fos_euler *ctx);
 // Resolves, once per device, the address of the file-scope scratch array behind
 // fos_euler_jtimes_noalloc (with that device current).  Called by fos_euler_create.
 int resolve_noalloc_scratch(int device);

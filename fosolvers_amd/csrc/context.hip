@@ -291,12 +291,12 @@ int jtimes_noalloc_dev(fos_euler *ctx, const double *v, double *Jv, const double
   if (wrms_sigma_into(ctx, v, y, sig, base, reuse)) return -1;
   if (ctx->flags & FOS_PREC_FP32) {
     if (ctx->useTet)
-      return launch_tet_dq_jv_diff<double, float>(ctx->T32, y, v, 0.0, sig + 2, Jv, ctx->stream, ctx->dNonFinite.p);
-    return launch_dq_jv_diff<double, float>(ctx->L32, y, v, 0.0, sig + 2, Jv, ctx->stream, ctx->dNonFinite.p);
+      return launch_tet_dq_jv_diff<double, float>(ctx->T32, y, v, 0.0, sig + 2, Jv, ctx->stream, ctx->dNonFinite);
+    return launch_dq_jv_diff<double, float>(ctx->L32, y, v, 0.0, sig + 2, Jv, ctx->stream, ctx->dNonFinite);
   }
   if (ctx->useTet)
-    return launch_tet_dq_jv<double, double>(ctx->T64, y, v, fy, 0.0, sig, Jv, ctx->stream, ctx->dNonFinite.p);
-  return launch_dq_jv<double, double>(ctx->L64, y, v, fy, 0.0, sig, Jv, ctx->stream, ctx->dNonFinite.p);
+    return launch_tet_dq_jv<double, double>(ctx->T64, y, v, fy, 0.0, sig, Jv, ctx->stream, ctx->dNonFinite);
+  return launch_dq_jv<double, double>(ctx->L64, y, v, fy, 0.0, sig, Jv, ctx->stream, ctx->dNonFinite);
 }
 
 int wrms_sigma(fos_euler *ctx, const double *v, const double *y, double *sigmaDev) {
@@ -658,8 +658,8 @@ int residual_dev(fos_euler *ctx, const double *y, double *ydot) {
     set_error("rhs: a *_UDF boundary condition is used but fos_euler_set_udf_bc was not called");
     return -1;
   }
-  if (ctx->useTet) return launch_tet_residual<double, double>(ctx->T64, y, ydot, ctx->stream, ctx->dNonFinite.p);
-  return launch_residual<double, double>(ctx->L64, y, ydot, ctx->stream, ctx->dNonFinite.p);
+  if (ctx->useTet) return launch_tet_residual<double, double>(ctx->T64, y, ydot, ctx->stream, ctx->dNonFinite);
+  return launch_residual<double, double>(ctx->L64, y, ydot, ctx->stream, ctx->dNonFinite);
 }
 
 int jv_dev(fos_euler *ctx, const double *v, double *Jv, const double *y, const double *fy, int newton, double ngam) {
@@ -670,20 +670,20 @@ int jv_dev(fos_euler *ctx, const double *v, double *Jv, const double *y, const d
     // scaled to FP32 would push a localised v's components by O(1) relative (NaN on rho or p < 0)
     if (ctx->useTet)
       return launch_tet_dq_jv_diff<double, float>(ctx->T32, y, v, 0.0, ctx->dSigma.p + 2, Jv, ctx->stream,
-                                                  ctx->dNonFinite.p, newton, ngam);
+                                                  ctx->dNonFinite, newton, ngam);
     return launch_dq_jv_diff<double, float>(ctx->L32, y, v, 0.0, ctx->dSigma.p + 2, Jv, ctx->stream,
-                                            ctx->dNonFinite.p, newton, ngam);
+                                            ctx->dNonFinite, newton, ngam);
   }
   if (ctx->useTet)
     return launch_tet_dq_jv<double, double>(ctx->T64, y, v, fy, 0.0, ctx->dSigma.p, Jv, ctx->stream,
-                                            ctx->dNonFinite.p, newton, ngam);
-  return launch_dq_jv<double, double>(ctx->L64, y, v, fy, 0.0, ctx->dSigma.p, Jv, ctx->stream, ctx->dNonFinite.p,
+                                            ctx->dNonFinite, newton, ngam);
+  return launch_dq_jv<double, double>(ctx->L64, y, v, fy, 0.0, ctx->dSigma.p, Jv, ctx->stream, ctx->dNonFinite,
                                       newton, ngam);
 }
 
 // the analytic product J v (or v - ngam J v with newton set) on device vectors
 static int jvp_dev(fos_euler *ctx, const double *v, double *out, const double *y, int newton, double ngam) {
-  unsigned *nf = ctx->dNonFinite.p;
+  unsigned *nf = ctx->dNonFinite;
   if (ctx->flags & FOS_PREC_FP32)
     return ctx->useTet ? launch_tet_jvp<double, float>(ctx->T32, y, v, out, ctx->stream, nf, newton, ngam)
                        : launch_jvp<double, float>(ctx->L32, y, v, out, ctx->stream, nf, newton, ngam);
@@ -691,16 +691,16 @@ static int jvp_dev(fos_euler *ctx, const double *v, double *out, const double *y
                      : launch_jvp<double, double>(ctx->L64, y, v, out, ctx->stream, nf, newton, ngam);
 }
 
+bool take_nonfinite(fos_euler *ctx) { return __atomic_exchange_n(ctx->hNonFinite, 0u, __ATOMIC_RELAXED) != 0; }
+
 int finish_call(fos_euler *ctx, const char *who) {
   if (ctx->flags & FOS_ASYNC_CALLBACKS) return 0;
-  FOS_HIP_TRY(hipMemcpyAsync(ctx->hNonFinite, ctx->dNonFinite.p, sizeof(unsigned), hipMemcpyDeviceToHost,
-                             ctx->stream));
+  if (ctx->defer) {
+    ctx->deferWho = who;
+    return 0;
+  }
   FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  if (*ctx->hNonFinite == 0) return 0;
-  *ctx->hNonFinite = 0;
-  FOS_HIP_TRY(hipMemcpyAsync(ctx->dNonFinite.p, ctx->hNonFinite, sizeof(unsigned), hipMemcpyHostToDevice,
-                             ctx->stream));
-  FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
+  if (!take_nonfinite(ctx)) return 0;
   set_error("%s: non-finite value in the result", who);
   return 1;
 }
@@ -758,14 +758,13 @@ fos_euler *fos_euler_create(const fos_fv_grid *grid, const fos_cond_tab *bc, dou
   ctx->nP = grid->nP;
   ctx->nPi = grid->nPi;
   ctx->maxNF = grid->maxNF;
-  const unsigned zero = 0;
   if (build_layout(ctx, grid, bc) || ctx->redPart.alloc(2 * RED_BLOCKS) || ctx->dSigma.alloc(4) ||
-      ctx->dNonFinite.upload(&zero, 1, ctx->stream) || save_grid_host(ctx, grid)) {
+      save_grid_host(ctx, grid)) {
     delete ctx;
     return nullptr;
   }
-  if (hipHostMalloc((void **)&ctx->hNonFinite, sizeof(unsigned)) != hipSuccess) {
-    ctx->hNonFinite = nullptr;
+  if (hipHostMalloc((void **)&ctx->hNonFinite, sizeof(unsigned)) != hipSuccess ||
+      hipHostGetDevicePointer((void **)&ctx->dNonFinite, ctx->hNonFinite, 0) != hipSuccess) {
     set_error("fos_euler_create: pinned host allocation failed");
     delete ctx;
     return nullptr;
@@ -925,8 +924,8 @@ int fos_euler_newton_matvec_analytic(double gamma, const double *v, double *out,
 int fos_euler_rhs_f32(fos_euler *ctx, const float *y, float *ydot) {
   if (!ctx) return -1;
   ctx->counters[0]++;
-  const int rc = ctx->useTet ? launch_tet_residual<float, float>(ctx->T32, y, ydot, ctx->stream, ctx->dNonFinite.p)
-                             : launch_residual<float, float>(ctx->L32, y, ydot, ctx->stream, ctx->dNonFinite.p);
+  const int rc = ctx->useTet ? launch_tet_residual<float, float>(ctx->T32, y, ydot, ctx->stream, ctx->dNonFinite)
+                             : launch_residual<float, float>(ctx->L32, y, ydot, ctx->stream, ctx->dNonFinite);
   return rc ? -1 : finish_call(ctx, "rhs_f32");
 }
 
@@ -934,24 +933,16 @@ int fos_euler_jtimes_f32(fos_euler *ctx, const float *v, float *Jv, const float 
   if (!ctx) return -1;
   ctx->counters[1]++;
   const int rc =
-      ctx->useTet ? launch_tet_dq_jv<float, float>(ctx->T32, y, v, fy, sigma, nullptr, Jv, ctx->stream, ctx->dNonFinite.p)
-                  : launch_dq_jv<float, float>(ctx->L32, y, v, fy, sigma, nullptr, Jv, ctx->stream, ctx->dNonFinite.p);
+      ctx->useTet ? launch_tet_dq_jv<float, float>(ctx->T32, y, v, fy, sigma, nullptr, Jv, ctx->stream, ctx->dNonFinite)
+                  : launch_dq_jv<float, float>(ctx->L32, y, v, fy, sigma, nullptr, Jv, ctx->stream, ctx->dNonFinite);
   return rc ? -1 : finish_call(ctx, "jtimes_f32");
 }
 
 int fos_euler_nonfinite(fos_euler *ctx, int clear) {
   if (!ctx) return -1;
-  FOS_HIP_TRY(hipMemcpyAsync(ctx->hNonFinite, ctx->dNonFinite.p, sizeof(unsigned), hipMemcpyDeviceToHost,
-                             ctx->stream));
   FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  const int bad = *ctx->hNonFinite != 0;
-  if (clear && bad) {
-    *ctx->hNonFinite = 0;
-    FOS_HIP_TRY(hipMemcpyAsync(ctx->dNonFinite.p, ctx->hNonFinite, sizeof(unsigned), hipMemcpyHostToDevice,
-                               ctx->stream));
-    FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
-  }
-  return bad;
+  if (clear) return take_nonfinite(ctx) ? 1 : 0;
+  return __atomic_load_n(ctx->hNonFinite, __ATOMIC_RELAXED) != 0 ? 1 : 0;
 }
 
 // ---- the callbacks with SUNDIALS' N_Vector signatures: resolve the data pointers, forward

@@ -195,7 +195,7 @@ __device__ inline void write_cell(const TC acc[5], TC iv, TS sigma, const TS *__
     else out[i] = o;
     bad |= !isfinite(o);
   }
-  if (bad && nf) atomicOr(nf, 1u);
+  if (bad && nf) flag_nonfinite(nf);
 }
 
 template <class TS, class TC, int MODE, int NS>

@@ -70,6 +70,12 @@ struct DBuf {
   }
 };
 
+// Sets a context's non-finite word, which lies in pinned host memory: the host reads it once the stream is
+// done, without a copy.  Any number of lanes may store the same 1.
+__device__ inline void flag_nonfinite(unsigned *nf) {
+  __hip_atomic_store(nf, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // blockIdx -> work item mapping that gives each of the 8 XCDs a contiguous range of work items
 // (workgroups are dealt round-robin to XCDs, and each XCD has its own L2).
 __device__ inline int xcd_remap(int bid, int nblocks) {

@@ -633,7 +633,7 @@ __global__ void apply_z_kernel(int R, int nC, const int *__restrict__ nbr, const
     z[(size_t)a * nC + c] = o;
     bad |= !isfinite(o);
   }
-  if (bad && nf) atomicOr(nf, 1u);
+  if (bad && nf) flag_nonfinite(nf);
 }
 
 // loss pieces: e = 2 (zhat - dhat) / R; ds[c][j] = e_c . t_nb(j) (j < 4), ds[c][4] = e_c . t_c (the
@@ -1035,7 +1035,7 @@ int learned_psolve(fos_euler *ctx, const double *r, double *z) {
   hipLaunchKernelGGL(apply_t_kernel, dim3(gb), dim3(256), 0, ctx->stream, nC, 0, nC, L->O.p, L->scale.p, r, L->t.p,
                      nullptr);
   hipLaunchKernelGGL(apply_z_kernel, dim3(gb), dim3(256), 0, ctx->stream, nC, nC, L->nbr.p, L->scale.p, L->t.p,
-                     z, ctx->dNonFinite.p);
+                     z, ctx->dNonFinite);
   FOS_HIP_TRY(hipGetLastError());
   return 0;
 }

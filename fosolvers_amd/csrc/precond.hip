@@ -965,7 +965,7 @@ __global__ __launch_bounds__(64) void bwd_colour_kernel(int nC, const int4 *__re
       for (int c = 0; c < 5; c++) Dc[c] = Dn[c];
     }
     chunk_store(z, S.val, nC, c0);
-    if (bad) atomicOr(nf, 1u);
+    if (bad) flag_nonfinite(nf);
     return;
   }
   // the loads of step st: row q of each U block and of inv(U_pp) (y_p comes from LDS)
@@ -1011,7 +1011,7 @@ __global__ __launch_bounds__(64) void bwd_colour_kernel(int nC, const int4 *__re
       for (int c = 0; c < 5; c++) Uc[j][c] = Un[j][c];
   }
   chunk_store(z, S.val, nC, c0);
-  if (bad) atomicOr(nf, 1u);
+  if (bad) flag_nonfinite(nf);
 }
 
 // ---------------------------------------------------------------- the solve in one launch
@@ -1147,7 +1147,7 @@ __global__ __launch_bounds__(FLOW_THREADS) void ilu_flow_kernel(
     item = sItem[0];
     __syncthreads();
   }
-  if (bad) atomicOr(nf, 1u);
+  if (bad) flag_nonfinite(nf);
   if (threadIdx.x == 0 && atomicAdd(ctl + FLOW_CTL, 1u) == gridDim.x - 1) {
     // the last workgroup: every other one has read the parity and taken its last item
     __hip_atomic_store(ctl, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1206,7 +1206,7 @@ __global__ __launch_bounds__(256) void bjac_apply_kernel(int nC, const TF *__res
     z[(size_t)a * nC + i] = s;
     bad |= !isfinite(s);
   }
-  if (bad) atomicOr(nf, 1u);
+  if (bad) flag_nonfinite(nf);
 }
 
 // to[src[m]] = m: the packed block of every slot that has one
@@ -1772,11 +1772,11 @@ static int ilu_sweeps(fos_euler *ctx, const TF *Lf, const TF *Uf, const TF *Db, 
     const int nCh = (b->nC + ICH - 1) / ICH;
     hipLaunchKernelGGL(ilu_flow_kernel<TF>, dim3(std::min(2 * nCh, b->flowGrid)), dim3(FLOW_THREADS), 0, ctx->stream,
                        b->nC, nCh, b->dFMeta.p, b->dBMeta.p, b->dFRow.p, b->dBRow.p, b->dFOutCell.p, b->dBOutCell.p,
-                       Lf, Uf, Db, r, z, b->dX.p, b->dCtl.p, ctx->dNonFinite.p);
+                       Lf, Uf, Db, r, z, b->dX.p, b->dCtl.p, ctx->dNonFinite);
     return 0;
   }
   if (!b->eager && !b->solveChain.ready()) {
-    if (ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite.p,
+    if (ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite,
                    [&](auto k, dim3 g, dim3 bl, size_t lds, auto... a) {
                      return b->solveChain.add(k, g, bl, lds, a...);
                    }) ||
@@ -1787,7 +1787,7 @@ static int ilu_sweeps(fos_euler *ctx, const TF *Lf, const TF *Uf, const TF *Db, 
   }
   hipLaunchKernelGGL(ilu_io_kernel, dim3(1), dim3(64), 0, ctx->stream, b->dIo.p, r, z);
   if (b->eager) {
-    ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite.p, [&](auto k, dim3 g, dim3 bl, size_t lds, auto... a) {
+    ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite, [&](auto k, dim3 g, dim3 bl, size_t lds, auto... a) {
       hipLaunchKernelGGL(k, g, bl, lds, ctx->stream, a...);
       return 0;
     });
@@ -1832,10 +1832,10 @@ int bjac_solve(fos_euler *ctx, const double *r, double *z) {
   const int nC = ctx->nC;
   if (ctx->flags & FOS_PREC_FP32)
     hipLaunchKernelGGL(bjac_apply_kernel<float>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dBj32.p, r, z,
-                       ctx->dNonFinite.p);
+                       ctx->dNonFinite);
   else
     hipLaunchKernelGGL(bjac_apply_kernel<double>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dBj.p, r, z,
-                       ctx->dNonFinite.p);
+                       ctx->dNonFinite);
   FOS_HIP_TRY(hipGetLastError());
   return 0;
 }

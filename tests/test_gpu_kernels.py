@@ -191,3 +191,41 @@ def test_learned_apply_matches_oracle_at_tile_edges(cuda, dims):
         print(f"  relative error {err:.2e}")
         assert err <= 3e-2
         eu.learned_loss_grad(y, _dev(r), _dev(r), gamma, 0, min(nC, 100))  # training overwrites the rows
+
+
+@pytest.mark.parametrize("precond", ["ilu", None])
+def test_integrator_reports_a_nonfinite_product_like_the_callback(cuda, precond):
+    """A state whose squares overflow FP32 but not FP64: the Newton residual is finite, the mixed-precision
+    product inside GMRES is not.  With the fused product (checked at GMRES's next wait) and without (checked
+    by the callback itself) the step fails as recoverable, with the state and the counters of iterations
+    unchanged and nothing left behind: the next good step is the one a fresh context takes."""
+    import torch
+    from fosolvers_amd import _capi
+    print(f"[case] non-finite product in GMRES precond={precond}", flush=True)
+    pg = M.box(8, 4, 4, jitter=0.2, seed=3, renumber=fa.RENUMBER_CHUNKS)
+    fv = pg.up()
+    ctab = fa.CondTab(*M.conds("wall"))
+    good = _dev(M.perturbed_state(fv.p[:fv.nC], mach=0.3, seed=5))
+    scale = torch.ones(5, fv.nC, dtype=torch.float64, device="cuda")
+    scale[0], scale[1:4], scale[4] = 1e-30, 1e-5, 1e20  # u ~ 1e25: finite in FP32 until it is squared
+    huge = (good.view(5, -1) * scale).reshape(-1).contiguous()
+    outs, fails = [], []
+    for fused in (True, False, None):
+        eu = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA, flags=fa.PREC_FP32)
+        b = fa.BDFNewtonKrylov.for_euler(eu, maxl=20, precond=precond, jtimes="analytic", fused=bool(fused))
+        b.set_newton(tol=1e-8, max_iter=20, lin_tol=1e-3, max_restarts=10)
+        y = torch.zeros_like(good)
+        if fused is not None:
+            b.set_dt(1e-28)
+            b.set_iv(0.0, huge)
+            rc, _t = b.step(0.0, y)
+            assert rc == 1 and "non-finite" in _capi.last_error(), (rc, _capi.last_error())
+            fails.append(b.stats()["nli"])
+            assert not eu.nonfinite()
+        b.set_dt(1e-3)
+        b.set_iv(0.0, good)
+        assert b.step(0.0, y)[0] == 0
+        outs.append(y.clone())
+    assert fails[0] == fails[1]
+    assert M.rel(outs[0].cpu().numpy(), outs[2].cpu().numpy()) <= 1e-13
+    assert M.rel(outs[1].cpu().numpy(), outs[2].cpu().numpy()) <= 1e-13
