@@ -339,6 +339,16 @@ int launch(const FluxLayout<TC> &L, const TS *y, const TS *v, TS sigma, const do
 
 // ---------------------------------------------------------------- tetrahedral layout
 //
+// the ghost primitives of boundary slot g from its cell's primitives A (setBC with the pair's normal)
+template <class TC>
+__device__ inline void boundary_prim(const TetLayout<TC> &L, int g, const Prim<TC> &A, Prim<TC> &B) {
+  const int b = L.bndPair[g], P = L.nPb;
+  TC gr, gx, gy, gz, gE;
+  ghost_state<TC>(L.bndType[b], L.bndPar + 5 * (size_t)b, L.bndNorm[g], L.bndNorm[P + g], L.bndNorm[2 * (size_t)P + g],
+                  A, L.gamma, L.r, gr, gx, gy, gz, gE);
+  make_prim(gr, gx, gy, gz, gE, L.gamma - TC(1), B);
+}
+
 // The generic kernel's three phases with 8 bytes per face instead of 32: the face record names the
 // cells (chunk-local, or global for a halo cell, or the boundary pair) and the face's three nodes;
 // phase A stages the chunk's node coordinates next to its cells and zeroes the cells' flux sums, and
@@ -359,13 +369,16 @@ int launch(const FluxLayout<TC> &L, const TS *y, const TS *v, TS sigma, const do
 template <class TC>
 constexpr bool tet_gathers(int mode) { return sizeof(TC) == 4 && mode != JVP; }
 
-template <class TS, class TC, int MODE, int NS, bool NT>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
-    MODE == 3 ? FOS_JVP_MIN_WAVES : FOS_TET_MIN_WAVES))) void tet_kernel(
+//
+// TB > THREADS (small meshes, SMALL_CHUNKS): more threads per chunk, and the ghost states formed here.
+template <class TS, class TC, int MODE, int NS, bool NT, int TB = THREADS>
+__global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(
+    TB > THREADS ? TB / 256 : MODE == 3 ? FOS_JVP_MIN_WAVES : FOS_TET_MIN_WAVES))) void tet_kernel(
     TetLayout<TC> L, const TS *__restrict__ y, const TS *__restrict__ v, TS sigmaVal,
     const double *__restrict__ sigmaPtr, const TS *__restrict__ fy, TS *__restrict__ out, unsigned *__restrict__ nf,
     int newton, TS ngam) {
-  constexpr bool JV = MODE != RES, GATHER = tet_gathers<TC>(MODE);
+  constexpr bool JV = MODE != RES, GATHER = tet_gathers<TC>(MODE), GHOST = TB > THREADS;
+  static_assert(!GHOST || MODE == RES || MODE == DQ_FY, "the small-mesh form has one state per cell");
   constexpr int NQ = nq_of(MODE);
   const TS sigma = JV && sigmaPtr ? (TS)*sigmaPtr : sigmaVal;
   extern __shared__ unsigned char smem_raw[];
@@ -382,8 +395,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
   const int t = threadIdx.x;
   // A: the first face record and the nodes are loaded before the cells are staged
   if constexpr (!GATHER)
-#pragma unroll
-    for (int k = 0; k < 5; k++) sA[k * CHUNK + t] = 0.0;
+    for (int k = t; k < 5 * CHUNK; k += TB) sA[k] = 0.0;
   const int fb = L.chunkBeg[chunk], fe = L.chunkBeg[chunk + 1];
   uint2 recN = make_uint2(0u, 0u);
   // NT (working sets beyond the 256 MB last-level cache): the face records, node coordinates and
@@ -398,11 +410,12 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
   };
   if (fb + t < fe) recN = ldrec(fb + t);
   const int nb = L.nodeBeg[chunk], nn = L.nodeBeg[chunk + 1] - nb;
-  if (t < nn) {  // nn <= TET_MAX_NODES = THREADS
-    const TC *p = L.node + 3 * (size_t)(nb + t);
-    sN[t] = ld(p);
-    sN[mn + t] = ld(p + 1);
-    sN[2 * mn + t] = ld(p + 2);
+  const int tn = TB >= 2 * THREADS ? t - THREADS : t;  // other threads than the cells', if there are
+  if (tn >= 0 && tn < nn) {                            // nn <= TET_MAX_NODES = THREADS
+    const TC *p = L.node + 3 * (size_t)(nb + tn);
+    sN[tn] = ld(p);
+    sN[mn + tn] = ld(p + 1);
+    sN[2 * mn + tn] = ld(p + 2);
   }
   unsigned long long slots = 0;  // the cell's face slots, for C
   if (t < ncell) {
@@ -412,9 +425,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
   __syncthreads();
   // B: one Roe flux (or flux difference) per chunk face
   const TC *sy = sN + mn, *sz = sN + 2 * mn;
-  for (int f = fb + t; f < fe; f += THREADS) {
+  for (int f = fb + t; f < fe; f += TB) {
     const uint2 rec = recN;
-    if (f + THREADS < fe) recN = ldrec(f + THREADS);
+    if (f + TB < fe) recN = ldrec(f + TB);
     const int payload = (int)(rec.x & (TET_MAX_PAYLOAD - 1)), kind = (rec.x >> 29) & 3u;
     const bool flip = rec.x >> 31;
     const int lc = rec.y & 255u, q0 = (rec.y >> 8) & 255u, q1 = (rec.y >> 16) & 255u, q2 = rec.y >> 24;
@@ -458,6 +471,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(
         read_prim(sq, CHUNK, lc, B);
       } else if (kind == 2) {
         halo(payload, B);
+      } else if constexpr (GHOST) {
+        boundary_prim(L, payload, A, B);
       } else {
         read_prim(L.ghost + (MODE == DQ_DIFF && pass == 1 ? 8 * (size_t)L.nPb : 0), L.nPb, payload, B);
       }
@@ -517,10 +532,11 @@ __global__ __launch_bounds__(256) void ghost_kernel(TetLayout<TC> L, const TS *_
   const int g = blockIdx.x * blockDim.x + threadIdx.x;  // ghost slot
   if (g >= L.nPb) return;
   const TS sigma = MODE != RES && sigmaPtr ? (TS)*sigmaPtr : sigmaVal;
-  const int c = L.bndCell[g], b = L.bndPair[g], nC = L.nC, P = L.nPb;
+  const int c = L.bndCell[g], nC = L.nC, P = L.nPb;
   const TC g1 = L.gamma - TC(1);
-  const TC nx = L.bndNorm[g], ny = L.bndNorm[P + g], nz = L.bndNorm[2 * P + g];
   if constexpr (MODE == JVP) {
+    const int b = L.bndPair[g];
+    const TC nx = L.bndNorm[g], ny = L.bndNorm[P + g], nz = L.bndNorm[2 * P + g];
     using DT = Dual<TC>;
     Prim<DT> A, B;
     load_cell_dual<TS, TC>(y, v, nC, c, g1, A);
@@ -536,13 +552,20 @@ __global__ __launch_bounds__(256) void ghost_kernel(TetLayout<TC> L, const TS *_
       Prim<TC> A, B;
       if (pert) load_cell<TS, TC, true>(y, v, sigma, nC, c, g1, A);
       else load_cell<TS, TC, false>(y, v, sigma, nC, c, g1, A);
-      TC gr, gx, gy, gz, gE;
-      ghost_state<TC>(L.bndType[b], L.bndPar + 5 * (size_t)b, nx, ny, nz, A, L.gamma, L.r, gr, gx, gy, gz, gE);
-      make_prim(gr, gx, gy, gz, gE, g1, B);
+      boundary_prim(L, g, A, B);
       store_prim(L.ghost + (size_t)pass * 8 * P, P, g, B);
     }
   }
 }
+
+// On a mesh of few chunks the chip is not full and a chunk's time counts: twice the threads per chunk halve
+// its face sweeps (a chunk has ~620 faces), and the ghost states are formed in the face pass, whose
+// register count (158 against 96) does not matter then, instead of by a launch of their own.  FP64 residual
+// and difference quotient; the FP32 forms keep one arithmetic on every mesh size.  Measured per
+// residual, without the callback's wait: 6,000 tets 15.0 -> 7.6 us, 24,000 14.7 -> 7.8, 104,000 (405
+// chunks) 15.0 -> 11.6, 270,000 (1,055 chunks) 20.8 -> 24.0.  768 and 1024 threads were slower (24,000
+// tets: 8.1, 9.5 us).  The generic kernel gains nothing from more threads (95,000 hexes, 370 chunks: the same).
+constexpr int SMALL_CHUNKS = 512, SMALL_THREADS = 512;
 
 constexpr size_t TET_LDS_LIMIT = 65536;
 
@@ -562,6 +585,14 @@ int launch_tet(const TetLayout<TC> &L, const TS *y, const TS *v, TS sigma, const
   if (!smem) {
     set_error("residual: tetrahedral chunk data exceeds LDS");
     return -1;
+  }
+  if constexpr (sizeof(TC) == 8 && (MODE == RES || MODE == DQ_FY)) {
+    if (L.nSlots <= 4 && L.nChunks <= SMALL_CHUNKS) {
+      hipLaunchKernelGGL((tet_kernel<TS, TC, MODE, 4, false, SMALL_THREADS>), dim3(L.nChunks),
+                         dim3(SMALL_THREADS), smem, s, L, y, v, sigma, sigmaPtr, fy, out, nf, newton, ngam);
+      FOS_HIP_TRY(hipGetLastError());
+      return 0;
+    }
   }
   if (L.nPb > 0)
     hipLaunchKernelGGL((ghost_kernel<TS, TC, MODE>), dim3((L.nPb + 255) / 256), dim3(256), 0, s, L, y, v, sigma,

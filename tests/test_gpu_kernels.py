@@ -229,3 +229,31 @@ def test_integrator_reports_a_nonfinite_product_like_the_callback(cuda, precond)
     assert fails[0] == fails[1]
     assert M.rel(outs[0].cpu().numpy(), outs[2].cpu().numpy()) <= 1e-13
     assert M.rel(outs[1].cpu().numpy(), outs[2].cpu().numpy()) <= 1e-13
+
+
+@pytest.mark.parametrize("kind", ["mixed", "wall"])
+@pytest.mark.parametrize("dims", [(1, 1, 1), (43, 2, 3), (31, 27, 26), (33, 27, 26)],
+                         ids=["6", "1548", "130572", "138996"])
+def test_residual_on_either_side_of_the_small_mesh_rule(cuda, dims, kind):
+    """The tetrahedral FP64 residual and difference quotient with the ghost states formed in the face pass
+    (up to 512 chunks) and by their own launch (beyond), against the generic layout, which forms both
+    from other geometry data: 1e-12 relative, the bound of the residual tests; the quotient amplifies the
+    residual's rounding (1e-16) by 1 / sigma (~1e6 with these vectors), so 1e-9."""
+    import torch
+    print(f"[case] small-mesh rule dims={dims} kind={kind}", flush=True)
+    pg = M.box(*dims, 1.0, 0.5, 0.5, jitter=0.2, seed=3, renumber=fa.RENUMBER_CHUNKS)
+    fv = pg.up()
+    ctab = fa.CondTab(*M.conds(kind))
+    y = _dev(M.perturbed_state(fv.p[:fv.nC], mach=0.6, amp=0.3, seed=5))
+    v = _dev(np.random.default_rng(2).standard_normal(5 * fv.nC)) * (y.abs() + 0.1) * 1e-3
+    out = []
+    for flags in (0, fa.LAYOUT_GENERIC):
+        eu = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA, flags=flags)
+        assert eu.layout == (0 if flags else 1)
+        f, jv = torch.zeros_like(y), torch.zeros_like(y)
+        eu.rhs(y, f)
+        eu.jtimes(v, jv, y, f)
+        out.append((f.cpu().numpy(), jv.cpu().numpy()))
+    ef, ej = M.rel(out[0][0], out[1][0]), M.rel(out[0][1], out[1][1])
+    print(f"  residual {ef:.1e}, quotient {ej:.1e}")
+    assert ef <= 1e-12 and ej <= 1e-9
