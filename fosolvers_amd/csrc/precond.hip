@@ -628,8 +628,9 @@ __host__ __device__ inline unsigned rec_nb(uint2 rc, int j) {
   return ((rc.x >> (8 * j)) & 255u) | ((rc.y >> (16 + j)) & 1u) << 8;
 }
 
-// Row records (solve in one launch): per cell the same uint2 with the row's in-chunk level in y bits 0-7
-// (0 .. ICH - 1; a level reads rows of lower ones) instead of its local index.
+// Row records (solve in one launch): per cell the same uint2, a chunk's rows in the order of their
+// in-chunk levels (0 .. ICH - 1; a level reads rows of lower ones), with the level in y bits 0-7 and the
+// row's local index in bits REC_BLK_SHIFT up.
 //
 // Per launch slot of a colour launch (chunks in launch order), two int4: {first cell c0, first step
 // record s0, steps ns, first outside entry o0}, {outside entries nOut, first packed block, first
@@ -1023,7 +1024,13 @@ __global__ __launch_bounds__(64) void bwd_colour_kernel(int nC, const int4 *__re
 // for items taken earlier by workgroups that are already running: whatever the dispatch order or the
 // number of resident workgroups, the first unfinished item can always proceed.  A lane owns one
 // component of one row (12 rows to a wave, 6 waves to a chunk), loads its blocks into registers while
-// the item waits, and the chunk's in-chunk levels then run out of LDS, a barrier each.
+// the item waits, and the chunk's in-chunk levels then run out of LDS, a barrier each.  The levels are
+// two thirds of the chain (6 on average, up to 11), so a level is kept short: rows are dealt to the
+// lanes in level order (a level then runs in one or two waves, and the others do not load the LDS),
+// chunk, outside and absent values lie in one array, so a row reads its 20 values at once, and its four
+// products of five terms run side by side.  With rows in cell order and one neighbour after the other
+// a level took 0.39 us; now 0.30.  The registers stay within 128: above, the second workgroup no
+// longer fits a CU, and 270,000 tets take 178 us.
 // A value is published with one 8-byte store at agent scope and is its own flag: the exchange array
 // holds FLOW_EMPTY (a NaN no result is stored as) until then, and readers load it at agent scope until
 // it differs.  Nothing else passes between workgroups, so no fence is needed.  Two copies of the array
@@ -1031,9 +1038,9 @@ __global__ __launch_bounds__(64) void bwd_colour_kernel(int nC, const int4 *__re
 // swaps the copies, so the state lives on the device (replays of a captured apply included).  A wait is
 // bounded (FLOW_MAX_POLLS, seconds): past it the value is a NaN, which the callback reports.
 // The arithmetic per row is the colour kernels', in the same order: the results are bitwise the same.
-// Per apply, colour launches -> one launch (FP64): 6,000 tets 136 -> 52 us, 24,000 174 -> 67, 270,000
-// 233 -> 142, 540,000 267 -> 244; FP32 factors alike.  What is left is the chain: about 3.3 us for each
-// of the 17 colours of both sweeps (publish, see, gather, the levels).
+// Per apply, colour launches -> one launch (FP64): 6,000 tets 136 -> 42 us, 24,000 174 -> 53, 270,000
+// 233 -> 128, 540,000 267 -> 232; FP32 factors alike.  What is left is the chain: about 2.8 us for each
+// of the 17 colours of both sweeps (publish, see, gather: 1.0; the levels: 1.8).
 constexpr int FLOW_THREADS = 384, FLOW_CTL = 32;
 constexpr unsigned long long FLOW_EMPTY = ~0ull;
 constexpr int FLOW_MAX_POLLS = 1 << 22;  // of a memory round trip (~1 us) each
@@ -1049,16 +1056,12 @@ __device__ inline void flow_put(unsigned long long *X, size_t at, double v) {
 template <int N>
 __device__ inline void flow_get(unsigned long long *X, size_t at, double (&v)[N]) {
   unsigned long long u[N];
-#pragma unroll
-  for (int c = 0; c < N; c++) u[c] = __hip_atomic_load(X + at + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   for (int polls = 0; polls < FLOW_MAX_POLLS; polls++) {
     bool there = true;
 #pragma unroll
-    for (int c = 0; c < N; c++)
-      if (u[c] == FLOW_EMPTY) {
-        there = false;
-        u[c] = __hip_atomic_load(X + at + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
+    for (int c = 0; c < N; c++) u[c] = __hip_atomic_load(X + at + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int c = 0; c < N; c++) there &= u[c] != FLOW_EMPTY;
     if (there) break;
     __builtin_amdgcn_s_sleep(1);
   }
@@ -1072,10 +1075,12 @@ __global__ __launch_bounds__(FLOW_THREADS) void ilu_flow_kernel(
     const uint2 *__restrict__ bRow, const int *__restrict__ fOut, const int *__restrict__ bOut,
     const TF *__restrict__ Lf, const TF *__restrict__ Uf, const TF *__restrict__ Db, const double *r, double *z,
     unsigned long long *X, unsigned *ctl, unsigned *__restrict__ nf) {
-  __shared__ double sv[5 * ICH], so[5 * MAX_OUT], sT[FLOW_THREADS / 64 * 64];
+  // the chunk's values, the outside ones (at the records' codes) and zeros for an absent neighbour
+  __shared__ double sv[5 * (REC_OUT0 + MAX_OUT + 1)], sT[FLOW_THREADS];
   __shared__ unsigned sItem[2];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, slot = lane / 5, q = lane - 5 * slot;
-  const int row = wave * SWEEP_ROWS + slot;
+  const int pos = wave * SWEEP_ROWS + slot;
+  if (threadIdx.x < 5) sv[5 * (REC_OUT0 + MAX_OUT) + threadIdx.x] = 0.0;
   if (threadIdx.x == 0) {
     sItem[0] = atomicAdd(ctl, 1u);
     sItem[1] = __hip_atomic_load(ctl + 2 * FLOW_CTL, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -1087,45 +1092,56 @@ __global__ __launch_bounds__(FLOW_THREADS) void ilu_flow_kernel(
   unsigned long long *Xf = X + 2 * nv * par, *Xb = Xf + nv, *clr = X + 2 * nv * (par ^ 1u);
   bool bad = false;
   while (item < 2u * (unsigned)nCh) {
-    unsigned next = 0;
-    if (threadIdx.x == 0) next = atomicAdd(ctl, 1u);
     const bool fwd = item < (unsigned)nCh;
     const int4 *meta = fwd ? fMeta + 2 * item : bMeta + 2 * (2u * nCh - 1u - item);
     const int4 m0 = meta[0], m1 = meta[1];
     const int c0 = m0.x, o0 = m0.w, nOut = m1.x, blk0 = m1.y, pb = m1.z, nLev = m1.w;
-    const bool act = slot < SWEEP_ROWS && row < min(ICH, nC - c0);
-    const size_t mine = 5 * (size_t)(c0 + row) + q;
+    const bool act = slot < SWEEP_ROWS && pos < min(ICH, nC - c0);
     uint2 rc = make_uint2(~0u, 0xF00FFu);  // no neighbours, a level that does not come
-    double own = 0.0;
     int oc = 0;
-    if (act) {
-      rc = (fwd ? fRow : bRow)[c0 + row];
-      if (fwd) own = r[(size_t)q * nC + c0 + row];
-      __hip_atomic_store(clr + (fwd ? 0 : nv) + mine, FLOW_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
+    if (act) rc = (fwd ? fRow : bRow)[c0 + pos];
     if ((int)threadIdx.x < nOut) oc = (fwd ? fOut : bOut)[o0 + threadIdx.x];
-    TF B[4][5], Dq[5];
+    const int row = (int)(rc.y >> REC_BLK_SHIFT);
+    const size_t mine = 5 * (size_t)(c0 + row) + q;
+    double own = 0.0;
+    TF B[4][5] = {}, Dq[5];
     if (act) {
+      if (fwd) own = r[(size_t)q * nC + c0 + row];
       load_blocks(rc, fwd ? Lf : Uf, blk0, q, B);
       if (!fwd)
 #pragma unroll
         for (int c = 0; c < 5; c++) Dq[c] = Db[(size_t)25 * (pb + row) + 5 * q + c];
+      __hip_atomic_store(clr + (fwd ? 0 : nv) + mine, FLOW_EMPTY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    unsigned next = 0;
+    if (threadIdx.x == FLOW_THREADS - 1) next = atomicAdd(ctl, 1u);  // in the wave with the fewest rows
     if ((int)threadIdx.x < nOut) {
       double v[5];
       flow_get<5>(fwd ? Xf : Xb, 5 * (size_t)oc, v);
 #pragma unroll
-      for (int c = 0; c < 5; c++) so[5 * threadIdx.x + c] = v[c];
+      for (int c = 0; c < 5; c++) sv[5 * (REC_OUT0 + threadIdx.x) + c] = v[c];
     }
     if (act && !fwd) {
       double v[1];
       flow_get<1>(Xf, mine, v);
       own = v[0];
     }
+    const double *xp[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const unsigned k = rec_nb(rc, j);
+      xp[j] = sv + 5 * (k == REC_NB_NONE ? REC_OUT0 + MAX_OUT : (int)k);
+    }
     __syncthreads();
     for (int l = 0; l < nLev; l++) {
-      if (act && (int)(rc.y & 255u) == l) {
-        double v = own - nb_dot(rc, B, sv, so);
+      if ((int)(rc.y & 255u) == l) {
+        // nb_dot's sums with its four chains side by side
+        double t[4] = {};
+#pragma unroll
+        for (int c = 0; c < 5; c++)
+#pragma unroll
+          for (int j = 0; j < 4; j++) t[j] += (double)B[j][c] * xp[j][c];
+        double v = own - (t[0] + t[1] + t[2] + t[3]);
         if (!fwd) {
           sT[64 * wave + lane] = v;
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -1142,7 +1158,7 @@ __global__ __launch_bounds__(FLOW_THREADS) void ilu_flow_kernel(
     if (!fwd && threadIdx.x < ICH && (int)threadIdx.x < nC - c0)
 #pragma unroll
       for (int c = 0; c < 5; c++) z[(size_t)c * nC + c0 + threadIdx.x] = sv[5 * threadIdx.x + c];
-    if (threadIdx.x == 0) sItem[0] = next;
+    if (threadIdx.x == FLOW_THREADS - 1) sItem[0] = next;
     __syncthreads();
     item = sItem[0];
     __syncthreads();
@@ -1278,9 +1294,9 @@ int build_factor_records(BlockIlu *b, const std::vector<int> &rows, const std::v
 
 // Chunks up to which a solve is one launch: beyond, the exchange's extra traffic (200 bytes a cell, and a
 // ticket per item) costs more than the launches.  Measured per apply, colour launches against one: 8,440
-// chunks FP64 267 / 244 us, FP32 239 / 233; 16,800 chunks 397 / 459 and 322 / 444; 93,750 chunks
-// 1,770 / 2,470 and 1,210 / 2,370.
-constexpr int FLOW_MAX_CHUNKS = 8192;
+// chunks FP64 268 / 232 us, FP32 241 / 216; 16,800 chunks 399 / 449 and 321 / 417; 46,800 chunks
+// 903 / 1,215 and 639 / 1,131.  Between the first two the lines cross at 10,500 chunks (FP32) and 12,000.
+constexpr int FLOW_MAX_CHUNKS = 10240;
 
 int build_ilu_into(fos_euler *ctx, BlockIlu *b);
 
@@ -1477,7 +1493,7 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
     std::vector<Sched> part(cparts);
     host_parallel((size_t)nCh, cparts, [&](size_t k0_, size_t k1_, int pi) {
       Sched &S = part[pi];
-      std::vector<int> outs, loc(ICH), byLev(ICH), pend(ICH), rowLev(ICH);
+      std::vector<int> outs, loc(ICH), byLev(ICH), pend(ICH), rowLev(ICH), rowPos(ICH);
       const size_t cap = (size_t)(k1_ - k0_) * (ICH + SWEEP_ROWS * 4);  // rows plus padding of a few levels
       S.rec.reserve(cap);
       for (int ch = (int)k0_; ch < (int)k1_; ch++) {
@@ -1513,6 +1529,9 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
           nLev = std::max(nLev, h + 1);
         }
         S.levels.push_back(nLev);
+        for (int l = 0, p = 0; l < nLev; l++)
+          for (int i = 0; i < n; i++)
+            if (rowLev[i] == l) rowPos[i] = p++;
         // the chunk's neighbours outside it, and the records' code for each neighbour
         const int pb = rank[c0];
         outs.clear();
@@ -1565,7 +1584,7 @@ int build_ilu_into(fos_euler *ctx, BlockIlu *b) {
               rc.y |= (k >> 8) << (16 + j);
             }
             S.rec.push_back(rc);
-            if (!rowRec.empty()) rowRec[c0 + i] = make_uint2(rc.x, (rc.y & 0xFFF00u) | (unsigned)rowLev[i]);
+            if (!rowRec.empty()) rowRec[c0 + rowPos[i]] = make_uint2(rc.x, (rc.y & 0xFFF00u) | (unsigned)rowLev[i] | (unsigned)i << REC_BLK_SHIFT);
           }
           for (int a = nr; a < REC_SLOTS; a++) S.rec.push_back(empty);  // pad the step
           for (size_t m = r0; m < S.rec.size(); m++) S.rec[m].y |= (unsigned)(acc - acc0) << REC_BLK_SHIFT;
