@@ -408,39 +408,47 @@ __global__ __launch_bounds__(TPB) void mlp_layer_kernel(LayerArgs P) {
 
 // Weight gradient partials of one slice of rows: w[k][n] = sum_r A[r][k] D[r][n] for KB of A's columns and
 // all N of D's, and from the first column block b[n] = sum_r D[r][n].  The row index is the MFMA
-// reduction dimension, so both operands are needed by column: 32 rows of each are staged in LDS with
-// 16-byte loads (the next 32 in flight) and read back by column, 2 bytes at a time, each value for four
-// MFMAs.  Rows are padded by 16 bytes: the four row groups of a fragment then lie 16 banks apart.  Loaded
-// straight from memory 2 bytes at a time, once per 32 x 32 block, the four products took 64 us each and
-// the bias sums, a workgroup per column, 86 us each (65,536 rows); now 29 us for the wide layers and 17 us
-// for the narrow ones, bias sums included.  What bounds it now is the 2-byte LDS reads.
+// reduction dimension, so both operands are needed by column: 32 rows of each are staged in LDS, an octet
+// of each per thread, and read back by transposing LDS reads, four rows to a read.  Rows are padded by 32
+// bytes: the eight rows that 32 lanes read then lie on different banks.  A slice is 16 stages of little
+// work, so what bounded it was the latency of each: four stages are in flight, the LDS is double-buffered
+// (one barrier per stage), and eight waves share a slice rather than two slices of four, whose partials
+// would be twice the traffic.  Measured at 65,536 rows, wide layers / narrow ones: loaded from memory 2
+// bytes at a time 64 us each, and the bias sums 86; staged in LDS and read 2 bytes at a time, the next
+// stage in flight, 29 / 17 with the bias sums; transposing reads and eight waves 19 / 17; four stages in
+// flight 15 / 13 (two or eight: the same within 1 %).  With the loads under conditions, which force a wait
+// at each, four in flight took 32 / 28.
+constexpr int WG_T = 512, WG_AHEAD = 4;  // threads (eight waves); stages of 32 rows in flight, an even number
 template <int KB, int N>
-__global__ __launch_bounds__(256) void wgrad_kernel(int R, int rows, const uint16_t *__restrict__ A, int lda,
-                                                    const uint16_t *__restrict__ D, float *__restrict__ w,
-                                                    float *__restrict__ b) {
-  constexpr int WK = KB == 32 ? 1 : N == 32 ? 4 : 2, WN = 4 / WK;      // waves along k and n
-  constexpr int TK = KB / 16 / WK, TN = N / 16 / WN;                   // 16 x 16 tiles per wave
-  constexpr int SA = KB + 8, SD = N + 8, OA = KB / 8, OD = N / 8;      // LDS rows; octets per row
-  constexpr int LA = (32 * OA + 255) / 256, LD = (32 * OD + 255) / 256;  // octets per thread
-  __shared__ alignas(16) uint16_t sA[32 * SA], sD[32 * SD];
-  __shared__ float sB[256 * 8];
+__global__ __launch_bounds__(WG_T) void wgrad_kernel(int R, int rows, const uint16_t *__restrict__ A, int lda,
+                                                     const uint16_t *__restrict__ D, float *__restrict__ w,
+                                                     float *__restrict__ b) {
+  constexpr int WK = KB == 32 ? 1 : N == 32 ? 8 : 2, WN = 8 / WK;   // waves along k and n
+  constexpr int TK = KB / 16 / WK, TN = N / 16 / WN;                // 16 x 16 tiles per wave
+  constexpr int SA = KB + 16, SD = N + 16, OA = KB / 8, OD = N / 8;  // LDS rows; octets per row
+  constexpr int BUF = 32 * (SA + SD);
+  static_assert(32 * OA <= WG_T && 32 * OD <= WG_T && WG_T % OD == 0, "an octet of each operand per thread");
+  static_assert(2 * BUF * 2 >= WG_T * 8 * 4, "the bias sums fit the buffers");
+  __shared__ alignas(16) uint16_t sm[2][BUF];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, lr = lane & 15, lk = (lane >> 4) * 4;
   const int kc = blockIdx.y * KB, kb = (wave % WK) * TK * 16, nb = (wave / WK) * TN * 16;
   const int rb = blockIdx.x * rows, re = min(R, rb + rows);
-  uint4 a[LA], d[LD];
-  auto load = [&](int r0) {
-#pragma unroll
-    for (int j = 0; j < LA; j++) {
-      const int o = tid + 256 * j, r = r0 + o / OA;
-      a[j] = o < 32 * OA && r < re ? *reinterpret_cast<const uint4 *>(&A[(size_t)r * lda + kc + 8 * (o % OA)])
-                                   : make_uint4(0u, 0u, 0u, 0u);
-    }
-#pragma unroll
-    for (int j = 0; j < LD; j++) {
-      const int o = tid + 256 * j, r = r0 + o / OD;
-      d[j] = o < 32 * OD && r < re ? *reinterpret_cast<const uint4 *>(&D[(size_t)r * N + 8 * (o % OD)])
-                                   : make_uint4(0u, 0u, 0u, 0u);
-    }
+  const int ra = tid / OA, ca = 8 * (tid % OA), rd = tid / OD, cd = 8 * (tid % OD);  // this thread's octets
+  uint4 a[WG_AHEAD], d[WG_AHEAD];
+  // unconditional (rows past the slice repeat its last one and are zeroed on the way to LDS), so that no
+  // wait is forced before the next stages' loads issue
+  auto load = [&](int r0, uint4 &x, uint4 &y) {
+    x = *reinterpret_cast<const uint4 *>(&A[(size_t)min(r0 + ra, re - 1) * lda + kc + ca]);
+    y = *reinterpret_cast<const uint4 *>(&D[(size_t)min(r0 + rd, re - 1) * N + cd]);
+  };
+  // column lr of rows lk .. lk + 3 and 16 + lk .. 16 + lk + 3 of a 16-column tile: a transposing read gives
+  // lane l of 16 column l of the four rows that the lanes hold, four lanes of 8 bytes to a row
+  auto column = [&](const uint16_t *t, int stride) {
+    const uint16_t *q = t + (lk + lr / 4) * stride + 4 * (lr % 4);
+    typedef __attribute__((address_space(3))) bf16x4 *lp;
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(q));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)(q + 16 * stride));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
   };
   f32x4 acc[TK][TN];
 #pragma unroll
@@ -448,42 +456,37 @@ __global__ __launch_bounds__(256) void wgrad_kernel(int R, int rows, const uint1
 #pragma unroll
     for (int j = 0; j < TN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   float cs[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // column sums of this thread's octets of D (one column octet)
-  load(rb);
-  for (int r0 = rb; r0 < re; r0 += 32) {
-#pragma unroll
-    for (int j = 0; j < LA; j++) {
-      const int o = tid + 256 * j;
-      if (o < 32 * OA) *reinterpret_cast<uint4 *>(&sA[(o / OA) * SA + 8 * (o % OA)]) = a[j];
-    }
-#pragma unroll
-    for (int j = 0; j < LD; j++) {
-      const int o = tid + 256 * j;
-      if (o < 32 * OD) *reinterpret_cast<uint4 *>(&sD[(o / OD) * SD + 8 * (o % OD)]) = d[j];
-      const uint16_t *h = reinterpret_cast<const uint16_t *>(&d[j]);
+  auto stage = [&](uint16_t *sA, uint4 &x, uint4 &y, int r0) {
+    uint16_t *sD = sA + 32 * SA;
+    const unsigned mx = r0 + ra < re ? ~0u : 0u, my = r0 + rd < re ? ~0u : 0u;
+    x = make_uint4(x.x & mx, x.y & mx, x.z & mx, x.w & mx);
+    y = make_uint4(y.x & my, y.y & my, y.z & my, y.w & my);
+    if (ra < 32) *reinterpret_cast<uint4 *>(&sA[ra * SA + ca]) = x;
+    if (rd < 32) {
+      *reinterpret_cast<uint4 *>(&sD[rd * SD + cd]) = y;
+      const uint16_t *h = reinterpret_cast<const uint16_t *>(&y);
 #pragma unroll
       for (int e = 0; e < 8; e++) cs[e] += bf2f(h[e]);
     }
-    if (r0 + 32 < re) load(r0 + 32);
-    __syncthreads();
+    load(r0 + 32 * WG_AHEAD, x, y);
+    __syncthreads();  // one per stage: the other buffer is written next, which every wave has read by then
+    bf16x8 fa[TK], fd[TN];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      bf16x4 fa[TK], fd[TN];
+    for (int i = 0; i < TK; i++) fa[i] = column(sA + kb + 16 * i, SA);
 #pragma unroll
-      for (int i = 0; i < TK; i++)
+    for (int j = 0; j < TN; j++) fd[j] = column(sD + nb + 16 * j, SD);
 #pragma unroll
-        for (int e = 0; e < 4; e++) fa[i][e] = (short)sA[(16 * h + lk + e) * SA + kb + 16 * i + lr];
+    for (int i = 0; i < TK; i++)
 #pragma unroll
       for (int j = 0; j < TN; j++)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fa[i], fd[j], acc[i][j], 0, 0, 0);
+  };
 #pragma unroll
-        for (int e = 0; e < 4; e++) fd[j][e] = (short)sD[(16 * h + lk + e) * SD + nb + 16 * j + lr];
+  for (int q = 0; q < WG_AHEAD; q++) load(rb + 32 * q, a[q], d[q]);
+  for (int r0 = rb; r0 < re; r0 += 32 * WG_AHEAD)
 #pragma unroll
-      for (int i = 0; i < TK; i++)
-#pragma unroll
-        for (int j = 0; j < TN; j++)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(fa[i], fd[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();
-  }
+    for (int q = 0; q < WG_AHEAD; q++)
+      stage(sm[q & 1], a[q], d[q], r0 + 32 * q);
   w += (size_t)blockIdx.x * NPART;
 #pragma unroll
   for (int i = 0; i < TK; i++)
@@ -492,13 +495,15 @@ __global__ __launch_bounds__(256) void wgrad_kernel(int R, int rows, const uint1
 #pragma unroll
       for (int e = 0; e < 4; e++) w[(size_t)(kc + kb + 16 * i + lk + e) * N + nb + 16 * j + lr] = acc[i][j][e];
   if (blockIdx.y) return;
-  // thread tid summed column octet tid % OD (256 is a multiple of OD)
+  // thread tid summed column octet tid % OD
+  float *sB = reinterpret_cast<float *>(sm[0]);
+  __syncthreads();
 #pragma unroll
   for (int e = 0; e < 8; e++) sB[tid * 8 + e] = cs[e];
   __syncthreads();
   if (tid < N) {
     float s = 0.f;
-    for (int t = tid / 8; t < 256; t += OD) s += sB[t * 8 + tid % 8];
+    for (int t = tid / 8; t < WG_T; t += OD) s += sB[t * 8 + tid % 8];
     b[(size_t)blockIdx.x * NPART + tid] = s;
   }
 }
@@ -972,7 +977,7 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
   const dim3 gr((unsigned)(((size_t)R * (NH / 8) + 255) / 256)), blk(256);
   float *pt = L->part.p;
   // layer 3: dW3 = H2^T dO, db3 = sum dO; dP = (dO W3^T) silu'(pre2)
-  hipLaunchKernelGGL((wgrad_kernel<NH, NOP>), dim3(ns, 1), blk, 0, s, R, rows, L->H2.p, NH, L->dO16.p, pt + PW3, pt + PB3);
+  hipLaunchKernelGGL((wgrad_kernel<NH, NOP>), dim3(ns, 1), dim3(WG_T), 0, s, R, rows, L->H2.p, NH, L->dO16.p, pt + PW3, pt + PB3);
   LayerArgs P{};
   P.R = R;
   P.A = L->dO16.p;
@@ -988,7 +993,7 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
   float *preIn[2] = {L->pre1.p, L->pre0.p};
   const int offW[2] = {PW2, PW1}, offB[2] = {PB2, PB1};
   for (int l = 0; l < 2; l++) {
-    hipLaunchKernelGGL((wgrad_kernel<NH, NH>), dim3(ns, 2), blk, 0, s, R, rows, Hin[l], 256, L->dP.p, pt + offW[l],
+    hipLaunchKernelGGL((wgrad_kernel<NH, NH>), dim3(ns, 2), dim3(WG_T), 0, s, R, rows, Hin[l], 256, L->dP.p, pt + offW[l],
                        pt + offB[l]);
     P.A = L->dP.p;
     P.lda = NH;
@@ -1000,7 +1005,7 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
     hipLaunchKernelGGL(mp_backward_kernel, gr, blk, 0, s, R, nb, L->dX.p, preIn[l], L->dP.p);
   }
   // layer 0: dW0 = X^T dP, db0
-  hipLaunchKernelGGL((wgrad_kernel<NIP, NH>), dim3(ns, 1), blk, 0, s, R, rows, L->X.p, NIP, L->dP.p, pt + PW0, pt + PB0);
+  hipLaunchKernelGGL((wgrad_kernel<NIP, NH>), dim3(ns, 1), dim3(WG_T), 0, s, R, rows, L->X.p, NIP, L->dP.p, pt + PW0, pt + PB0);
   hipLaunchKernelGGL(wgrad_reduce, dim3((NPAR + 63) / 64), blk, 0, s, pt, ns, L->grad.p);
   FOS_HIP_TRY(hipGetLastError());
   FOS_HIP_TRY(hipStreamSynchronize(s));
