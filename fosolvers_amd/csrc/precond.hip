@@ -103,30 +103,30 @@ __device__ inline void anfj(double nx, double ny, double nz, double ux, double u
                             double g, double *J) {
   const double n[3] = {nx, ny, nz}, u[3] = {ux, uy, uz};
   const double v2 = ux * ux + uy * uy + uz * uz, vn = ux * nx + uy * ny + uz * nz;
-  const double g1 = g - 1.0, ic = 1.0 / c, g2 = g1 * ic * ic, M2 = v2 * ic * ic, Mn = vn * ic;
+  const double g1 = g - 1.0, c2 = c * c, M2 = v2 / c2, Mn = vn / c;
   const double av = fabs(vn);
   // entropy + shear part, weight |vn|
   J[0] = av * (1.0 - 0.5 * g1 * M2);
   for (int d = 0; d < 3; d++) J[1 + d] = av * (-(1.0 + 0.5 * g1 * M2) * u[d] + vn * n[d]);
   J[4] = av * (vn * vn - 0.5 * v2 * (1.0 + 0.5 * g1 * M2));
   for (int cc = 0; cc < 3; cc++) {
-    J[5 * (1 + cc)] = av * (g2 * u[cc]);
+    J[5 * (1 + cc)] = av * (g1 / c2 * u[cc]);
     for (int r = 0; r < 3; r++)
-      J[5 * (1 + cc) + 1 + r] = av * (g2 * u[r] * u[cc] - n[r] * n[cc] + (r == cc ? 1.0 : 0.0));
+      J[5 * (1 + cc) + 1 + r] = av * (g1 / c2 * u[r] * u[cc] - n[r] * n[cc] + (r == cc ? 1.0 : 0.0));
     J[5 * (1 + cc) + 4] = av * ((1.0 + 0.5 * g1 * M2) * u[cc] - vn * n[cc]);
   }
-  J[20] = av * (-g2);
-  for (int d = 0; d < 3; d++) J[21 + d] = av * (-g2 * u[d]);
+  J[20] = av * (-g1 / c2);
+  for (int d = 0; d < 3; d++) J[21 + d] = av * (-g1 / c2 * u[d]);
   J[24] = av * (-0.5 * g1 * M2);
   // acoustic parts, weights |vn -+ c|
   for (int s = -1; s <= 1; s += 2) {
     double a[3], b[3];
     for (int d = 0; d < 3; d++) {
       a[d] = u[d] + s * c * n[d];
-      b[d] = -0.5 * g2 * u[d] + s * 0.5 * n[d] * ic;
+      b[d] = -0.5 * g1 / c2 * u[d] + s * 0.5 * n[d] / c;
     }
     const double hh = H + s * vn * c, lam = fabs(vn + s * c);
-    const double t11 = 0.25 * g1 * M2 - s * 0.5 * Mn, t15 = 0.5 * g2;
+    const double t11 = 0.25 * g1 * M2 - s * 0.5 * Mn, t15 = 0.5 * g1 / c2;
     J[0] += lam * t11;
     for (int d = 0; d < 3; d++) J[1 + d] += lam * (a[d] * t11);
     J[4] += lam * (hh * t11);
@@ -139,6 +139,16 @@ __device__ inline void anfj(double nx, double ny, double nz, double ux, double u
     for (int d = 0; d < 3; d++) J[21 + d] += lam * (a[d] * t15);
     J[24] += lam * (hh * t15);
   }
+}
+
+// v of lane ^ m: within four lanes a permuting move, which leaves the LDS alone
+__device__ inline double lane_xor(double v, int m) {
+  if (m > 2) return __shfl_xor(v, m, 64);
+  const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+  const int lo = (int)u, hi = (int)(u >> 32);
+  const int a = m == 1 ? __builtin_amdgcn_mov_dpp(lo, 0xB1, 0xF, 0xF, true) : __builtin_amdgcn_mov_dpp(lo, 0x4E, 0xF, 0xF, true);
+  const int b = m == 1 ? __builtin_amdgcn_mov_dpp(hi, 0xB1, 0xF, 0xF, true) : __builtin_amdgcn_mov_dpp(hi, 0x4E, 0xF, 0xF, true);
+  return __longlong_as_double((long long)((unsigned long long)(unsigned)b << 32 | (unsigned)a));
 }
 
 __device__ inline void load_state(const double *y, int nC, int c, double g1, Prim<double> &q) {
@@ -273,11 +283,13 @@ __global__ __launch_bounds__(JAC_THREADS) void jac_exact_kernel(FluxLayout<doubl
 // One thread per (cell, face slot): NS consecutive lanes hold one cell.  Each lane forms its face's
 // neighbour block of JacC (a neighbour shares one face with the cell) and its
 // contribution to the diagonal block, which the cell's lanes sum by butterfly shuffles; the lanes
-// then zero the neighbour blocks no face wrote (facets).  What bounds it is FP64 arithmetic at 2.5 waves per
-// SIMD (the staged rows' LDS), then the 1000 bytes a cell that it writes.  Two states per lane (the cell's
-// own is one of them), two flux Jacobians chosen by side instead of three in two divergent branches, and one
-// reciprocal of c in |A~|: with the factorisation and an apply behind it 1.07M tets 1893 -> 1854 us, 6M
-// 9.24 -> 9.02 ms (the kernel 2.18 -> 1.96 ms).
+// then zero the neighbour blocks no face wrote (facets).  What bounds it is a chain of four dependent reads
+// and its FP64 arithmetic at 2.5 waves per SIMD (the staged rows' LDS), then the 1000 bytes a cell that it
+// writes.  Two states per lane (the cell's own is one of them) and two flux Jacobians chosen by side instead
+// of three in two divergent branches: with the factorisation and an apply behind it 1.07M tets 1893 -> 1864
+// us, 6M 9.24 -> 9.07 ms; the butterfly's steps within four lanes by permuting moves instead of 100 LDS
+// permutes: another 7 us and 0.08 ms (the kernel 2.18 -> 1.97 ms).  One reciprocal of c in |A~| would give
+// 0.5 % more, and entries up to an ulp further from exact ones.
 template <int NS>
 __global__ __launch_bounds__(JAC_THREADS) void jac_kernel(FluxLayout<double> L, const int *__restrict__ jslot,
                                                   const double *__restrict__ y, double *__restrict__ jac) {
@@ -342,7 +354,7 @@ __global__ __launch_bounds__(JAC_THREADS) void jac_kernel(FluxLayout<double> L, 
 #pragma unroll
   for (int m = 1; m < NS; m <<= 1) {
 #pragma unroll
-    for (int k = 0; k < 25; k++) D[k] += __shfl_xor(D[k], m, NS);
+    for (int k = 0; k < 25; k++) D[k] += lane_xor(D[k], m);
     written |= __shfl_xor(written, m, NS);
   }
 #pragma unroll
