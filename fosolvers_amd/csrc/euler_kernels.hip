@@ -395,7 +395,9 @@ __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(
   const int t = threadIdx.x;
   // A: the first face record and the nodes are loaded before the cells are staged
   if constexpr (!GATHER)
-    for (int k = t; k < 5 * CHUNK; k += TB) sA[k] = 0.0;
+#pragma unroll
+    for (int k = 0; k < (5 * CHUNK + TB - 1) / TB; k++)
+      if (5 * CHUNK % TB == 0 || k * TB + t < 5 * CHUNK) sA[k * TB + t] = 0.0;
   const int fb = L.chunkBeg[chunk], fe = L.chunkBeg[chunk + 1];
   uint2 recN = make_uint2(0u, 0u);
   // NT (working sets beyond the 256 MB last-level cache): the face records, node coordinates and
