@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "context.h"
+#include "learned_slices.h"
 
 namespace fos {
 
@@ -32,9 +33,6 @@ constexpr int OFF_W2 = OFF_B1 + NH, OFF_B2 = OFF_W2 + 2 * NH * NH, OFF_W3 = OFF_
 // operands are, then the bias gradients
 constexpr int PW3 = 0, PW2 = PW3 + NH * NOP, PW1 = PW2 + 2 * NH * NH, PW0 = PW1 + 2 * NH * NH, PB3 = PW0 + NIP * NH;
 constexpr int PB2 = PB3 + NOP, PB1 = PB2 + NH, PB0 = PB1 + NH, NPART = PB0 + NH;
-// rows per slice: 512, so that 65,536 rows give each of the 256 CUs work, and more where there would be
-// over 256 slices (whose partials the last pass reads)
-inline int slice_rows(size_t n) { return (int)std::max<size_t>(512, ((n + 255) / 256 + 31) / 32 * 32); }
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -848,9 +846,8 @@ int ensure_train(Learned *L, size_t n) {
   if (ensure_fwd(L, n)) return -1;
   if (L->capT >= n) return 0;
   L->capT = n;
-  const size_t rows = slice_rows(n), ns = (n + rows - 1) / rows;
   return (L->pre0.alloc(n * NH) || L->pre1.alloc(n * NH) || L->pre2.alloc(n * NH) || L->rh.alloc(n * 8) ||
-          L->e.alloc(n * 8) || L->ds.alloc(n * 8) || L->part.alloc(ns * NPART) || L->dO16.alloc(n * NOP) ||
+          L->e.alloc(n * 8) || L->ds.alloc(n * 8) || L->part.alloc(slice_room(n) * NPART) || L->dO16.alloc(n * NOP) ||
           L->dP.alloc(n * NH) || L->dX.alloc(n * 256) || L->bnbr.alloc(n * NBR) ||
           L->red.alloc(std::max<size_t>(1024, (n + 255) / 256 + 8))) ? -1 : 0;
 }
@@ -986,7 +983,12 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
   Learned *L = ctx->learned;
   hipStream_t s = ctx->stream;
   L->haveO = false;
-  if (ensure_train(L, R) || compute_scale(ctx, L, y)) return -1;
+  if (ensure_train(L, R)) return -1;
+  if (slice_count(R) * NPART > L->part.n) {  // slice_room's bound, checked before anything writes them
+    set_error("learned: %zu slices of a %d-row batch exceed the workspace", slice_count(R), R);
+    return -1;
+  }
+  if (compute_scale(ctx, L, y)) return -1;
   hipLaunchKernelGGL(batch_nbr_kernel, dim3((R + 255) / 256), dim3(256), 0, s, R, c0, L->nbr.p, L->bnbr.p);
   const int *nb = L->bnbr.p;
   if (forward(ctx, L, y, c0, R, nb, gamma, true)) return -1;
@@ -997,7 +999,7 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
                      L->e.p, L->ds.p, L->red.p);
   hipLaunchKernelGGL(loss_dO_kernel, dim3(gb), dim3(256), 0, s, R, nb, L->O.p, L->e.p, L->rh.p, L->ds.p, L->kappa.p,
                      L->dO16.p);
-  const int rows = slice_rows(R), ns = (R + rows - 1) / rows;
+  const int rows = (int)slice_rows(R), ns = (int)slice_count(R);
   const dim3 gr((unsigned)(((size_t)R * (NH / 8) + 255) / 256)), blk(256);
   float *pt = L->part.p;
   // layer 3: dW3 = H2^T dO, db3 = sum dO; dP = (dO W3^T) silu'(pre2)

@@ -166,6 +166,77 @@ def test_learned_gradient_of_a_batch_matches_oracle(cuda, start, size):
     assert loss2 == loss and np.array_equal(g, g2)
 
 
+def _torch_learned_gradient(X, nbr, par, S, r, delta, device):
+    """Loss and gradient of the learned preconditioner in plain FP64 torch (oracle/learned.c's definition,
+    for batches that the oracle's single thread takes too long for).  nbr: cells of the batch or -1."""
+    import torch
+    from tests.test_gpu_learned import BLOCKS, NH, NI, NO
+    n = len(X)
+    P = torch.tensor(np.asarray(par, np.float64), device=device, requires_grad=True)
+    shape = {"W0": (NI, NH), "W1": (2 * NH, NH), "W2": (2 * NH, NH), "W3": (NH, NO)}
+    W = {k: P[a:a + m].view(shape.get(k, (m,))) for k, (a, m) in BLOCKS.items()}
+    nb = torch.tensor(np.where(nbr < 0, n, nbr).astype(np.int64), device=device)
+    cnt = (nb < n).sum(1, keepdim=True).clamp(min=1)
+
+    def at(h, j):
+        return torch.cat([h, h.new_zeros(1, h.shape[1])]).index_select(0, nb[:, j])
+
+    def hidden(h, k):
+        m = (at(h, 0) + at(h, 1) + at(h, 2) + at(h, 3)) / cnt
+        return torch.nn.functional.silu(torch.cat([h, m], 1) @ W["W" + k] + W["b" + k])
+    x = torch.tensor(np.asarray(X, np.float64), device=device)
+    h = torch.nn.functional.silu(x @ W["W0"] + W["b0"])
+    kappa = (x[:, 18] * (1.0 + x[:, 19])).clamp(max=1.0)
+    o = (hidden(hidden(h, "1"), "2") @ W["W3"] + W["b3"]) * kappa[:, None]
+    sc = torch.tensor(np.asarray(S, np.float64), device=device)
+    rh, dh = r.view(5, n).T / sc, delta.view(5, n).T / sc
+    t = rh + (o[:, :25].reshape(n, 5, 5) * rh[:, None, :]).sum(2)
+    z = (1.0 + o[:, 29:30]) * t + sum(o[:, 25 + j:26 + j] * at(t, j) for j in range(4))
+    loss = ((z - dh) ** 2).sum() / n
+    loss.backward()
+    return float(loss.detach()), P.grad.cpu().numpy()
+
+
+def test_learned_gradient_after_a_larger_batch(cuda):
+    """Batches past 131,072 rows, where a slice is more than 512 rows (140,001 rows: 244 slices), then on the
+    same context a smaller batch with more slices (130,001 rows: 254): against the plain arithmetic with
+    the batch tests' tolerance (5e-2, derived there), and the second bitwise a fresh context's."""
+    import torch
+    from tests.test_gpu_learned import BLOCKS, _random_params, bf16
+    pg = M.box(30, 28, 28, 1.0, 0.5, 0.5, jitter=0.2, seed=3, renumber=fa.RENUMBER_CHUNKS)
+    fv = pg.up()
+    ctab = fa.CondTab(*M.conds("mixed"))
+    nC = fv.nC
+    assert nC == 141120
+    y = _dev(M.perturbed_state(fv.p[:nC], mach=0.7, seed=6, width=0.2))
+    gamma, start = 0.02, 7
+    nb0 = np.asarray(fv.neib)
+
+    def context():
+        eu = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA)
+        return eu, _random_params(eu, 5)
+    eu, p = context()
+    X, S = eu.learned_inputs(y, gamma)
+    rng = np.random.default_rng(1)
+    r = rng.standard_normal(5 * nC) * np.repeat(S, nC)
+    delta = 0.5 * r + 0.1 * rng.standard_normal(5 * nC) * np.repeat(S, nC)
+    r, delta = _dev(r), _dev(delta)
+    for size in (140_001, 130_001):
+        print(f"[case] learned gradient start={start} size={size}", flush=True)
+        cells = slice(start, start + size)
+        nb = np.where((nb0[cells] >= start) & (nb0[cells] < start + size), nb0[cells] - start, -1)
+        loss_t, g_t = _torch_learned_gradient(X[cells], nb, bf16(p), S, r.view(5, nC)[:, cells].reshape(-1),
+                                              delta.view(5, nC)[:, cells].reshape(-1), y.device)
+        loss, g = eu.learned_loss_grad(y, r, delta, gamma, start, size)
+        assert abs(loss - loss_t) <= 2e-2 * loss_t
+        worst = {k: M.rel(g[a:a + n].astype(np.float64), g_t[a:a + n]) for k, (a, n) in BLOCKS.items()}
+        print("  " + " ".join(f"{k} {e:.1e}" for k, e in worst.items()))
+        assert max(worst.values()) <= 5e-2
+    fresh, _p = context()
+    loss_f, g_f = fresh.learned_loss_grad(y, r, delta, gamma, start, size)
+    assert loss == loss_f and np.array_equal(g, g_f)
+
+
 @pytest.mark.parametrize("dims", [(1, 1, 1), (11, 1, 1), (13, 3, 3), (40, 10, 10)], ids=["6", "66", "702", "24000"])
 def test_learned_apply_matches_oracle_at_tile_edges(cuda, dims):
     """Inference (features, fused layers, apply) where the last 64-row group or 16-row tile is partial and
