@@ -686,11 +686,21 @@ struct fos_bdf {
     fos_euler *eu = static_cast<fos_euler *>(ud);
     return eu->stream == stream && !(eu->flags & FOS_ASYNC_CALLBACKS) ? eu : nullptr;
   }
-  // after a wait: 1 if a deferred callback's result was not finite
-  int deferred_check() {
+  // after a wait: 1 if a deferred callback's result was not finite.  A product's comes first, and the
+  // preconditioner solve of it (solved), which a callback that waits would have kept from being called, is
+  // not counted.
+  int deferred_check(bool solved) {
     fos_euler *eu = own_euler();
-    if (!eu || !eu->defer || !take_nonfinite(eu)) return 0;
-    set_error("%s: non-finite value in the result", eu->deferWho);
+    if (!eu || !eu->defer) return 0;
+    const unsigned bad = take_nonfinite(eu);
+    if (!bad) return 0;
+    const bool product = bad & 1u << fos_euler::NF_RESULT;
+    if (product && solved) {
+      st.nps--;
+      eu->counters[3]--;
+    }
+    set_error("%s: non-finite value in the result",
+              eu->deferWho[product ? fos_euler::NF_RESULT : fos_euler::NF_SOLVE]);
     return 1;
   }
   template <class TV>
@@ -738,7 +748,7 @@ struct fos_bdf {
       }
       double bb;
       if (dots<TV>(nullptr, 0, r, dres.p, true) || fetch(1, &bb)) return -1;  // GMRES's own weights
-      if (deferred_check()) return 1;
+      if (deferred_check(precd)) return 1;
       double beta = std::sqrt(bb);
       if (beta0 < 0) beta0 = beta;
       const double tol = absTol > 0.0 ? absTol : linTol * beta0;
@@ -785,7 +795,7 @@ struct fos_bdf {
         std::fill(hc.begin(), hc.end(), 0.0);
         std::vector<double> hp(j + 2);
         if (dots<TV>(V, j + 1, w, hcol.p, true, vj, theta) || fetch(j + 2, hp.data())) return -1;
-        if (deferred_check()) {
+        if (deferred_check(precd)) {
           iters--;  // not an iteration: its product or preconditioner solve failed
           return 1;
         }

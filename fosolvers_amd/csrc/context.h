@@ -80,13 +80,16 @@ struct fos_euler {
   fos::DBuf<int> dStatus;
   fos::Learned *learned = nullptr;
 
-  // non-finite results: the kernels that write a callback's output set this word in pinned host memory
-  // (dNonFinite: its device address); a callback reads and clears it once the stream is done, unless
-  // FOS_ASYNC_CALLBACKS, where it accumulates until fos_euler_nonfinite.  While the integrator sets defer,
-  // the callbacks return without waiting and it takes the word at its next wait (take_nonfinite).
+  // non-finite results: the kernels that write a callback's output set a word in pinned host memory
+  // (hNonFinite[NF_RESULT]: residuals and products, [NF_SOLVE]: preconditioner solves; dNonFinite: their
+  // device address); a callback reads and clears them once the stream is done, unless
+  // FOS_ASYNC_CALLBACKS, where they accumulate until fos_euler_nonfinite.  While the integrator sets defer,
+  // the callbacks return without waiting and it takes the words at its next wait (take_nonfinite); deferWho
+  // names the last callback of each kind.
+  enum { NF_RESULT = 0, NF_SOLVE = 1, NF_WORDS = 2 };
   unsigned *hNonFinite = nullptr, *dNonFinite = nullptr;
   bool defer = false;
-  const char *deferWho = "";
+  const char *deferWho[NF_WORDS] = {"", ""};
 
   // the host's N_Vector data accessor for the *_nv callbacks (N_VGetArrayPointer or its device form)
   fos_nvector_data_fn nvData = nullptr;
@@ -115,9 +118,9 @@ int ensure_pair_arrays(fos_euler *ctx);
 // End of a callback: unless FOS_ASYNC_CALLBACKS, wait for the stream and return 1 (recoverable, the
 // SUNDIALS convention) when a kernel flagged a non-finite output since the last check, 0 otherwise
 // (the word is cleared); -1 on a HIP error.
-int finish_call(fos_euler *ctx, const char *who);
-// Whether a kernel flagged a non-finite output; clears the word.  The stream must be done.
-bool take_nonfinite(fos_euler *ctx);
+int finish_call(fos_euler *ctx, const char *who, int word = fos_euler::NF_RESULT);
+// The words that a kernel flagged a non-finite output in, as a mask; clears them.  The stream must be done.
+unsigned take_nonfinite(fos_euler *ctx);
 // Resolves, once per device, the address of the file-scope scratch array behind
 // fos_euler_jtimes_noalloc (with that device current).  Called by fos_euler_create.
 int resolve_noalloc_scratch(int device);

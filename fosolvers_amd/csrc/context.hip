@@ -691,12 +691,17 @@ static int jvp_dev(fos_euler *ctx, const double *v, double *out, const double *y
                      : launch_jvp<double, double>(ctx->L64, y, v, out, ctx->stream, nf, newton, ngam);
 }
 
-bool take_nonfinite(fos_euler *ctx) { return __atomic_exchange_n(ctx->hNonFinite, 0u, __ATOMIC_RELAXED) != 0; }
+unsigned take_nonfinite(fos_euler *ctx) {
+  unsigned mask = 0;
+  for (int w = 0; w < fos_euler::NF_WORDS; w++)
+    if (__atomic_exchange_n(ctx->hNonFinite + w, 0u, __ATOMIC_RELAXED)) mask |= 1u << w;
+  return mask;
+}
 
-int finish_call(fos_euler *ctx, const char *who) {
+int finish_call(fos_euler *ctx, const char *who, int word) {
   if (ctx->flags & FOS_ASYNC_CALLBACKS) return 0;
   if (ctx->defer) {
-    ctx->deferWho = who;
+    ctx->deferWho[word] = who;
     return 0;
   }
   FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -763,13 +768,13 @@ fos_euler *fos_euler_create(const fos_fv_grid *grid, const fos_cond_tab *bc, dou
     delete ctx;
     return nullptr;
   }
-  if (hipHostMalloc((void **)&ctx->hNonFinite, sizeof(unsigned)) != hipSuccess ||
+  if (hipHostMalloc((void **)&ctx->hNonFinite, sizeof(unsigned) * fos_euler::NF_WORDS) != hipSuccess ||
       hipHostGetDevicePointer((void **)&ctx->dNonFinite, ctx->hNonFinite, 0) != hipSuccess) {
     set_error("fos_euler_create: pinned host allocation failed");
     delete ctx;
     return nullptr;
   }
-  *ctx->hNonFinite = 0;
+  std::fill_n(ctx->hNonFinite, (int)fos_euler::NF_WORDS, 0u);
   return ctx;
 }
 
@@ -942,7 +947,9 @@ int fos_euler_nonfinite(fos_euler *ctx, int clear) {
   if (!ctx) return -1;
   FOS_HIP_TRY(hipStreamSynchronize(ctx->stream));
   if (clear) return take_nonfinite(ctx) ? 1 : 0;
-  return __atomic_load_n(ctx->hNonFinite, __ATOMIC_RELAXED) != 0 ? 1 : 0;
+  for (int w = 0; w < fos_euler::NF_WORDS; w++)
+    if (__atomic_load_n(ctx->hNonFinite + w, __ATOMIC_RELAXED)) return 1;
+  return 0;
 }
 
 // ---- the callbacks with SUNDIALS' N_Vector signatures: resolve the data pointers, forward

@@ -1064,7 +1064,7 @@ int learned_psolve(fos_euler *ctx, const double *r, double *z) {
   hipLaunchKernelGGL(apply_t_kernel, dim3(gb), dim3(256), 0, ctx->stream, nC, 0, nC, L->O.p, L->scale.p, r, L->t.p,
                      nullptr);
   hipLaunchKernelGGL(apply_z_kernel, dim3(gb), dim3(256), 0, ctx->stream, nC, nC, L->nbr.p, L->scale.p, L->t.p,
-                     z, ctx->dNonFinite);
+                     z, ctx->dNonFinite + fos_euler::NF_SOLVE);
   FOS_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -1171,7 +1171,7 @@ int fos_euler_psolve_learned(double t, const double *y, const double *fy, const 
   if (!ctx || !ctx->learned || !ctx->learned->ready) { set_error("psolve_learned: not set up"); return -1; }
   ctx->counters[3]++;
   if (learned_psolve(ctx, r, z)) return -1;
-  return finish_call(ctx, "psolve_learned");
+  return finish_call(ctx, "psolve_learned", fos_euler::NF_SOLVE);
 }
 
 }  // extern "C"

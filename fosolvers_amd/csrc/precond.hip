@@ -1792,11 +1792,11 @@ static int ilu_sweeps(fos_euler *ctx, const TF *Lf, const TF *Uf, const TF *Db, 
     const int nCh = (b->nC + ICH - 1) / ICH;
     hipLaunchKernelGGL(ilu_flow_kernel<TF>, dim3(std::min(2 * nCh, b->flowGrid)), dim3(FLOW_THREADS), 0, ctx->stream,
                        b->nC, nCh, b->dFMeta.p, b->dBMeta.p, b->dFRow.p, b->dBRow.p, b->dFOutCell.p, b->dBOutCell.p,
-                       Lf, Uf, Db, r, z, b->dX.p, b->dCtl.p, ctx->dNonFinite);
+                       Lf, Uf, Db, r, z, b->dX.p, b->dCtl.p, ctx->dNonFinite + fos_euler::NF_SOLVE);
     return 0;
   }
   if (!b->eager && !b->solveChain.ready()) {
-    if (ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite,
+    if (ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite + fos_euler::NF_SOLVE,
                    [&](auto k, dim3 g, dim3 bl, size_t lds, auto... a) {
                      return b->solveChain.add(k, g, bl, lds, a...);
                    }) ||
@@ -1807,7 +1807,7 @@ static int ilu_sweeps(fos_euler *ctx, const TF *Lf, const TF *Uf, const TF *Db, 
   }
   hipLaunchKernelGGL(ilu_io_kernel, dim3(1), dim3(64), 0, ctx->stream, b->dIo.p, r, z);
   if (b->eager) {
-    ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite, [&](auto k, dim3 g, dim3 bl, size_t lds, auto... a) {
+    ilu_levels(b, Lf, Uf, Db, ctx->dNonFinite + fos_euler::NF_SOLVE, [&](auto k, dim3 g, dim3 bl, size_t lds, auto... a) {
       hipLaunchKernelGGL(k, g, bl, lds, ctx->stream, a...);
       return 0;
     });
@@ -1852,10 +1852,10 @@ int bjac_solve(fos_euler *ctx, const double *r, double *z) {
   const int nC = ctx->nC;
   if (ctx->flags & FOS_PREC_FP32)
     hipLaunchKernelGGL(bjac_apply_kernel<float>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dBj32.p, r, z,
-                       ctx->dNonFinite);
+                       ctx->dNonFinite + fos_euler::NF_SOLVE);
   else
     hipLaunchKernelGGL(bjac_apply_kernel<double>, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, b->dBj.p, r, z,
-                       ctx->dNonFinite);
+                       ctx->dNonFinite + fos_euler::NF_SOLVE);
   FOS_HIP_TRY(hipGetLastError());
   return 0;
 }
@@ -1923,10 +1923,10 @@ int fos_euler_psolve(double t, const double *y, const double *fy, const double *
   if (ctx->flags & FOS_VECTORS_ON_HOST) {
     if (stage_in(ctx, ctx->hR, r) || ensure_vec(ctx->hZ, 5 * (size_t)ctx->nC)) return -1;
     if (ilu_solve(ctx, ctx->hR.p, ctx->hZ.p) || stage_out(ctx, ctx->hZ, z)) return -1;
-    return finish_call(ctx, "psolve");
+    return finish_call(ctx, "psolve", fos_euler::NF_SOLVE);
   }
   if (ilu_solve(ctx, r, z)) return -1;
-  return finish_call(ctx, "psolve");
+  return finish_call(ctx, "psolve", fos_euler::NF_SOLVE);
 }
 
 int fos_euler_psetup_bjac(double t, const double *y, const double *fy, int jok, int *jcur, double gamma,
@@ -1954,7 +1954,7 @@ int fos_euler_psolve_bjac(double t, const double *y, const double *fy, const dou
     return -1;
   }
   if (bjac_solve(ctx, r, z)) return -1;
-  return finish_call(ctx, "psolve_bjac");
+  return finish_call(ctx, "psolve_bjac", fos_euler::NF_SOLVE);
 }
 
 int fos_euler_ilu_order(fos_euler *ctx, int *order) {

@@ -302,6 +302,62 @@ def test_integrator_reports_a_nonfinite_product_like_the_callback(cuda, precond)
     assert M.rel(outs[1].cpu().numpy(), outs[2].cpu().numpy()) <= 1e-13
 
 
+@pytest.mark.parametrize("precond", ["ilu", "bjac", None])
+def test_integrator_names_the_nonfinite_callback(cuda, precond):
+    """A product that overflows is named, also where a preconditioner solve of its result was launched before
+    GMRES's wait, and no counter counts that solve: the integrator's and the context's counters are those
+    of the callbacks that check for themselves.  State and step: the factors' largest entries (2e35) fit
+    FP32, the enthalpy (2e40) that the product forms does not."""
+    from fosolvers_amd import _capi
+    import torch
+    print(f"[case] name of a non-finite callback precond={precond}", flush=True)
+    pg = M.box(8, 4, 4, jitter=0.2, seed=3, renumber=fa.RENUMBER_CHUNKS)
+    fv = pg.up()
+    ctab = fa.CondTab(*M.conds("wall"))
+    good = _dev(M.perturbed_state(fv.p[:fv.nC], mach=0.3, seed=5))
+    scale = torch.ones(5, fv.nC, dtype=torch.float64, device="cuda")
+    scale[0], scale[4] = 1e-20, 1e20
+    huge = (good.view(5, -1) * scale).reshape(-1).contiguous()
+    counts = []
+    for fused, name in ((True, "newton_matvec_analytic"), (False, "jtimes_analytic")):
+        eu = fa.Euler(fv, ctab, r=M.R, gamma=M.GAMMA, flags=fa.PREC_FP32)
+        b = fa.BDFNewtonKrylov.for_euler(eu, maxl=20, precond=precond, jtimes="analytic", fused=fused)
+        b.set_newton(tol=1e-8, max_iter=20, lin_tol=1e-3, max_restarts=10)
+        b.set_dt(1e-26)
+        b.set_iv(0.0, huge)
+        assert b.step(0.0, torch.zeros_like(good))[0] == 1
+        assert _capi.last_error() == f"{name}: non-finite value in the result"
+        st = b.stats()
+        counts.append(({k: st[k] for k in ("nfe", "nli", "npe", "nps", "njv")}, list(eu.counters())))
+    print(f"  {counts[0]}")
+    assert counts[0] == counts[1] and counts[0][0]["njv"] == 1
+
+
+def test_integrator_names_the_nonfinite_solve(cuda):
+    """A preconditioner whose output overflows FP32 on a good state: the solve is named and counted, and no
+    product was formed."""
+    from fosolvers_amd import _capi
+    from tests.test_gpu_learned import BLOCKS, _random_params
+    import torch
+    print("[case] name of a non-finite solve", flush=True)
+    pg = M.box(8, 4, 4, jitter=0.2, seed=3, renumber=fa.RENUMBER_CHUNKS)
+    fv = pg.up()
+    eu = fa.Euler(fv, fa.CondTab(*M.conds("wall")), r=M.R, gamma=M.GAMMA)
+    p = _random_params(eu, 5)
+    a, n = BLOCKS["b3"]
+    p[a:a + n] = 3e38  # an output of this size times itself overflows
+    eu.learned_set_params(p)
+    b = fa.BDFNewtonKrylov.for_euler(eu, maxl=20, precond="learned", jtimes="analytic")
+    b.set_newton(tol=1e-8, max_iter=20, lin_tol=1e-3, max_restarts=10)
+    b.set_dt(1e-3)
+    good = _dev(M.perturbed_state(fv.p[:fv.nC], mach=0.3, seed=5))
+    b.set_iv(0.0, good)
+    assert b.step(0.0, torch.zeros_like(good))[0] == 1
+    assert _capi.last_error() == "psolve_learned: non-finite value in the result"
+    st = b.stats()
+    assert (st["nps"], st["njv"], st["nli"]) == (1, 0, 0) and not eu.nonfinite()
+
+
 @pytest.mark.parametrize("kind", ["mixed", "wall"])
 @pytest.mark.parametrize("dims", [(1, 1, 1), (43, 2, 3), (31, 27, 26), (33, 27, 26)],
                          ids=["6", "1548", "130572", "138996"])
