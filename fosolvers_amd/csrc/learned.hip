@@ -21,18 +21,13 @@
 #include <vector>
 
 #include "context.h"
-#include "learned_slices.h"
+#include "learned_space.h"
 
 namespace fos {
 
-constexpr int NI = 20, NIP = 32, NH = 128, NO = 30, NOP = 32, NBR = 4, NTR = 12;
 constexpr int NPAR = NI * NH + NH + 2 * NH * NH + NH + 2 * NH * NH + NH + NH * NO + NO;
 constexpr int OFF_W0 = 0, OFF_B0 = OFF_W0 + NI * NH, OFF_W1 = OFF_B0 + NH, OFF_B1 = OFF_W1 + 2 * NH * NH;
 constexpr int OFF_W2 = OFF_B1 + NH, OFF_B2 = OFF_W2 + 2 * NH * NH, OFF_W3 = OFF_B2 + NH, OFF_B3 = OFF_W3 + NH * NO;
-// The weight-gradient partials of one slice of rows: the layers' [K][N] products, padded as their
-// operands are, then the bias gradients
-constexpr int PW3 = 0, PW2 = PW3 + NH * NOP, PW1 = PW2 + 2 * NH * NH, PW0 = PW1 + 2 * NH * NH, PB3 = PW0 + NIP * NH;
-constexpr int PB2 = PB3 + NOP, PB1 = PB2 + NH, PB0 = PB1 + NH, NPART = PB0 + NH;
 
 typedef short bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -57,7 +52,7 @@ __device__ inline float dsilu_f(float x) {
   return s * (1.0f + x * (1.0f - s));
 }
 
-struct Learned {
+struct Learned : LearnedSpace<DBuf> {
   int nC = 0;
   bool ready = false, haveO = false;  // parameters set; network output O computed for the mesh
   long long step = 0;
@@ -67,15 +62,6 @@ struct Learned {
   DBuf<int> nbr;          // [nC][4] cell neighbours (-1 none)
   DBuf<float> geo;        // [nC][13] log(v/vmean), area normals / v^(2/3) per neib slot
   DBuf<float> scale;      // [8]: S[5], then scratch
-  // forward activations (rows = max(nC used for inference, training batch))
-  size_t capF = 0, capT = 0;
-  DBuf<uint16_t> X, H0, H1, H2;  // X [.][32], H0/H1 [.][256] = (h | mean_nb h), H2 [.][128]
-  DBuf<float> O, t, kappa;       // O [.][32] network output, t [.][12] = B^ r^ and the weights, kappa [.] output scale
-  // training-only buffers (rows = batch)
-  DBuf<float> pre0, pre1, pre2, rh, e, ds, part;
-  DBuf<uint16_t> dO16, dP, dX;   // dO16 [.][32], dP [.][128], dX [.][256]
-  DBuf<int> bnbr;                // batch-local neighbours [.][4]
-  DBuf<double> red;              // reductions
   double *pinned = nullptr, *dpinned = nullptr;  // the loss in host memory, and its device address
   ~Learned() {
     if (pinned) (void)hipHostFree(pinned);
@@ -835,23 +821,6 @@ void layer(hipStream_t s, const LayerArgs &P) {
   hipLaunchKernelGGL((mlp_layer_kernel<K, N, FEAT, MEAN, TAIL, EPI>), dim3(grid), dim3(TPB), lds, s, P);
 }
 
-int ensure_fwd(Learned *L, size_t n) {
-  if (L->capF >= n) return 0;
-  L->capF = n;
-  return (L->X.alloc(n * NIP) || L->H0.alloc(n * 256) || L->H1.alloc(n * 256) || L->H2.alloc(n * NH) ||
-          L->O.alloc(n * NOP) || L->t.alloc(n * NTR) || L->kappa.alloc(n)) ? -1 : 0;
-}
-
-int ensure_train(Learned *L, size_t n) {
-  if (ensure_fwd(L, n)) return -1;
-  if (L->capT >= n) return 0;
-  L->capT = n;
-  return (L->pre0.alloc(n * NH) || L->pre1.alloc(n * NH) || L->pre2.alloc(n * NH) || L->rh.alloc(n * 8) ||
-          L->e.alloc(n * 8) || L->ds.alloc(n * 8) || L->part.alloc(slice_room(n) * NPART) || L->dO16.alloc(n * NOP) ||
-          L->dP.alloc(n * NH) || L->dX.alloc(n * 256) || L->bnbr.alloc(n * NBR) ||
-          L->red.alloc(std::max<size_t>(1024, (n + 255) / 256 + 8))) ? -1 : 0;
-}
-
 int compute_scale(fos_euler *ctx, Learned *L, const double *y) {
   const int nb = std::max(1, std::min(256, (ctx->nC + SC_T - 1) / SC_T));
   hipLaunchKernelGGL(scale_partial, dim3(nb), dim3(SC_T), 0, ctx->stream, ctx->nC, y, L->red.p);
@@ -955,7 +924,7 @@ int create_learned(fos_euler *ctx) {
       L->m1.alloc(NPAR) || L->m2.alloc(NPAR) || L->grad.alloc(NPAR) || L->bias.alloc(3 * NH + NOP) ||
       L->W0t.alloc(NH * NIP) || L->W1t.alloc(NH * 256) || L->W2t.alloc(NH * 256) || L->W3t.alloc(NOP * NH) ||
       L->W1b.alloc(256 * NH) || L->W2b.alloc(256 * NH) || L->W3b.alloc(NH * NOP) || L->scale.alloc(8) ||
-      L->red.alloc(1024) || hipHostMalloc((void **)&L->pinned, sizeof(double)) != hipSuccess ||
+      hipHostMalloc((void **)&L->pinned, sizeof(double)) != hipSuccess ||
       hipHostGetDevicePointer((void **)&L->dpinned, L->pinned, 0) != hipSuccess) {
     if (!L->pinned) set_error("learned preconditioner: pinned host buffer allocation failed");
     delete L;
@@ -983,7 +952,7 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
   Learned *L = ctx->learned;
   hipStream_t s = ctx->stream;
   L->haveO = false;
-  if (ensure_train(L, R)) return -1;
+  if (L->train(R)) return -1;
   if (slice_count(R) * NPART > L->part.n) {  // slice_room's bound, checked before anything writes them
     set_error("learned: %zu slices of a %d-row batch exceed the workspace", slice_count(R), R);
     return -1;
@@ -1048,7 +1017,7 @@ int learned_psetup(fos_euler *ctx, const double *y, double gamma) {
     return -1;
   }
   L->haveO = false;  // training overwrites O with batch rows; the mesh output is recomputed here
-  if (ensure_fwd(L, ctx->nC) || compute_scale(ctx, L, y)) return -1;
+  if (L->forward(ctx->nC) || compute_scale(ctx, L, y)) return -1;
   if (forward(ctx, L, y, 0, ctx->nC, L->nbr.p, gamma, false)) return -1;
   L->haveO = true;
   return 0;
@@ -1134,7 +1103,7 @@ int fos_learned_inputs(fos_euler *ctx, const double *y, double gamma, float *X, 
   Learned *L = ctx->learned;
   const int nC = ctx->nC;
   L->haveO = false;
-  if (ensure_fwd(L, nC) || compute_scale(ctx, L, y)) return -1;
+  if (L->forward(nC) || compute_scale(ctx, L, y)) return -1;
   hipLaunchKernelGGL(features_kernel, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, 0, nC, y, L->geo.p,
                      L->scale.p, gamma, ctx->gamm, L->X.p);
   FOS_HIP_TRY(hipGetLastError());
