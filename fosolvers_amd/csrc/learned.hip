@@ -836,6 +836,7 @@ int forward(fos_euler *ctx, Learned *L, const double *y, int c0, int R, const in
   // training also stores the features, the means, the last hidden layer and the layers' inputs to silu
   // (the weight gradients read [h, mean h] as one row); inference keeps the hidden rows at 256 bytes
   const int ld = keepPre ? 256 : NH;
+  uint16_t *h0 = keepPre ? L->HM0.p : L->H0.p, *h1 = keepPre ? L->HM1.p : L->H1.p;
   LayerArgs P{};
   P.R = R;
   P.lda = P.ldo = ld;
@@ -852,22 +853,22 @@ int forward(fos_euler *ctx, Learned *L, const double *y, int c0, int R, const in
   P.Bn = L->W0t.p;
   P.bias = bias;
   P.pre = keepPre ? L->pre0.p : nullptr;
-  P.outb = L->H0.p;
+  P.outb = h0;
   layer<NIP, NH, true, false, false, EPI_SILU>(s, P);
-  P.A = L->H0.p;
+  P.A = h0;
   P.Bn = L->W1t.p;
   P.bias = bias + NH;
   P.pre = keepPre ? L->pre1.p : nullptr;
-  P.outb = L->H1.p;
-  P.meanOut = keepPre ? L->H0.p : nullptr;
+  P.outb = h1;
+  P.meanOut = keepPre ? h0 : nullptr;
   layer<256, NH, false, true, false, EPI_SILU>(s, P);
-  P.A = L->H1.p;
+  P.A = h1;
   P.Bn = L->W2t.p;
   P.bias = bias + 2 * NH;
   P.pre = keepPre ? L->pre2.p : nullptr;
   P.outb = keepPre ? L->H2.p : nullptr;
   P.ldo = NH;
-  P.meanOut = keepPre ? L->H1.p : nullptr;
+  P.meanOut = keepPre ? h1 : nullptr;
   P.B3 = L->W3t.p;
   P.bias3 = bias + 3 * NH;
   P.O = L->O.p;
@@ -983,7 +984,7 @@ int loss_grad(fos_euler *ctx, const double *y, const double *r, const double *de
   P.ldo = NH;
   layer<NOP, NH, false, false, false, EPI_DSILU>(s, P);
   // layers 2 and 1: dW = [h, m]^T dP, db = sum dP; dX = dP W^T; dP <- mp-backward(dX) silu'(pre)
-  const uint16_t *Hin[2] = {L->H1.p, L->H0.p};
+  const uint16_t *Hin[2] = {L->HM1.p, L->HM0.p};
   const uint16_t *Wb[2] = {L->W2b.p, L->W1b.p};
   float *preIn[2] = {L->pre1.p, L->pre0.p};
   const int offW[2] = {PW2, PW1}, offB[2] = {PB2, PB1};
@@ -1017,7 +1018,7 @@ int learned_psetup(fos_euler *ctx, const double *y, double gamma) {
     return -1;
   }
   L->haveO = false;  // training overwrites O with batch rows; the mesh output is recomputed here
-  if (L->forward(ctx->nC) || compute_scale(ctx, L, y)) return -1;
+  if (L->apply(ctx->nC) || compute_scale(ctx, L, y)) return -1;
   if (forward(ctx, L, y, 0, ctx->nC, L->nbr.p, gamma, false)) return -1;
   L->haveO = true;
   return 0;
@@ -1103,7 +1104,7 @@ int fos_learned_inputs(fos_euler *ctx, const double *y, double gamma, float *X, 
   Learned *L = ctx->learned;
   const int nC = ctx->nC;
   L->haveO = false;
-  if (L->forward(nC) || compute_scale(ctx, L, y)) return -1;
+  if (L->inputs(nC) || compute_scale(ctx, L, y)) return -1;
   hipLaunchKernelGGL(features_kernel, dim3((nC + 255) / 256), dim3(256), 0, ctx->stream, nC, 0, nC, y, L->geo.p,
                      L->scale.p, gamma, ctx->gamm, L->X.p);
   FOS_HIP_TRY(hipGetLastError());
