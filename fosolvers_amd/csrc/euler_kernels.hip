@@ -362,14 +362,13 @@ __device__ inline void boundary_prim(const TetLayout<TC> &L, int g, const Prim<T
 // faces in slot order (FP64 sums, bitwise reproducible), else each face adds its flux to the sums with
 // LDS atomics.  The FP32 residual and difference quotients gather: their fluxes are half as wide, and
 // the ten FP64 atomics of a face took about half of the LDS pipe, which was busy 78 % of the kernel
-// (6M tets, FP32 residual: 151 -> 134 us).  In FP64 the parked fluxes cost a workgroup per CU and the
+// (6M tets, FP32 residual: 151 -> 137 us).  In FP64 the parked fluxes cost a workgroup per CU and the
 // slots 8 bytes per cell, and the kernel moves its traffic at the copy rate already (6M tets: 210 us,
 // 251 gathered; 222 with the fluxes held in registers until the staged cells' space is free); the
 // analytic Jv is bound by its arithmetic (FP32, 6M tets: 319 us, 323 gathered).
 template <class TC>
 constexpr bool tet_gathers(int mode) { return sizeof(TC) == 4 && mode != JVP; }
 
-//
 // TB > THREADS (small meshes, SMALL_CHUNKS): more threads per chunk, and the ghost states formed here.
 template <class TS, class TC, int MODE, int NS, bool NT, int TB = THREADS>
 __global__ __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(
@@ -563,10 +562,11 @@ __global__ __launch_bounds__(256) void ghost_kernel(TetLayout<TC> L, const TS *_
 // On a mesh of few chunks the chip is not full and a chunk's time counts: twice the threads per chunk halve
 // its face sweeps (a chunk has ~620 faces), and the ghost states are formed in the face pass, whose
 // register count (158 against 96) does not matter then, instead of by a launch of their own.  FP64 residual
-// and difference quotient; the FP32 forms keep one arithmetic on every mesh size.  Measured per
+// and difference quotient only: the FP32 forms have not been measured this way.  Measured per
 // residual, without the callback's wait: 6,000 tets 15.0 -> 7.6 us, 24,000 14.7 -> 7.8, 104,000 (405
 // chunks) 15.0 -> 11.6, 270,000 (1,055 chunks) 20.8 -> 24.0.  768 and 1024 threads were slower (24,000
-// tets: 8.1, 9.5 us).  The generic kernel gains nothing from more threads (95,000 hexes, 370 chunks: the same).
+// tets: 8.1, 9.5 us).  The generic kernel gains nothing from more threads (95,000 hexes, 370 chunks: 25.4
+// -> 25.9 us a callback).
 constexpr int SMALL_CHUNKS = 512, SMALL_THREADS = 512;
 
 constexpr size_t TET_LDS_LIMIT = 65536;

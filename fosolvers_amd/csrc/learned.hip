@@ -6,10 +6,9 @@
 // (S = per-variable RMS of the state), a fixed linear operator for GMRES.  Trained with Adam on
 // pairs (r, target) at the solver's states, loss |S^-1 (P r - target)|^2.
 //
-// Dense layers run on MFMA: BF16 weights and activations, FP32 accumulation.  The forward layers
-// and the backward data products use v_mfma_f32_16x16x32_bf16 in persistent workgroups
-// (mlp_layer_kernel), the weight gradients (MFMA reductions over cells) v_mfma_f32_16x16x16_bf16.  FP32
-// master weights and Adam moments.  Parameter packing (flat FP32): W0[20][128] b0 W1[256][128] b1 W2[256][128] b2
+// Dense layers run on MFMA (v_mfma_f32_16x16x32_bf16): BF16 weights and activations, FP32 accumulation; the
+// forward layers and the backward data products in persistent workgroups (mlp_layer_kernel), the weight
+// gradients as reductions over cells (wgrad_kernel).  FP32 master weights and Adam moments.  Parameter packing (flat FP32): W0[20][128] b0 W1[256][128] b1 W2[256][128] b2
 // W3[128][30] b3, the same as the oracle (oracle/learned.c).
 #include <hip/hip_runtime.h>
 
@@ -145,8 +144,8 @@ __device__ inline float out_kappa(uint4 octet2) {
 // A's rows (training: the weight gradients read it).
 // TAIL (layer 2): the output layer's 128 x 32 product and the output scale follow on the lane's own
 // octets, so the last hidden layer is not stored (outb, when given, still receives it: training).
-// At 1.5M cells, per layer: 0 with the features 48 + 184 -> 128 us, 1 399 -> 327 us, 2 with the output
-// layer and its scale 399 + 110 + 102 -> 347 us (the whole set-up and apply 1,382 -> 844 us), all bitwise
+// At 1.5M cells, per layer: 0 with the features 48 + 184 -> 124 us, 1 399 -> 312 us, 2 with the output
+// layer and its scale 399 + 110 + 102 -> 328 us (the whole set-up and apply 1,380 -> 831 us), all bitwise
 // the same.  The mean layers are bound by the latency of the gathers and the arithmetic of the means and
 // silu at two waves per SIMD (64 KB of weights per workgroup); 384 and 512 threads around the same weights
 // were 14 % and 50 % slower (fewer registers per wave, spills).
@@ -178,7 +177,7 @@ __device__ inline int oct_slot(int n, int o) {
 // Memory is read and written with four consecutive lanes on 64 consecutive bytes of a row (lane l: row
 // l / 4, 16-byte piece l % 4); the MFMAs want row l % 16, octet l / 16.  In that order no two neighbouring
 // lanes share a row, every 16 bytes are an access of their own to the L1, and the L1 bounded the mean
-// layers (157M accesses, 69 % of the cycles at 1.5M cells).  The neighbours are summed in memory order, and
+// layers (1.5M cells: 181M accesses a layer, 0.79 per CU and cycle; now 38M, 0.22).  The neighbours are summed in memory order, and
 // four lane permutations per octet change the order (to_mfma, from_mfma).
 __device__ inline uint4 lane_perm(int from, uint4 v) {
   return make_uint4(__builtin_amdgcn_ds_bpermute(4 * from, v.x), __builtin_amdgcn_ds_bpermute(4 * from, v.y),

@@ -187,7 +187,7 @@ __device__ inline void flux_col(const double (&Um)[5], const double (&Un)[5], bo
 // The Jacobian kernels' workgroup (one wave: JAC_THREADS / NS cells) stages its cells' rows of JacC, 1000
 // bytes each, in LDS and stores them as one contiguous run.  Stored by the lanes that formed them (8
 // bytes each, 200 bytes apart) they went out at 1.7 TB/s and set jac_kernel's time: 593 us at 1.07M tets
-// and 3.65 ms at 6M, 401 us and 2.17 ms as a run (4 TB/s with the reads, of the copy's 4.9).  8-byte
+// and 3.65 ms at 6M, 401 us and 2.17 ms as a run (3.2 TB/s with the reads, of the copy's 4.9).  8-byte
 // stores: a caller's array need not be aligned to more.
 constexpr int JAC_THREADS = 64;
 template <int NS>
@@ -439,10 +439,11 @@ __global__ void factor_begin_kernel(double *gamma, double g, int *status) {
 // later rows) read them.  Every block the row needs is read at once, row q by lane q, and passed around
 // through LDS.  Before, one thread per row worked on a stored M, with M and the packed copies made in
 // passes of their own: 2.0 ms for the levels and 1.07 ms for the passes at 1.07M tets, 6.0 and 6.0 ms at
-// 6M; now 1.06 ms and 5.3 ms.  What bounds a level is its traffic (3.1 KB a row at 3.6 TB/s, 200-byte
-// blocks straddling cache lines), and on small meshes (24,000 tets: 25 -> 7 us a level) the latency of
-// its two dependent reads, its arithmetic and its stores.  At 204 registers two waves fit a SIMD; held to
-// 168 for three it was 18 % slower, and non-temporal reads of JacC were 7 % slower.
+// 6M; now 1.06 ms and 5.3 ms.  What bounds a level is its traffic (6M, FP32 factors: 3.3 KB a row at
+// 3.3 TB/s of the copy's 4.9, 200-byte blocks straddling cache lines), and on small meshes (24,000 tets:
+// 25 -> 7 us a level) the latency of its two dependent reads, its arithmetic and its stores.  At 204
+// registers two waves fit a SIMD; held to 168 for three it was 18 % slower, and non-temporal reads of JacC
+// were 7 % slower.
 // rec: per row {cell, elimination position p, first packed L block, first packed U block}, the lower
 // neighbours' positions in elimination order, and the packed U blocks that couple them to this row.
 // bits: 0-3 upper slots, 4-7 lower slots, 8-15 the lower neighbours' slots in elimination order (2
@@ -1040,8 +1041,9 @@ __global__ __launch_bounds__(64) void bwd_colour_kernel(int nC, const int4 *__re
 // bounded (FLOW_MAX_POLLS, seconds): past it the value is a NaN, which the callback reports.
 // The arithmetic per row is the colour kernels', in the same order: the results are bitwise the same.
 // Per apply, colour launches -> one launch (FP64): 6,000 tets 136 -> 42 us, 24,000 174 -> 53, 270,000
-// 233 -> 128, 540,000 267 -> 232; FP32 factors alike.  What is left is the chain: about 2.8 us for each
-// of the 17 colours of both sweeps (publish, see, gather: 1.0; the levels: 1.8).
+// 233 -> 128, 540,000 268 -> 232; FP32 factors alike.  What is left is the chain: about 2.8 us for each
+// of the 17 colours of both sweeps (publish, see, gather: 1.0; the levels: 1.8; by clock reads
+// in a copy of the kernel).
 constexpr int FLOW_THREADS = 384, FLOW_CTL = 32;
 constexpr unsigned long long FLOW_EMPTY = ~0ull;
 constexpr int FLOW_MAX_POLLS = 1 << 22;  // of a memory round trip (~1 us) each
